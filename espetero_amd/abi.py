@@ -10,6 +10,7 @@ import os
 import numpy as np
 
 ESP_F16, ESP_BF16 = 0, 1
+ESP_EWORKSPACE = 4
 ESP_LAYOUT_REFERENCE, ESP_LAYOUT_NATIVE = 0, 1
 ESP_ABI_VERSION = 3
 ESP_PASS_FUSED, ESP_PASS_ROWS_IN_POOL = 1, 2

@@ -84,6 +84,128 @@ struct AttnPlan {
   int rows_per_tile = 8;
 };
 
+struct RowTile {
+  int tree, r, k0, b0, span;
+  int batch;  // batch keys the tile scans after its cached range (balanced rule: part of its work)
+};
+
+// Streaming kernel, balanced rule: the parts of every row tile of a pass. `room`: tiles resident at once (all the KV
+// heads of a tile run side by side, so a tile stands for one workgroup on each of `groups` shares of the chip).
+//
+// What a split costs is worked out by running it: the tiles go to the compute units in the order the hardware will
+// start them, two workgroups on one compute unit share what it can pull (36 GB/s, whether one or two ask), all of them
+// together what memory gives (0.75 of that per unit), every workgroup has a fixed set-up and end, and a pass with any
+// split tile a merge behind it. Those two are kFixed and kMerge, in keys of head dim 128 (two workgroups per compute
+// unit: 512 bytes per key and head) or 256 (one: 1024 bytes): 60 KB and 4.6 us at 36 GB/s. Against 61 measured passes
+// (16 to 96 ragged sequences, head dims 128 and 256, 24 to 258 tiles) this is right within 10 %. Before, a pass that filled more than half of the chip with whole sequences was not split at
+// all: 48 sequences of 60 .. 3000 keys on 8 KV heads 72.5 us (62.6 at 74 tiles), 24 of 300 .. 6000 at head dim 256 175
+// us (114 at 53 tiles).
+template <typename PartsOf>
+inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const PlanOptions& o, int room, const PartsOf& parts_of) {
+  const int n = int(rts.size());
+  const int per_cu = o.groups_target >= 512 ? 2 : 1, cus = std::max(1, room / per_cu);
+  const double kFixed = per_cu == 2 ? 117 : 58, kMerge = per_cu == 2 ? 323 : 161;
+  long long total = 0;
+  for (const RowTile& rt : rts) total += rt.span + rt.batch;
+  std::vector<int> ns(size_t(n), 1), best(size_t(n), 1);
+  struct Item {
+    bool last;
+    int keys;
+  };
+  std::vector<Item> items;
+  auto count_at = [&](long long chunk) {
+    long long k = 0;
+    for (const RowTile& rt : rts) k += parts_of(rt, chunk);
+    return k;
+  };
+  struct Cu {
+    double rem[2], since;
+    int running;
+  };
+  std::vector<Cu> cu;
+  std::vector<double> idle;
+  auto time_at = [&](long long chunk) {
+    items.clear();
+    bool split = false;
+    for (int i = 0; i < n; ++i) {
+      const RowTile& rt = rts[size_t(i)];
+      const int k = int(parts_of(rt, chunk));
+      ns[size_t(i)] = k;
+      split = split || k > 1;
+      const int work = rt.span + rt.batch, step = ((work + k - 1) / k + o.granule - 1) / o.granule * o.granule;
+      for (int p = 0; p + 1 < k && p * step < rt.span; ++p) items.push_back({false, std::min(step, rt.span - p * step)});
+      items.push_back({true, std::max(0, work - (k - 1) * step)});
+    }
+    const bool one_round = int(items.size()) <= room;
+    std::stable_sort(items.begin(), items.end(), [&](const Item& x, const Item& y) {
+      if (one_round && x.last != y.last) return x.last;
+      return x.keys > y.keys;
+    });
+    // Every compute unit's own clock advances with the bytes it may pull; the real time follows from how many pull.
+    cu.assign(size_t(cus), Cu{{0, 0}, 0, 0});
+    size_t next = 0;
+    for (int s = 0; s < per_cu; ++s)
+      for (int c = 0; c < cus && next < items.size(); ++c) cu[size_t(c)].rem[cu[size_t(c)].running++] = items[next++].keys + kFixed;
+    using Event = std::pair<double, int>;
+    std::priority_queue<Event, std::vector<Event>, std::greater<Event>> q;
+    auto next_end = [&](const Cu& x) { return x.since + (x.running == 2 ? 2 * std::min(x.rem[0], x.rem[1]) : x.rem[0]); };
+    for (int c = 0; c < cus; ++c)
+      if (cu[size_t(c)].running) q.push({next_end(cu[size_t(c)]), c});
+    idle.clear();
+    while (!q.empty()) {
+      const auto [at, c] = q.top();
+      q.pop();
+      Cu& x = cu[size_t(c)];
+      if (x.running == 2) {
+        const double d = std::min(x.rem[0], x.rem[1]);
+        x.rem[0] = std::max(x.rem[0], x.rem[1]) - d;
+      }
+      --x.running;
+      x.since = at;
+      if (next < items.size()) x.rem[x.running++] = items[next++].keys + kFixed;
+      if (x.running) q.push({next_end(x), c});
+      else idle.push_back(at);
+    }
+    double t = 0, was = 0;
+    size_t pulling = idle.size();
+    for (double at : idle) {  // ascending: the queue hands events out in time order
+      t += (at - was) / std::min(1.0, 0.75 * cus / double(pulling--));
+      was = at;
+    }
+    return t + (split ? kMerge : 0);
+  };
+  // The smallest chunk whose tiles are all resident at once (a pass that overshoots that by a few tiles pays a second
+  // round for them), or no split where whole sequences already overfill the chip; any other candidate has to win by 5 %,
+  // a margin for kernels whose workgroups pull less alone than the model's (two column tiles, wavefront pairs): no
+  // split, and chunks of one and a half, three quarters and half of the pass's keys per resident tile.
+  double least = 0;
+  auto consider = [&](long long chunk, double win) {
+    chunk = std::max<long long>(chunk, std::max(1, o.min_chunk));
+    chunk = (chunk + o.granule - 1) / o.granule * o.granule;
+    const double t = time_at(chunk);
+    if (win == 0 || t < win * least) least = t, best = ns;
+  };
+  const long long whole = total + o.min_chunk;
+  if (n <= room) {
+    long long lo = std::max(1, o.min_chunk / o.granule), hi = std::max<long long>(lo, (total + o.granule - 1) / o.granule + 1);
+    while (lo < hi) {
+      const long long mid = (lo + hi) / 2;
+      if (count_at(mid * o.granule) <= room) hi = mid;
+      else lo = mid + 1;
+    }
+    consider(lo * o.granule, 0);
+    consider(whole, 0.95);
+  } else {
+    consider(whole, 0);
+  }
+  // Where the compute units end together no other split does better; within 10 % of that none is tried.
+  long long n_best = 0;
+  for (int k : best) n_best += k;
+  if (least > 1.1 * ((double(total) + kFixed * double(n_best)) / (0.75 * cus) + kMerge))
+    for (const double share : {1.5, 0.75, 0.5}) consider((long long)(double(total) / room * share), 0.95);
+  return best;
+}
+
 // groups: workgroups per tile (KV heads, or KV heads x head splits).
 // window > 0 needs pos (4 ints per row, pos[4 * row] = position).
 inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, const PlanOptions& o) {
@@ -92,12 +214,7 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
   A.parts = 0;
   A.rows_per_tile = o.rows_per_tile;
   const int R = o.rows_per_tile;
-  struct RowTile {
-    int tree, r, k0, b0, span;
-    int batch;  // batch keys the tile scans after its cached range (balanced rule: part of its work)
-  };
   std::vector<RowTile> rts;
-  long long total_span = 0;
   for (int ti = 0; ti < int(A.trees.size()); ++ti) {
     const esp_tree& t = A.trees[size_t(ti)];
     for (int r = 0; r < t.M; r += R) {
@@ -113,17 +230,15 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
       // A causal tile scans the batch rows up to its own last row; one split part takes them all.
       const int batch = o.balanced ? std::max(0, std::min(t.M, r + R) - b0) : 0;
       rts.push_back({ti, r, k0, b0, t.P - k0, batch});
-      total_span += t.P - k0 + batch;
     }
   }
   const int n_tiles = int(rts.size());
   int budget = std::max(1, o.groups_target / std::max(1, groups * n_tiles));
-  int chunk_all = 0;  // balanced rule: keys per workgroup
   auto cuttable = [&](const RowTile& rt) { return rt.span + (o.cut_batch ? rt.batch : 0) >= o.min_span; };
   auto parts_of = [&](const RowTile& rt, long long chunk) {
     return cuttable(rt) ? std::min<long long>((rt.span + rt.batch + chunk - 1) / chunk, o.max_splits) : 1;
   };
-  std::vector<int> ns_of;  // tiled kernel: parts of every row tile, once chosen
+  std::vector<int> ns_of;  // balanced rule: parts of every row tile, once chosen
   if (o.balanced && o.item_steps > 0) {
     // Tiled kernel. A pass is tiles x groups workgroups of unequal length (a causal chunk's later tiles
     // see more keys) on groups_target slots; the hardware hands the next workgroup to the first free slot,
@@ -200,22 +315,8 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
         if (t < best) best = t, ns_of = cand;
       }
     }
-  } else if (o.balanced && budget > 1) {
-    // The smallest chunk (a granule multiple) whose tile count fits the target: a pass
-    // that overshoots the resident workgroup count by a few tiles pays a whole extra round.
-    const long long cap = std::max(1, o.groups_target / std::max(1, groups));
-    auto tiles_at = [&](long long chunk) {
-      long long n = 0;
-      for (const RowTile& rt : rts) n += parts_of(rt, chunk);
-      return n;
-    };
-    long long lo = std::max(1, o.min_chunk / o.granule), hi = std::max<long long>(lo, (total_span + o.granule - 1) / o.granule + 1);
-    while (lo < hi) {
-      const long long mid = (lo + hi) / 2;
-      if (tiles_at(mid * o.granule) <= cap) hi = mid;
-      else lo = mid + 1;
-    }
-    chunk_all = int(lo * o.granule);
+  } else if (o.balanced && n_tiles > 0) {
+    ns_of = stream_split(rts, o, std::max(1, o.groups_target / std::max(1, groups)), parts_of);
   }
   for (const RowTile& rt : rts) {
     const esp_tree& t = A.trees[size_t(rt.tree)];
@@ -223,10 +324,8 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
     int ns = 1;
     if (!ns_of.empty()) {
       ns = ns_of[size_t(&rt - rts.data())];
-    } else if (budget > 1 && span >= o.min_span) {
-      if (o.balanced) {
-        ns = std::min((span + rt.batch + chunk_all - 1) / chunk_all, o.max_splits);
-      } else if (o.split > 0) {
+    } else if (!o.balanced && budget > 1 && span >= o.min_span) {
+      if (o.split > 0) {
         const int chunk =
             std::max(std::max(32, o.min_chunk),
                      std::min(o.split, ((span + budget - 1) / budget + o.granule - 1) / o.granule * o.granule));
@@ -309,15 +408,17 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
     }
     A.combine.push_back({t.base + rt.r, std::min(R, t.M - rt.r), part0, used});
   }
-  // Streaming kernel, balanced rule: every workgroup of the pass is resident at once and the hardware starts them
-  // in record order over a few microseconds. The tiles that own their tree's batch keys go first - behind their
-  // stream of cached keys they have a serial tail (the batch rows through the masked path) that the others'
-  // streaming then covers - and the rest follow by cached range, longest first. (Measured on the batched decode of
-  // 16 ragged sequences: 26.6 -> 25.8 us; with the owners of the batch keys last instead, 26.9 us.) The records'
-  // partial-record indices stay as assigned, so the merge order does not change.
+  // Streaming kernel, balanced rule: the hardware starts the workgroups in record order over a few microseconds. Where
+  // all of them are resident at once the tiles that own their tree's batch keys go first - behind their stream of
+  // cached keys they have a serial tail (the batch rows through the masked path) that the others' streaming then
+  // covers - and the rest follow by cached range, longest first. (Measured on the batched decode of 16 ragged
+  // sequences: 26.6 -> 25.8 us; with the owners of the batch keys last instead, 26.9 us.) Where there are more, the
+  // longest go first whatever they own, so that the pass ends on short ones (48 ragged sequences, 74 tiles of 64
+  // resident: 67.3 -> 62.6 us). The records' partial-record indices stay as assigned, so the merge order does not change.
   if (o.balanced && o.item_steps == 0) {
-    std::stable_sort(A.tiles.begin(), A.tiles.end(), [](const esp_tile& x, const esp_tile& y) {
-      if (x.last != y.last) return x.last > y.last;
+    const bool one_round = int(A.tiles.size()) <= std::max(1, o.groups_target / std::max(1, groups));
+    std::stable_sort(A.tiles.begin(), A.tiles.end(), [&](const esp_tile& x, const esp_tile& y) {
+      if (one_round && x.last != y.last) return x.last > y.last;
       return (x.k1 - x.k0) > (y.k1 - y.k0);
     });
   }

@@ -103,17 +103,21 @@ def plan_tiles(trees, groups, window, pos, options):
     pos_a = None if pos is None else np.ascontiguousarray(pos, dtype=np.int32)
     err = C.create_string_buffer(256)
     nt, nj, npart = C.c_int32(0), C.c_int32(0), C.c_int32(0)
-    rc = lib.esp_plan_tiles(trees.ctypes.data, len(trees), groups, window, None if pos_a is None else pos_a.ctypes.data,
-                            C.byref(options), None, 0, C.byref(nt), None, 0, C.byref(nj), C.byref(npart), err, 256)
-    if rc not in (0, 4):
-        abi.check(rc, err)
-    tiles = np.zeros(nt.value, abi.TILE_DT)
-    jobs = np.zeros(nj.value, abi.COMBINE_DT)
-    rc = lib.esp_plan_tiles(trees.ctypes.data, len(trees), groups, window, None if pos_a is None else pos_a.ctypes.data,
-                            C.byref(options), tiles.ctypes.data, len(tiles), C.byref(nt), jobs.ctypes.data, len(jobs),
-                            C.byref(nj), C.byref(npart), err, 256)
+    # Room for one tile per row group and three resident rounds of parts serves nearly every plan in one call; a plan that needs more
+    # says how many.
+    room = len(trees) + int(trees["M"].sum()) // max(options.rows_per_tile, 1) + 3 * max(options.groups_target // max(groups, 1), 1) + 64
+    n_tiles = n_jobs = room
+    while True:
+        tiles = np.empty(n_tiles, abi.TILE_DT)
+        jobs = np.empty(n_jobs, abi.COMBINE_DT)
+        rc = lib.esp_plan_tiles(trees.ctypes.data, len(trees), groups, window, None if pos_a is None else pos_a.ctypes.data,
+                                C.byref(options), tiles.ctypes.data, n_tiles, C.byref(nt), jobs.ctypes.data, n_jobs, C.byref(nj),
+                                C.byref(npart), err, 256)
+        if rc != abi.ESP_EWORKSPACE or (nt.value <= n_tiles and nj.value <= n_jobs):
+            break
+        n_tiles, n_jobs = max(n_tiles, nt.value), max(n_jobs, nj.value)
     abi.check(rc, err)
-    return tiles, jobs, npart.value
+    return tiles[:nt.value].copy(), jobs[:nj.value].copy(), npart.value
 
 
 def slot_file_save(path, length, next_pos, n_layers, blocks_kv):

@@ -229,6 +229,26 @@ def test_balanced_rule_equalises_keys_per_workgroup():
     assert 0.5 * 1024 / 4 <= len(bal_t) <= 1.5 * 1024 / 4
 
 
+@pytest.mark.parametrize("n,hi,slots", [(33, 3000, 512), (48, 3000, 512), (64, 3000, 512), (65, 3000, 512), (24, 6000, 256), (40, 90, 512), (1, 20000, 8)])
+def test_streaming_split_of_passes_that_nearly_fill_or_overfill_the_chip(n, hi, slots):
+    """Ragged sequences on 8 KV heads around the number of tiles resident at once: ranges partition every sequence, and
+    a pass whose longest sequence is well beyond an even share is cut until its longest part is at most about twice one."""
+    rng = np.random.default_rng(n)
+    lens = np.concatenate([[hi], rng.integers(max(1, hi // 40), hi + 1, n - 1)])
+    trees = np.array([(i, int(L), 0, 1) for i, L in enumerate(lens)], abi.TREE_DT)
+    tiles, jobs, parts = host.plan_tiles(trees, 8, 0, None, host.options_mi355x(1, slots))
+    for i, L in enumerate(lens):
+        xs = sorted((int(x["k0"]), int(x["k1"])) for x in tiles if x["tree"] == i)
+        assert xs[0][0] == 0 and xs[-1][1] == L and all(a[1] == b[0] for a, b in zip(xs, xs[1:]))
+    assert sum(int(x["part"]) >= 0 for x in tiles) == parts == sum(int(j["nparts"]) for j in jobs)
+    share = lens.sum() / max(1, slots // 8)
+    longest = max(int(x["k1"] - x["k0"]) for x in tiles)
+    if hi > 2.5 * share and hi > 1000 and slots > 8:
+        assert longest <= 2.2 * share
+    if hi < 128:
+        assert len(tiles) == n and parts == 0
+
+
 # ---------------------------------------------------------------- pool: allocator and copy-on-write lists
 def _conservation(e, n_blocks, slots):
     """Sum of refcounts == sum of list memberships; free + live == n_blocks."""
