@@ -1,0 +1,125 @@
+// CPython entry points of the calls a decode loop makes per layer and step (include/espetero_attn.h), arguments in the
+// header's order without the error buffer: records (ctypes structures) as objects with a buffer, device memory as
+// torch tensors, integers (addresses) or None, the stream as an integer. A failing call raises abi.EspError.
+//
+// Why native: a decode step of one short sequence is 8 us of GPU work behind two launches, and the ctypes form of the
+// same call - an error buffer, twenty pointer objects, a Stream object - cost the host about as much as the launches
+// themselves (10.6 us a step of one 1024-key sequence; in this form 8.3, the GPU being the slower side). The conversions below take one pass over the arguments.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <cstdint>
+#include <cstdio>
+#include <tuple>
+#include <type_traits>
+#include <utility>
+
+#include "../../include/espetero_attn.h"
+
+namespace {
+
+PyObject* g_data_ptr;  // interned "data_ptr"
+PyObject* g_error;     // abi.EspError
+
+// A structure's bytes, held until the call has returned.
+struct Record {
+  Py_buffer view{};
+  ~Record() {
+    if (view.obj) PyBuffer_Release(&view);
+  }
+};
+
+bool address(PyObject* o, void*& out) {
+  if (o == Py_None) {
+    out = nullptr;
+    return true;
+  }
+  if (PyLong_Check(o)) {
+    out = PyLong_AsVoidPtr(o);
+    return !(out == nullptr && PyErr_Occurred());
+  }
+  PyObject* v = PyObject_VectorcallMethod(g_data_ptr, &o, 1 | PY_VECTORCALL_ARGUMENTS_OFFSET, nullptr);
+  if (!v) return false;
+  out = PyLong_AsVoidPtr(v);
+  Py_DECREF(v);
+  return !(out == nullptr && PyErr_Occurred());
+}
+
+template <typename T>
+constexpr bool is_params = std::is_same_v<T, const esp_attn_params*> || std::is_same_v<T, const esp_prep_params*> ||
+                           std::is_same_v<T, const esp_gate_params*>;
+
+template <typename T>
+bool convert(PyObject* o, T& out, Record& rec) {
+  if constexpr (is_params<T>) {
+    if (PyObject_GetBuffer(o, &rec.view, PyBUF_SIMPLE) != 0) return false;
+    if (size_t(rec.view.len) < sizeof(std::remove_pointer_t<T>)) {
+      PyErr_SetString(PyExc_ValueError, "parameter record too small");
+      return false;
+    }
+    out = static_cast<T>(rec.view.buf);
+    return true;
+  } else if constexpr (std::is_pointer_v<T>) {
+    void* p = nullptr;
+    if (!address(o, p)) return false;
+    out = static_cast<T>(p);
+    return true;
+  } else if constexpr (std::is_signed_v<T>) {
+    const long v = PyLong_AsLong(o);
+    if (v == -1 && PyErr_Occurred()) return false;
+    if (v < INT32_MIN || v > INT32_MAX) {
+      PyErr_SetString(PyExc_OverflowError, "a count or size does not fit 32 bits");
+      return false;
+    }
+    out = T(v);
+    return true;
+  } else {
+    out = T(PyLong_AsUnsignedLongLong(o));
+    return !(out == T(-1) && PyErr_Occurred());
+  }
+}
+
+// The function's parameters less the last two (the error buffer and its length).
+template <auto Fn, typename... A, size_t... I>
+PyObject* run(int (*)(A...), std::index_sequence<I...>, PyObject* const* args, Py_ssize_t n) {
+  if (n != Py_ssize_t(sizeof...(I))) return PyErr_Format(PyExc_TypeError, "%zd arguments, %zd expected", n, Py_ssize_t(sizeof...(I)));
+  using All = std::tuple<A...>;
+  std::tuple<std::tuple_element_t<I, All>...> v{};
+  Record rec[sizeof...(I)];
+  if (!(convert(args[I], std::get<I>(v), rec[I]) && ...)) return nullptr;
+  char err[512];
+  err[0] = 0;
+  int rc;
+  Py_BEGIN_ALLOW_THREADS;
+  rc = Fn(std::get<I>(v)..., err, sizeof err);
+  Py_END_ALLOW_THREADS;
+  if (rc == ESP_OK) Py_RETURN_NONE;
+  return PyErr_Format(g_error, "esp error %d: %s", rc, err);
+}
+
+template <typename... A>
+constexpr size_t arity(int (*)(A...)) {
+  return sizeof...(A);
+}
+
+template <auto Fn>
+PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return run<Fn>(Fn, std::make_index_sequence<arity(Fn) - 2>{}, args, n);
+}
+
+#define ESP_CALL(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&call<esp_##name>)), METH_FASTCALL, nullptr}
+PyMethodDef g_methods[] = {ESP_CALL(attn_forward),   ESP_CALL(attn_forward_static), ESP_CALL(attn_decode_fused), ESP_CALL(attn_prep),
+                           ESP_CALL(attn_combine),   ESP_CALL(head_gate),           ESP_CALL(kv_save),           ESP_CALL(kv_copy_blocks),
+                           ESP_CALL(kv_export_blocks), ESP_CALL(kv_import_blocks),  ESP_CALL(chain_advance),     {nullptr, nullptr, 0, nullptr}};
+PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__calls() {
+  PyObject* abi = PyImport_ImportModule("espetero_amd.abi");
+  if (!abi) return nullptr;
+  g_error = PyObject_GetAttrString(abi, "EspError");
+  Py_DECREF(abi);
+  g_data_ptr = PyUnicode_InternFromString("data_ptr");
+  return g_error && g_data_ptr ? PyModule_Create(&g_module) : nullptr;
+}

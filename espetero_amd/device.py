@@ -11,17 +11,24 @@ import torch
 
 from . import abi
 
+try:
+    from . import _calls  # the per-step calls, csrc/calls.cpp
+except ImportError as e:
+    raise abi.EspError(f"espetero_amd/_calls.so is not built (run __graft_entry__.build()): {e}") from e
+
 _ERRLEN = 512
 
 
 def _ptr(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream(stream):
+    """hipStream_t as an int. The current stream is asked for as a raw handle: torch.cuda.current_stream() builds a Stream
+    object, 2.5 us of a decode step that has 8 us of GPU work."""
     if stream is None:
-        stream = torch.cuda.current_stream()
-    return C.c_void_p(stream.cuda_stream)
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return stream.cuda_stream
 
 
 def init(device=0):
@@ -59,22 +66,15 @@ def workspace_bytes(params, n_rows, n_parts):
 def forward(params, Q, Kb, Vb, pool, blocks, desc, pos, O, tiles, n_tiles, trees, n_trees, jobs, n_jobs, n_parts, n_rows,
             workspace, stream=None):
     """All tensors are device tensors (records as byte tensors). Enqueues on `stream`."""
-    err = C.create_string_buffer(_ERRLEN)
-    rc = abi.attn_lib().esp_attn_forward(
-        C.byref(params), _ptr(Q), _ptr(Kb), _ptr(Vb), _ptr(pool), _ptr(blocks), _ptr(desc), _ptr(pos), _ptr(O),
-        _ptr(tiles), n_tiles, _ptr(trees), n_trees, _ptr(jobs), n_jobs, n_parts, n_rows, _ptr(workspace),
-        0 if workspace is None else workspace.numel() * workspace.element_size(), _stream(stream), err, _ERRLEN)
-    abi.check(rc, err)
+    _calls.attn_forward(params, Q, Kb, Vb, pool, blocks, desc, pos, O, tiles, n_tiles, trees, n_trees, jobs, n_jobs, n_parts, n_rows,
+                        workspace, 0 if workspace is None else workspace.nbytes, _stream(stream))
 
 
 def forward_static(params, Q, Kb, Vb, pool, blocks, desc, pos, O, tiles, n_tiles, trees, n_trees, jobs, n_jobs, n_parts, n_rows,
                    stream=None):
     """forward() over the library's own scratch array: no workspace, no allocation."""
-    err = C.create_string_buffer(_ERRLEN)
-    rc = abi.attn_lib().esp_attn_forward_static(
-        C.byref(params), _ptr(Q), _ptr(Kb), _ptr(Vb), _ptr(pool), _ptr(blocks), _ptr(desc), _ptr(pos), _ptr(O),
-        _ptr(tiles), n_tiles, _ptr(trees), n_trees, _ptr(jobs), n_jobs, n_parts, n_rows, _stream(stream), err, _ERRLEN)
-    abi.check(rc, err)
+    _calls.attn_forward_static(params, Q, Kb, Vb, pool, blocks, desc, pos, O, tiles, n_tiles, trees, n_trees, jobs, n_jobs, n_parts, n_rows,
+                               _stream(stream))
 
 
 def validate(params, tiles, trees, jobs, n_parts, n_rows, blocks, pool_blocks, fused=False, rows_in_pool=False):
@@ -102,21 +102,15 @@ def time_next(start, stop):
 
 
 def combine(params, O, jobs, n_jobs, n_parts, n_rows, workspace, stream=None):
-    err = C.create_string_buffer(_ERRLEN)
-    abi.check(abi.attn_lib().esp_attn_combine(C.byref(params), _ptr(O), _ptr(jobs), n_jobs, n_parts, n_rows, _ptr(workspace),
-                                              workspace.numel() * workspace.element_size(), _stream(stream), err, _ERRLEN), err)
+    _calls.attn_combine(params, O, jobs, n_jobs, n_parts, n_rows, workspace, workspace.nbytes, _stream(stream))
 
 
 def kv_save(params, Kb, Vb, pool, entries, n_entries, stream=None):
-    err = C.create_string_buffer(_ERRLEN)
-    abi.check(abi.attn_lib().esp_kv_save(C.byref(params), _ptr(Kb), _ptr(Vb), _ptr(pool), _ptr(entries), n_entries,
-                                         _stream(stream), err, _ERRLEN), err)
+    _calls.kv_save(params, Kb, Vb, pool, entries, n_entries, _stream(stream))
 
 
 def kv_copy_blocks(params, pool, pairs, n_pairs, n_layers, region_elems, stream=None):
-    err = C.create_string_buffer(_ERRLEN)
-    abi.check(abi.attn_lib().esp_kv_copy_blocks(C.byref(params), _ptr(pool), _ptr(pairs), n_pairs, n_layers,
-                                                C.c_uint64(region_elems), _stream(stream), err, _ERRLEN), err)
+    _calls.kv_copy_blocks(params, pool, pairs, n_pairs, n_layers, region_elems, _stream(stream))
 
 
 def kv_gather(params, pool, blocks, n_tokens, K_out, V_out, stream=None):
@@ -132,47 +126,33 @@ def kv_relayout(params, src, src_layout, dst, dst_layout, n_blocks, stream=None)
 
 
 def kv_export_blocks(params, pool, blocks, n_blocks, out, stream=None):
-    err = C.create_string_buffer(_ERRLEN)
-    abi.check(abi.attn_lib().esp_kv_export_blocks(C.byref(params), _ptr(pool), _ptr(blocks), n_blocks, _ptr(out),
-                                                  _stream(stream), err, _ERRLEN), err)
+    _calls.kv_export_blocks(params, pool, blocks, n_blocks, out, _stream(stream))
 
 
 def kv_import_blocks(params, src, blocks, n_blocks, pool, stream=None):
-    err = C.create_string_buffer(_ERRLEN)
-    abi.check(abi.attn_lib().esp_kv_import_blocks(C.byref(params), _ptr(src), _ptr(blocks), n_blocks, _ptr(pool),
-                                                  _stream(stream), err, _ERRLEN), err)
+    _calls.kv_import_blocks(params, src, blocks, n_blocks, pool, _stream(stream))
 
 
 def attn_prep(params, X, qn_w, kn_w, pos, inv_freq, rope_sel, Q, Kb, Vb, row_table, pool, n_rows, stream=None):
     """All device tensors; rope_sel, row_table and pool may be None."""
-    err = C.create_string_buffer(_ERRLEN)
-    abi.check(abi.attn_lib().esp_attn_prep(C.byref(params), _ptr(X), _ptr(qn_w), _ptr(kn_w), _ptr(pos), _ptr(inv_freq),
-                                           _ptr(rope_sel), _ptr(Q), _ptr(Kb), _ptr(Vb), _ptr(row_table), _ptr(pool), n_rows,
-                                           _stream(stream), err, _ERRLEN), err)
+    _calls.attn_prep(params, X, qn_w, kn_w, pos, inv_freq, rope_sel, Q, Kb, Vb, row_table, pool, n_rows, _stream(stream))
 
 
 def decode_fused(pp, params, X, qn_w, kn_w, pos, inv_freq, rope_sel, row_table, pool, dp, O, stream=None):
     """attn_prep fused into the attention of a decode / short verify pass. dp: the DevicePass holding the records."""
-    err = C.create_string_buffer(_ERRLEN)
     ws = dp.workspace
-    abi.check(abi.attn_lib().esp_attn_decode_fused(
-        C.byref(pp), C.byref(params), _ptr(X), _ptr(qn_w), _ptr(kn_w), _ptr(pos), _ptr(inv_freq), _ptr(rope_sel), _ptr(row_table),
-        _ptr(pool), _ptr(dp.blocks), _ptr(dp.desc), _ptr(O), _ptr(dp.tiles), dp.n_tiles, _ptr(dp.trees), dp.n_trees, _ptr(dp.jobs),
-        dp.n_jobs, dp.n_parts, dp.n_rows, _ptr(ws), ws.numel() * ws.element_size(), _stream(stream), err, _ERRLEN), err)
+    _calls.attn_decode_fused(pp, params, X, qn_w, kn_w, pos, inv_freq, rope_sel, row_table, pool, dp.blocks, dp.desc, O, dp.tiles, dp.n_tiles,
+                             dp.trees, dp.n_trees, dp.jobs, dp.n_jobs, dp.n_parts, dp.n_rows, ws, ws.nbytes, _stream(stream))
 
 
 def head_gate(params, O, X, Wg, dots, n_rows, stream=None):
     """Device tensors. O (gated in place) or dots (fp32 [n_rows][H], written) may be None, not both."""
-    err = C.create_string_buffer(_ERRLEN)
-    abi.check(abi.attn_lib().esp_head_gate(C.byref(params), _ptr(O), _ptr(X), _ptr(Wg), _ptr(dots), n_rows,
-                                           _stream(stream), err, _ERRLEN), err)
+    _calls.head_gate(params, O, X, Wg, dots, n_rows, _stream(stream))
 
 
 def chain_advance(trees, n_trees, pos, row_table, blocks, bt, ring=0, stream=None):
     """Device tensors: trees (TREE_DT bytes), pos / row_table int32 [rows][4], blocks int32."""
-    err = C.create_string_buffer(_ERRLEN)
-    abi.check(abi.attn_lib().esp_chain_advance(_ptr(trees), n_trees, _ptr(pos), _ptr(row_table), _ptr(blocks), bt, ring,
-                                               _stream(stream), err, _ERRLEN), err)
+    _calls.chain_advance(trees, n_trees, pos, row_table, blocks, bt, ring, _stream(stream))
 
 
 class DevicePass:
@@ -199,28 +179,17 @@ class DevicePass:
         self.pos = to_dev(np.ascontiguousarray(pos, dtype=np.int32), device) if pos is not None else None
         nbytes = workspace_bytes(params, n_rows, n_parts)
         self.workspace = None if static else torch.empty(nbytes, dtype=torch.uint8, device=device)
-        self._key, self._fn, self._args, self._err = None, None, None, C.create_string_buffer(_ERRLEN)
 
     def run(self, Q, Kb, Vb, pool, O, stream=None, merge=True):
-        """Enqueues the pass. The ctypes argument list is built once per set of buffers and reused: a decode step is
-        tens of microseconds on the GPU, and rebuilding twenty pointer objects per call costs the host as much."""
-        st = torch.cuda.current_stream().cuda_stream if stream is None else stream.cuda_stream
-        key = (Q.data_ptr(), None if Kb is None else Kb.data_ptr(), None if Vb is None else Vb.data_ptr(), pool.data_ptr(), O.data_ptr(), st, merge,
-               None if self.pos is None else self.pos.data_ptr())
-        if self._key != key:
-            jobs, n_jobs = (self.jobs, self.n_jobs) if merge else (None, 0)
-            head = [C.byref(self.params), _ptr(Q), _ptr(Kb), _ptr(Vb), _ptr(pool), _ptr(self.blocks), _ptr(self.desc), _ptr(self.pos),
-                    _ptr(O), _ptr(self.tiles), self.n_tiles, _ptr(self.trees), self.n_trees, _ptr(jobs), n_jobs, self.n_parts, self.n_rows]
-            if self.static:
-                self._fn, self._args = abi.attn_lib().esp_attn_forward_static, head + [C.c_void_p(st), self._err, _ERRLEN]
-            else:
-                ws = self.workspace
-                self._fn = abi.attn_lib().esp_attn_forward
-                self._args = head + [_ptr(ws), ws.numel() * ws.element_size(), C.c_void_p(st), self._err, _ERRLEN]
-            self._key = key
-        rc = self._fn(*self._args)
-        if rc:
-            abi.check(rc, self._err)
+        """Enqueues the pass."""
+        jobs, n_jobs = (self.jobs, self.n_jobs) if merge else (None, 0)
+        if self.static:
+            _calls.attn_forward_static(self.params, Q, Kb, Vb, pool, self.blocks, self.desc, self.pos, O, self.tiles, self.n_tiles, self.trees,
+                                       self.n_trees, jobs, n_jobs, self.n_parts, self.n_rows, _stream(stream))
+        else:
+            ws = self.workspace
+            _calls.attn_forward(self.params, Q, Kb, Vb, pool, self.blocks, self.desc, self.pos, O, self.tiles, self.n_tiles, self.trees,
+                                self.n_trees, jobs, n_jobs, self.n_parts, self.n_rows, ws, ws.nbytes, _stream(stream))
 
     def merge(self, O, stream=None):
         if self.n_jobs:
