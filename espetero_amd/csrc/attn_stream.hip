@@ -181,39 +181,40 @@ __global__ __launch_bounds__(HD >= 512 ? 128 * NC : 256, OCC) void attn_stream_k
   uint16_t* k_lds = q_lds + NC * 16 * HD;                  // [kFusedRows][HD] this KV head's key rows
   uint16_t* v_lds = k_lds + kFusedRows * HD;               // [kFusedRows][HD] and value rows
   if constexpr (FUSED) {
-    constexpr int EPL = prep_epl(HD), LPH = HD / EPL, HPP = 256 / LPH;
+    constexpr int LPH = HD / kPrepDims, HPP = 256 / LPH;
     float2* cs = reinterpret_cast<float2*>(v_lds + kFusedRows * HD);  // [kFusedRows][HD / 2]
     const esp_prep_params& pp = pa.p;
     const int half = pp.rope_dims / 2;
     for (int i = threadIdx.x; i < rows_live * half; i += 256) {
       const int r = i / half, f = i - r * half;
-      cs[r * (HD / 2) + f] = prep_cos_sin(pa.pos[tile.r0 + r], pa.rope_sel, pa.inv_freq, f);
+      cs[r * (HD / 2) + f] = prep_cos_sin(pa.pos[tile.r0 + r], pa.rope_sel ? pa.rope_sel[f] : 0, pa.inv_freq[f]);
     }
     __syncthreads();
     const int n_q = rows_live * a.G, n_items = n_q + (tile.last ? 2 * rows_live : 0);
-    const int li = threadIdx.x % LPH, d0 = EPL * li;
+    const int li = threadIdx.x % LPH;
+    const PrepDims pd = prep_dims<HD>(pp, li);
     for (int it = threadIdx.x / LPH; it < n_items; it += HPP) {
       const int kind = it < n_q ? 0 : 1 + (it - n_q) / rows_live;
       const int m = it < n_q ? it / a.G : (it - n_q) % rows_live;
       const int h = it < n_q ? kvh * a.G + (it - m * a.G) : kvh;
       const size_t row = size_t(tile.r0 + m);
-      const size_t col = size_t(kind == 0 ? pp.q_off + h * pp.q_hs : (kind == 1 ? pp.k_off : pp.v_off) + h * HD) + d0;
-      float x[EPL], w[EPL];
+      const size_t col = size_t(kind == 0 ? pp.q_off + h * pp.q_hs : (kind == 1 ? pp.k_off : pp.v_off) + h * HD);
+      const float* xr = pa.X + row * pp.x_ld + col;
+      const f32x4 xa = *reinterpret_cast<const f32x4*>(xr + pd.a), xb = *reinterpret_cast<const f32x4*>(xr + pd.b);
+      const float* wn = kind == 0 ? pa.qn_w : pa.kn_w;
+      float x[kPrepDims], w[kPrepDims];
 #pragma unroll
-      for (int v = 0; v < EPL / 4; ++v) {
-        const f32x4 xv = *(reinterpret_cast<const f32x4*>(pa.X + row * pp.x_ld + col) + v);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[4 * v + i] = xv[i];
+      for (int i = 0; i < 4; ++i) {
+        x[i] = xa[i];
+        x[4 + i] = xb[i];
+        w[i] = kind != 2 ? wn[pd.a + i] : 1.0f;
+        w[4 + i] = kind != 2 ? wn[pd.b + i] : 1.0f;
       }
-#pragma unroll
-      for (int i = 0; i < EPL; ++i) w[i] = kind != 2 ? (kind == 0 ? pa.qn_w : pa.kn_w)[d0 + i] : 1.0f;
-      prep_lane<HD>(x, kind, w, cs + m * (HD / 2), pp, d0);
-      using out_t = std::conditional_t<EPL == 8, u32x4, u32x2>;
-      out_t out;
-#pragma unroll
-      for (int i = 0; i < EPL / 2; ++i) out[i] = pack2<DT>(x[2 * i], x[2 * i + 1]);
+      prep_lane<HD>(x, kind, w, cs + m * (HD / 2), pp, li, pd.rot);
+      const u32x2 out[2] = {{pack2<DT>(x[0], x[1]), pack2<DT>(x[2], x[3])}, {pack2<DT>(x[4], x[5]), pack2<DT>(x[6], x[7])}};
       uint16_t* dst = kind == 0 ? q_lds + it * HD : (kind == 1 ? k_lds : v_lds) + m * HD;
-      *reinterpret_cast<out_t*>(dst + d0) = out;
+      *reinterpret_cast<u32x2*>(dst + pd.a) = out[0];
+      *reinterpret_cast<u32x2*>(dst + pd.b) = out[1];
       if (kind == 0 || !pa.row_table) continue;
       // the folded append: the row's key and value of this KV head into its pool entries
       const int4 ent = pa.row_table[row];
@@ -222,16 +223,8 @@ __global__ __launch_bounds__(HD >= 512 ? 128 * NC : 256, OCC) void attn_stream_k
         const int b = e ? ent.z : ent.x, ps = e ? ent.w : ent.y;
         if (b < 0) continue;
         uint16_t* hb = pa.pool + pp.kv_base + (size_t(b) * pp.Hkv + h) * size_t(2 * pp.bt * HD);
-        if (kind == 1) {
-          *reinterpret_cast<out_t*>(hb + size_t(ps) * HD + d0) = out;
-        } else {
-          uint16_t* vt = hb + vt_elem(pp.bt, HD, ps, d0);
 #pragma unroll
-          for (int i = 0; i < EPL / 2; ++i) {
-            vt[(2 * i) * kVtDim] = uint16_t(out[i] & 0xffffu);
-            vt[(2 * i + 1) * kVtDim] = uint16_t(out[i] >> 16);
-          }
-        }
+        for (int c = 0; c < 2; ++c) prep_append<HD>(hb, kind, pp.bt, ps, c ? pd.b : pd.a, out[c]);
       }
     }
     __syncthreads();

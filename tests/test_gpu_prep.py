@@ -59,6 +59,24 @@ def test_prep_matches_checker(kind, H, Hkv, HD, dtype):
     assert np.array_equal(got[2], want[2]) or p.v_norm                    # a plain cast has nothing to differ in
 
 
+@pytest.mark.parametrize("HD,rope", [(128, 0), (128, 8), (128, 64), (256, 8), (256, 128), (512, 16), (512, 256)])
+@pytest.mark.parametrize("n_rows", [1, 8, 9])
+def test_prep_partial_rotation_edges(HD, rope, n_rows):
+    """Every split of a head into rotating chunk pairs and the rest (none, one lane, half of the lanes), and row groups of one
+    row, exactly one workgroup's and one more: the same bar as above."""
+    device.init(0)
+    p, a = synth.make_prep("omni", 5, 3, HD, abi.ESP_F16, n_rows, seed=12)
+    p.rope_dims = rope
+    half = rope // 2
+    a["inv_freq"], a["rope_sel"] = (a["inv_freq"][:half].copy(), a["rope_sel"][:half].copy()) if half else (None, None)
+    print(f"prep rope HD={HD} rope={rope} rows={n_rows}", flush=True)
+    ref = dict(a, inv_freq=a["inv_freq"] if half else np.zeros(1, np.float32), rope_sel=a["rope_sel"] if half else np.zeros(1, np.int32))
+    want = ob.attn_prep(p, a["X"], a["qn_w"], a["kn_w"], a["pos"], ref["inv_freq"], ref["rope_sel"], n_rows)
+    for g, w in zip(_run_gpu(p, a, n_rows), want):
+        far = (_ulps(g, w, p.dtype) > 1) & (np.abs(ob.to_f32(g, p.dtype) - ob.to_f32(w, p.dtype)) > 2.0 ** -11)
+        assert not far.any()
+
+
 def test_prep_folded_append_is_bitwise_kv_save():
     device.init(0)
     n_rows, bt, n_blocks = 50, 16, 12
