@@ -42,6 +42,8 @@
 
 namespace esp {
 
+constexpr unsigned kComputeUnits = 256;  // of one MI355X
+
 template <int DT, int HD, int OCC>
 __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int n_tiles) {
   constexpr int KS = HD / 16, NT = HD / 32;
@@ -69,7 +71,6 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   const int rest = blockIdx.x / a.Hkv;
   const int hg = rest % a.G;
   const int tile_i = n_tiles - 1 - rest / a.G;
-  const int h = kvh * a.G + hg;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l32 = lane & 31, hb = lane >> 5;
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   // ---- this lane's row. Its loads need the tile's record only (a row past the tree's last one reads the pass's
   // last row instead and is zeroed once the tree's record says so): they are in flight while that record arrives.
   const int m_row = 32 * wave + l32;
-  const int row = min(tile.r0 + m_row, a.n_rows - 1);
+  int row = min(tile.r0 + m_row, a.n_rows - 1);
   int4 d = a.desc ? a.desc[row] : make_int4(0, 0, 0, 0);
   int qpos = a.window > 0 ? a.pos[row].x : 0;
   // Q fragments as stored. The scale (times log2 e) is applied to the fp32 score in the same fused
@@ -87,11 +88,12 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   // of a few units is more than the 2e-3 the path promises (the reference pre-scales Q only by an
   // exact power of two, kernels/40_attention.metal:195-200).
   u32x4 qf[KS];
-  {
+  auto load_q = [&](int h) __attribute__((always_inline)) {
     const uint16_t* qp = a.Q + size_t(row) * a.q_ld + size_t(h) * HD + 8 * hb;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const u32x4*>(qp + 16 * ks);
-  }
+  };
+  load_q(kvh * a.G + hg);
 
   const esp_tree tree = a.trees[tile.tree];
   if (tile.k1 == INT32_MAX) tile.k1 = tree.P;  // open-ended range: up to the tree's cached length as it is now
@@ -99,7 +101,24 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   const int end = tree.base + tree.M;
   const int rows_live = min(a.R, end - tile.r0);
   const int rr0 = tile.r0 - tree.base;
-  const int rr = rr0 + m_row;
+  // A short tile whose rows of all G query heads fit the tile's 128 places - a decoding sequence in a pass of prompt
+  // chunks, a prompt's remainder - is one workgroup per KV head: place x of it is row x / G, query head x % G, and the
+  // workgroups of the other heads end here. One head at a time such a tile streams its keys through LDS and the matrix
+  // cores G times for a few live rows of 128. (512 prompt rows behind 2048 keys with 12 decoding sequences of 200 .. 6000
+  // keys, 32 / 4 heads of 128, whole step: 117.7 us before, 109 so, 73 with the plan that counts on it.) Where every workgroup of the
+  // grid has a compute unit to itself nothing is gained, and the second load of the rows behind the tree's record is 1.6 us
+  // of an 18.5 us step of short prompts: such passes keep one head per workgroup.
+  const bool packed = rows_live * a.G <= 128 && gridDim.x > kComputeUnits;
+  int m = m_row;
+  if (packed && a.G > 1) {
+    if (hg != 0) return;
+    m = m_row / a.G;
+    row = min(tile.r0 + m, a.n_rows - 1);
+    if (a.desc) d = a.desc[row];
+    if (a.window > 0) qpos = a.pos[row].x;
+    load_q(kvh * a.G + m_row - m * a.G);
+  }
+  const int rr = rr0 + m;
 
   // ---- the key range as 16-key sub-blocks: cached [k0, k1), then batch rows [b0, k_last]
   const int c0 = tile.k0 >> 4;
@@ -186,7 +205,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   const bool early = n_c + n_b_sure >= 4;
   if (early) stage_pool(0, 0);
 
-  const bool row_ok = m_row < rows_live;
+  const bool row_ok = m < rows_live;
   if (!row_ok) {
     d = make_int4(0, 0, 0, 0);
     qpos = 0;
@@ -376,7 +395,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
     for (int i = 0; i < 16; ++i) acc[nt][i] = 0.0f;
 
   // Batch steps past this wavefront's last row hold nothing it can see (plain causal rows).
-  const int wave_last = rr0 + min(32 * wave + 31, rows_live - 1);
+  const int wave_last = min(__builtin_amdgcn_readlane(rr, 31), rr0 + rows_live - 1);
   auto skipped = [&](int step) {
     const int s0 = 4 * step;
     if (s0 < n_c || seg_max == INT32_MAX) return false;
@@ -461,7 +480,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
       } else if (s0 >= n_c && s0 + 2 <= n_sb) {
         const int j0 = ((a0 + s0 - n_c) << 4) - tree.base;
         // (j0 + 31 <= k_last matters where the part's batch range ends early: without a cut every row of the tile lies below k_last)
-        half_full = !batch_window && j0 >= seg_max && j0 + 31 <= min(rr0 + 32 * wave, k_last) && j0 >= tile.b0 && j0 >= bw_lo;
+        half_full = !batch_window && j0 >= seg_max && j0 + 31 <= min(__builtin_amdgcn_readfirstlane(rr), k_last) && j0 >= tile.b0 && j0 >= bw_lo;
       } else {
         half_full = false;
       }
@@ -717,8 +736,9 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
     (phase.template operator()<S, G>(step, interior), ...);
   };
 
-  // Steps this wavefront computes: batch steps past its last row hold nothing it can see.
-  int my_steps = n_steps;
+  // Steps this wavefront computes: batch steps past its last row hold nothing it can see, and one without a row has
+  // only its share of the staging to do.
+  int my_steps = __builtin_amdgcn_readfirstlane(rr) < rr0 + rows_live ? n_steps : 0;
   while (my_steps > 0 && skipped(my_steps - 1)) --my_steps;
 
   // At the top of iteration i the barrier that publishes step i has been passed, step i + 1 is
@@ -820,8 +840,9 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   // ---- output: lane (row l32, half hb) holds dims 32 nt + 8 i + 4 hb + j at acc[nt][4 i + j]
   const float l = l_run + __shfl_xor(l_run, 32);
   if (!row_ok) return;
+  const int h_in_group = packed ? m_row % a.G : hg;
   if (tile.part >= 0) {
-    const size_t rec = (size_t(tile.part) * a.Hkv + kvh) * a.cols + size_t(m_row) * a.G + hg;
+    const size_t rec = (size_t(tile.part) * a.Hkv + kvh) * a.cols + size_t(rr - rr0) * a.G + h_in_group;
     float* po = a.parts_o + rec * HD;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
@@ -836,6 +857,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
     return;
   }
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  const int h = kvh * a.G + h_in_group;
   uint16_t* op = a.O + size_t(row) * a.q_ld + size_t(h) * HD;
   const float* gp = a.gate ? a.gate + size_t(row) * a.gate_ld + size_t(h) * a.gate_hs + a.gate_off : nullptr;
 #pragma unroll

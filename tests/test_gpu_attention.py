@@ -165,6 +165,30 @@ def test_tiled_kernel_matches_checker(kw):
     _check(small_case(seed=41, rows_per_tile=128, **kw))
 
 
+# ---- tiled kernel: short tiles (all query heads of their rows in one workgroup) beside whole ones
+@pytest.mark.parametrize("kw", [
+    dict(seqs=((300, 140), (70, 1), (1500, 1), (0, 1)), H=16),                     # G = 8: riders, one with nothing cached
+    dict(seqs=((40, 15), (40, 16), (40, 17)), H=16),                               # 120, 128 places; 17 rows do not fit
+    dict(seqs=((33, 25), (33, 26), (90, 129)), H=10, dtype=abi.ESP_BF16),          # G = 5: 125 places, 130; a prompt's last row
+    dict(seqs=((100, 64), (100, 65), (31, 32)), H=4),                              # G = 2, and whole wavefronts without a row
+    dict(seqs=((50, 128), (60, 1)), H=2),                                          # G = 1: every tile fits
+    dict(seqs=((1000, 200), (900, 1), (700, 3)), window=128, ring_layer=True, H=12),  # G = 6, windows over rings
+    dict(seqs=((700, 9), (100, 130)), H=8, desc_fn=lambda M: synth.verify_desc(M, 1)),  # drafts: descriptors per row
+    dict(seqs=((200, 30),), H=8, bidi=1, desc_fn=lambda M: synth.image_desc(M, 2, 20)),  # rows that see beyond themselves
+    dict(seqs=((1100, 5), (400, 150)), H=24, Hkv=4, HD=256, bt=64),                # head dim 256
+])
+@pytest.mark.parametrize("split", [False, True])
+def test_tiled_kernel_short_tiles(kw, split):
+    """Splits: the partial records of a short tile lie where the merge looks for them (chunks of 64 keys, so that every tile has
+    several)."""
+    c = small_case(seed=43, rows_per_tile=128, fill_unused=not kw.get("ring_layer", False), **kw)
+    opts = None
+    if split:
+        opts = host.options_mi355x(128, 8192)
+        opts.min_chunk, opts.min_span, opts.item_steps, opts.part_steps = 64, 128, 1, 0
+    _check(c, opts)
+
+
 # ---- logits of several units, a row maximum that keeps moving
 @pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
 @pytest.mark.parametrize("kw", [
