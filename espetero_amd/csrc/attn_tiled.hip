@@ -11,7 +11,7 @@
 // partial record for attention_combine.
 //
 // Mapping to gfx950. One workgroup = one tile of up to 128 query rows x one
-// query head, 4 wavefronts of 32 rows each. Keys advance in steps of 64 (four
+// query head (of a short tile: x all query heads of a KV head), 4 wavefronts of 32 rows each. Keys advance in steps of 64 (four
 // 16-key sub-blocks: one page each at page size 16). Wavefront w stages
 // sub-block w of a step with global_load_lds_dwordx4: 16 bytes per lane travel
 // from global memory straight into LDS (lane l's bytes land at base + 16 l),
@@ -395,6 +395,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
     for (int i = 0; i < 16; ++i) acc[nt][i] = 0.0f;
 
   // Batch steps past this wavefront's last row hold nothing it can see (plain causal rows).
+  const int wave_first = __builtin_amdgcn_readfirstlane(rr);
   const int wave_last = min(__builtin_amdgcn_readlane(rr, 31), rr0 + rows_live - 1);
   auto skipped = [&](int step) {
     const int s0 = 4 * step;
@@ -480,7 +481,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
       } else if (s0 >= n_c && s0 + 2 <= n_sb) {
         const int j0 = ((a0 + s0 - n_c) << 4) - tree.base;
         // (j0 + 31 <= k_last matters where the part's batch range ends early: without a cut every row of the tile lies below k_last)
-        half_full = !batch_window && j0 >= seg_max && j0 + 31 <= min(__builtin_amdgcn_readfirstlane(rr), k_last) && j0 >= tile.b0 && j0 >= bw_lo;
+        half_full = !batch_window && j0 >= seg_max && j0 + 31 <= min(wave_first, k_last) && j0 >= tile.b0 && j0 >= bw_lo;
       } else {
         half_full = false;
       }
@@ -738,7 +739,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
 
   // Steps this wavefront computes: batch steps past its last row hold nothing it can see, and one without a row has
   // only its share of the staging to do.
-  int my_steps = __builtin_amdgcn_readfirstlane(rr) < rr0 + rows_live ? n_steps : 0;
+  int my_steps = wave_first < rr0 + rows_live ? n_steps : 0;
   while (my_steps > 0 && skipped(my_steps - 1)) --my_steps;
 
   // At the top of iteration i the barrier that publishes step i has been passed, step i + 1 is

@@ -179,8 +179,10 @@ def test_tiled_kernel_matches_checker(kw):
 ])
 @pytest.mark.parametrize("split", [False, True])
 def test_tiled_kernel_short_tiles(kw, split):
-    """Splits: the partial records of a short tile lie where the merge looks for them (chunks of 64 keys, so that every tile has
+    """Enough copies of the sequences that the grid is more than a workgroup per compute unit, where short tiles are packed.
+    Splits: the partial records of a short tile lie where the merge looks for them (chunks of 64 keys, so that every tile has
     several)."""
+    kw = dict(kw, seqs=kw["seqs"] * -(-257 // (kw["H"] * len(kw["seqs"]))))
     c = small_case(seed=43, rows_per_tile=128, fill_unused=not kw.get("ring_layer", False), **kw)
     opts = None
     if split:
