@@ -1,6 +1,7 @@
 // CPython entry points of the calls a decode loop makes per layer and step (include/espetero_attn.h), arguments in the
-// header's order without the error buffer: records (ctypes structures) as objects with a buffer, device memory as
-// torch tensors, integers (addresses) or None, the stream as an integer. A failing call raises abi.EspError.
+// header's order without the error buffer: records as instances of their own ctypes classes (abi.AttnParams, PrepParams,
+// GateParams), device memory as torch tensors or None, the stream as an integer. Anything else is refused before the library
+// is called: it would read another record's bytes, or a number, as an address. A failing call raises abi.EspError.
 //
 // Why native: a decode step of one short sequence is 8 us of GPU work behind two launches, and the ctypes form of the
 // same call - an error buffer, twenty pointer objects, a Stream object - cost the host about as much as the launches
@@ -20,6 +21,8 @@ namespace {
 
 PyObject* g_data_ptr;  // interned "data_ptr"
 PyObject* g_error;     // abi.EspError
+// abi's classes of the parameter records
+PyTypeObject *g_attn_params, *g_prep_params, *g_gate_params;
 
 // A structure's bytes, held until the call has returned.
 struct Record {
@@ -29,14 +32,11 @@ struct Record {
   }
 };
 
+// The address of a tensor (of whatever has a data_ptr method); None: a null pointer.
 bool address(PyObject* o, void*& out) {
   if (o == Py_None) {
     out = nullptr;
     return true;
-  }
-  if (PyLong_Check(o)) {
-    out = PyLong_AsVoidPtr(o);
-    return !(out == nullptr && PyErr_Occurred());
   }
   PyObject* v = PyObject_VectorcallMethod(g_data_ptr, &o, 1 | PY_VECTORCALL_ARGUMENTS_OFFSET, nullptr);
   if (!v) return false;
@@ -46,12 +46,26 @@ bool address(PyObject* o, void*& out) {
 }
 
 template <typename T>
+PyTypeObject* record_class() {
+  if constexpr (std::is_same_v<T, const esp_attn_params*>) return g_attn_params;
+  else if constexpr (std::is_same_v<T, const esp_prep_params*>) return g_prep_params;
+  else if constexpr (std::is_same_v<T, const esp_gate_params*>) return g_gate_params;
+  else return nullptr;
+}
+
+template <typename T>
 constexpr bool is_params = std::is_same_v<T, const esp_attn_params*> || std::is_same_v<T, const esp_prep_params*> ||
                            std::is_same_v<T, const esp_gate_params*>;
 
-template <typename T>
+// stream: the call's last argument, a hipStream_t as an integer.
+template <bool stream, typename T>
 bool convert(PyObject* o, T& out, Record& rec) {
   if constexpr (is_params<T>) {
+    PyTypeObject* const cls = record_class<T>();
+    if (!PyObject_TypeCheck(o, cls)) {
+      PyErr_Format(PyExc_TypeError, "%s expected, not %s", cls->tp_name, Py_TYPE(o)->tp_name);
+      return false;
+    }
     if (PyObject_GetBuffer(o, &rec.view, PyBUF_SIMPLE) != 0) return false;
     if (size_t(rec.view.len) < sizeof(std::remove_pointer_t<T>)) {
       PyErr_SetString(PyExc_ValueError, "parameter record too small");
@@ -59,6 +73,9 @@ bool convert(PyObject* o, T& out, Record& rec) {
     }
     out = static_cast<T>(rec.view.buf);
     return true;
+  } else if constexpr (stream) {
+    out = static_cast<T>(PyLong_AsVoidPtr(o));
+    return !(out == nullptr && PyErr_Occurred());
   } else if constexpr (std::is_pointer_v<T>) {
     void* p = nullptr;
     if (!address(o, p)) return false;
@@ -86,7 +103,7 @@ PyObject* run(int (*)(A...), std::index_sequence<I...>, PyObject* const* args, P
   using All = std::tuple<A...>;
   std::tuple<std::tuple_element_t<I, All>...> v{};
   Record rec[sizeof...(I)];
-  if (!(convert(args[I], std::get<I>(v), rec[I]) && ...)) return nullptr;
+  if (!(convert<I + 1 == sizeof...(I)>(args[I], std::get<I>(v), rec[I]) && ...)) return nullptr;
   char err[512];
   err[0] = 0;
   int rc;
@@ -119,7 +136,11 @@ PyMODINIT_FUNC PyInit__calls() {
   PyObject* abi = PyImport_ImportModule("espetero_amd.abi");
   if (!abi) return nullptr;
   g_error = PyObject_GetAttrString(abi, "EspError");
+  g_attn_params = reinterpret_cast<PyTypeObject*>(PyObject_GetAttrString(abi, "AttnParams"));
+  g_prep_params = reinterpret_cast<PyTypeObject*>(PyObject_GetAttrString(abi, "PrepParams"));
+  g_gate_params = reinterpret_cast<PyTypeObject*>(PyObject_GetAttrString(abi, "GateParams"));
   Py_DECREF(abi);
   g_data_ptr = PyUnicode_InternFromString("data_ptr");
-  return g_error && g_data_ptr ? PyModule_Create(&g_module) : nullptr;
+  if (!g_error || !g_attn_params || !g_prep_params || !g_gate_params || !g_data_ptr) return nullptr;
+  return PyModule_Create(&g_module);
 }

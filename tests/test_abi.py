@@ -4,6 +4,9 @@ import ctypes as C
 import os
 import re
 
+import numpy as np
+import pytest
+
 from espetero_amd import abi, host
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -295,3 +298,24 @@ def test_forward_static_refuses_what_does_not_fit_its_scratch_array():
     assert rc == 1 and b"multiple of Hkv" in err.value
     p = synth.make_params(32, 4, 128, abi.ESP_F16, 16, rows_per_tile=4)
     assert lib.esp_attn_workspace_bytes(C.byref(p), 32, 4096) > abi.ESP_STATIC_SCRATCH_BYTES
+
+
+def _stream_stub():
+    return type("Stream", (), {"cuda_stream": 0})()
+
+
+@pytest.mark.parametrize("call,refusal", [
+    (lambda d, p, t, s: d.attn_prep(abi.AttnParams(), t, t, t, t, t, None, t, t, t, None, None, 0, s), "PrepParams expected, not AttnParams"),
+    (lambda d, p, t, s: d.head_gate(abi.AttnParams(), t, t, t, None, 0, s), "GateParams expected, not AttnParams"),
+    (lambda d, p, t, s: d.kv_save(bytes(80), t, t, t, t, 0, s), "AttnParams expected, not bytes"),
+    (lambda d, p, t, s: d.kv_save(None, t, t, t, t, 0, s), "AttnParams expected, not NoneType"),
+    (lambda d, p, t, s: d.kv_save(p, 1, 2, 3, 4, 0, s), "data_ptr"),                    # a number is no tensor
+    (lambda d, p, t, s: d.kv_save(p, t, t, t, t, 0.0, s), "float"),
+    (lambda d, p, t, s: d.kv_save(p, t, t, t, t, 1 << 32, s), "32 bits"),
+])
+def test_per_step_calls_refuse_what_is_not_their_record_or_a_tensor(call, refusal):
+    """Refused while the arguments are read: the library never sees them."""
+    import torch
+    from espetero_amd import device, synth
+    with pytest.raises((TypeError, AttributeError, OverflowError), match=refusal):
+        call(device, synth.make_params(32, 4, 128, abi.ESP_F16, 16), torch.zeros(64), _stream_stub())
