@@ -90,8 +90,8 @@ bool convert(PyObject* o, T& out, Record& rec) {
     }
     out = T(v);
     return true;
-  } else {
-    out = T(PyLong_AsUnsignedLongLong(o));
+  } else {  // any integer, numpy's among them
+    out = T(PyLong_AsUnsignedLongLongMask(o));
     return !(out == T(-1) && PyErr_Occurred());
   }
 }

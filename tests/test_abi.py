@@ -312,6 +312,7 @@ def _stream_stub():
     (lambda d, p, t, s: d.kv_save(p, 1, 2, 3, 4, 0, s), "data_ptr"),                    # a number is no tensor
     (lambda d, p, t, s: d.kv_save(p, t, t, t, t, 0.0, s), "float"),
     (lambda d, p, t, s: d.kv_save(p, t, t, t, t, 1 << 32, s), "32 bits"),
+    (lambda d, p, t, s: d.kv_copy_blocks(p, t, t, 0, 1, 64.0, s), "float"),
 ])
 def test_per_step_calls_refuse_what_is_not_their_record_or_a_tensor(call, refusal):
     """Refused while the arguments are read: the library never sees them."""
@@ -319,3 +320,17 @@ def test_per_step_calls_refuse_what_is_not_their_record_or_a_tensor(call, refusa
     from espetero_amd import device, synth
     with pytest.raises((TypeError, AttributeError, OverflowError), match=refusal):
         call(device, synth.make_params(32, 4, 128, abi.ESP_F16, 16), torch.zeros(64), _stream_stub())
+
+
+def test_per_step_calls_take_numpy_integers_and_derived_records():
+    """Counts of 0: nothing is launched."""
+    import torch
+    from espetero_amd import device, synth
+
+    class Params(abi.AttnParams):
+        pass
+
+    p, t, s = synth.make_params(32, 4, 128, abi.ESP_F16, 16), torch.zeros(64), _stream_stub()
+    device.kv_copy_blocks(p, t, t, np.int32(0), np.int64(1), np.int64(64), s)
+    device.kv_copy_blocks(p, t, t, 0, 1, np.uint64(64), s)
+    device.kv_save(Params.from_buffer_copy(p), None, None, t, None, 0, s)
