@@ -139,8 +139,20 @@ PyMODINIT_FUNC PyInit__calls() {
   g_attn_params = reinterpret_cast<PyTypeObject*>(PyObject_GetAttrString(abi, "AttnParams"));
   g_prep_params = reinterpret_cast<PyTypeObject*>(PyObject_GetAttrString(abi, "PrepParams"));
   g_gate_params = reinterpret_cast<PyTypeObject*>(PyObject_GetAttrString(abi, "GateParams"));
+  PyObject* version = PyObject_GetAttrString(abi, "ESP_ABI_VERSION");
   Py_DECREF(abi);
   g_data_ptr = PyUnicode_InternFromString("data_ptr");
-  if (!g_error || !g_attn_params || !g_prep_params || !g_gate_params || !g_data_ptr) return nullptr;
+  if (!g_error || !g_attn_params || !g_prep_params || !g_gate_params || !version || !g_data_ptr) {
+    Py_XDECREF(version);
+    return nullptr;
+  }
+  // The library that was loaded, this file and abi's records have to be of one version: as abi.attn_lib() checks for ctypes.
+  const long want = PyLong_AsLong(version);
+  Py_DECREF(version);
+  if (want == -1 && PyErr_Occurred()) return nullptr;
+  if (esp_attn_abi_version() != want || want != ESP_ABI_VERSION) {
+    PyErr_SetString(g_error, "libespetero_attn.so: ABI version mismatch");
+    return nullptr;
+  }
   return PyModule_Create(&g_module);
 }

@@ -334,3 +334,14 @@ def test_per_step_calls_take_numpy_integers_and_derived_records():
     device.kv_copy_blocks(p, t, t, np.int32(0), np.int64(1), np.int64(64), s)
     device.kv_copy_blocks(p, t, t, 0, 1, np.uint64(64), s)
     device.kv_save(Params.from_buffer_copy(p), None, None, t, None, 0, s)
+
+
+def test_per_step_calls_compare_the_abi_version():
+    """The extension is not imported against a library or records of another version (its own process: a module is
+    initialised once)."""
+    import subprocess
+    import sys
+    code = ("from espetero_amd import abi\nabi.ESP_ABI_VERSION += 1\n"
+            "try:\n    from espetero_amd import device\nexcept abi.EspError as e:\n    print(e)\n")
+    r = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(abi._PKG_DIR), capture_output=True, text=True, timeout=300)
+    assert "ABI version mismatch" in r.stdout, r.stdout + r.stderr
