@@ -242,7 +242,8 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
   int budget = std::max(1, o.groups_target / std::max(1, groups * n_tiles));
   auto cuttable = [&](const RowTile& rt) { return rt.span + (o.cut_batch ? rt.batch : 0) >= o.min_span; };
   auto parts_of = [&](const RowTile& rt, long long chunk) {
-    return cuttable(rt) ? std::min<long long>((rt.span + rt.batch + chunk - 1) / chunk, o.max_splits) : 1;
+    // (at least one: with min_span <= 0 a tile that sees no key at all may be asked for)
+    return cuttable(rt) ? std::clamp<long long>((rt.span + rt.batch + chunk - 1) / chunk, 1, o.max_splits) : 1;
   };
   std::vector<int> ns_of;  // balanced rule: parts of every row tile, once chosen
   if (o.balanced && o.item_steps > 0) {

@@ -720,3 +720,13 @@ def test_noncausal_root_rows_are_described_as_seeing_the_whole_root():
     for bad in (dict(save=s), dict(parent=s), dict(leaves=[[1]])):
         with pytest.raises(abi.EspError, match="noncausal"):
             e.pass_begin([host.make_spec(root_len=5, noncausal=1, **bad)])
+
+
+@pytest.mark.parametrize("rows,slots", [(1, 512), (128, 512)])
+def test_tiles_without_a_key_in_sight_are_planned(rows, slots):
+    """A windowed row so far behind its cached keys that it sees none, and no lower bound on what may be split: one tile, no part."""
+    o = host.options_mi355x(rows, slots)
+    o.min_span = 0
+    pos = np.full((1, 4), 10 ** 6, np.int32)
+    tiles, jobs, parts = host.plan_tiles(np.array([(0, 100, 0, 1)], abi.TREE_DT), 8, 64, pos, o)
+    assert len(tiles) == 1 and parts == 0 and len(jobs) == 0
