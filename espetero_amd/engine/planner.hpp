@@ -142,15 +142,17 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
       if (one_round && x.last != y.last) return x.last;
       return x.keys > y.keys;
     });
-    // Every compute unit's own clock advances with the bytes it may pull; the real time follows from how many pull.
-    cu.assign(size_t(cus), Cu{{0, 0}, 0, 0});
+    // Every compute unit's own clock advances with the bytes it may pull; the real time follows from how many pull. (Units
+    // beyond the number of tiles get none: a target of any size is planned in the memory of the tiles.)
+    const int used = int(std::min(size_t(cus), items.size()));
+    cu.assign(size_t(used), Cu{{0, 0}, 0, 0});
     size_t next = 0;
     for (int s = 0; s < per_cu; ++s)
-      for (int c = 0; c < cus && next < items.size(); ++c) cu[size_t(c)].rem[cu[size_t(c)].running++] = items[next++].keys + kFixed;
+      for (int c = 0; c < used && next < items.size(); ++c) cu[size_t(c)].rem[cu[size_t(c)].running++] = items[next++].keys + kFixed;
     using Event = std::pair<double, int>;
     std::priority_queue<Event, std::vector<Event>, std::greater<Event>> q;
     auto next_end = [&](const Cu& x) { return x.since + (x.running == 2 ? 2 * std::min(x.rem[0], x.rem[1]) : x.rem[0]); };
-    for (int c = 0; c < cus; ++c)
+    for (int c = 0; c < used; ++c)
       if (cu[size_t(c)].running) q.push({next_end(cu[size_t(c)]), c});
     idle.clear();
     while (!q.empty()) {

@@ -103,9 +103,10 @@ def plan_tiles(trees, groups, window, pos, options):
     pos_a = None if pos is None else np.ascontiguousarray(pos, dtype=np.int32)
     err = C.create_string_buffer(256)
     nt, nj, npart = C.c_int32(0), C.c_int32(0), C.c_int32(0)
-    # Room for one tile per row group and three resident rounds of parts serves nearly every plan in one call; a plan that needs more
-    # says how many.
-    room = len(trees) + int(trees["M"].sum()) // max(options.rows_per_tile, 1) + 3 * max(options.groups_target // max(groups, 1), 1) + 64
+    # Room for one tile per row group and three resident rounds of parts (of a chip as large as any) serves nearly every plan in one
+    # call; a plan that needs more says how many.
+    rounds = 3 * min(max(options.groups_target // max(groups, 1), 1), 4096)
+    room = len(trees) + int(np.maximum(trees["M"], 0).sum()) // max(options.rows_per_tile, 1) + rounds + 64
     n_tiles = n_jobs = room
     while True:
         tiles = np.empty(n_tiles, abi.TILE_DT)

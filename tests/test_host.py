@@ -730,3 +730,16 @@ def test_tiles_without_a_key_in_sight_are_planned(rows, slots):
     pos = np.full((1, 4), 10 ** 6, np.int32)
     tiles, jobs, parts = host.plan_tiles(np.array([(0, 100, 0, 1)], abi.TREE_DT), 8, 64, pos, o)
     assert len(tiles) == 1 and parts == 0 and len(jobs) == 0
+
+
+def test_a_split_target_of_any_size_is_planned_in_the_memory_of_its_tiles():
+    """Parts as small as they may be, in little memory whatever the target (in a process of its own: the bound is its address space)."""
+    import subprocess
+    import sys
+    code = ("import resource\nresource.setrlimit(resource.RLIMIT_AS, (4 << 30, 4 << 30))\nimport numpy as np\nfrom espetero_amd import abi, host\n"
+            "t, j, p = host.plan_tiles(np.array([(0, 50000, 0, 1), (1, 3000, 0, 1)], abi.TREE_DT), 1, 0, None, host.options_mi355x(1, 2**31 - 1))\n"
+            "print(len(t), len(j), p)")
+    r = subprocess.run([sys.executable, "-c", code], cwd=abi._PKG_DIR + "/..", capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
+    n, jobs, parts = (int(x) for x in r.stdout.split())
+    assert jobs == 2 and parts == n > 200
