@@ -110,6 +110,16 @@ class EspError(RuntimeError):
     pass
 
 
+class PlanGroups(int):
+    """Workgroups per tile, as plan_hint reports them: a plain count, which also knows the layer it was asked for, so that the
+    planner needs no argument of its own for that. A count worked out otherwise is planned for any layer."""
+
+    def __new__(cls, value, params=None):
+        g = super().__new__(cls, value)
+        g.layer = None if params is None else (params.H, params.Hkv, params.head_dim)
+        return g
+
+
 _attn_lib = None
 
 

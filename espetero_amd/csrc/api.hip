@@ -25,8 +25,6 @@ hipError_t launch_chain_advance(esp_tree* trees, int n_trees, int32_t* pos, int3
 hipError_t launch_vt_stage(const esp_attn_params* p, const void* Vb, void* vt, int n_rows, hipStream_t st);
 hipError_t launch_attn_prep(const PrepArgs& a, int n_rows, hipStream_t st);
 hipError_t launch_head_gate(int dt, const GateArgs& a, hipStream_t st);
-int stream_workgroups_per_cu(int HD, int NC);
-int tiled_workgroups_per_cu(int HD);
 int tiled_max_rows(int HD);
 hipError_t stream_init_attributes();
 hipError_t tiled_init_attributes();
@@ -76,11 +74,7 @@ int check_params(const esp_attn_params* p, char* err, size_t errlen) {
 // Which kernel family serves rows_per_tile x G packed rows: 0 none, else the
 // streaming kernel's column tiles (1, 2) or -1 for the tiled kernel.
 int family(const esp_attn_params* p) {
-  const int packed = p->rows_per_tile * (p->H / p->Hkv);
-  const int nc = (packed + 15) / 16;
-  // two column tiles: in one wavefront's registers at head dim 128, as two wavefront pairs of one workgroup at head dim 512
-  if (nc == 1 || (nc == 2 && (p->head_dim == 128 || p->head_dim == 512))) return nc;
-  return -1;
+  return esp::kernel_family(p->head_dim, p->rows_per_tile, p->H / p->Hkv);
 }
 
 struct Carve {

@@ -707,12 +707,6 @@ size_t stream_smem_bytes(int HD, int NC) {
   return size_t(4 * NC * 16) * (HD + 4 + 2) * sizeof(float);
 }
 
-// Resident workgroups per CU of each variant: the single-column-tile head_dim-128 kernel
-// fits two; the wider ones need more than 256 VGPRs and run one.
-constexpr int stream_occ(int HD, int NC) { return (HD == 128 && NC == 1) ? 2 : 1; }  // wavefronts per SIMD
-// Head dim 512: workgroups of one wavefront pair per column tile, one wavefront per SIMD: two pairs fill a compute unit.
-int stream_workgroups_per_cu(int HD, int NC) { return HD >= 512 ? 2 / NC : stream_occ(HD, NC); }
-
 template <int DT, int HD, int NC, int FUSED>
 static hipError_t launch_stream_t(const KArgs& a, const PrepArgs& pa, int n_tiles, hipStream_t st) {
   constexpr int SBU = HD == 128 ? 2 : 1;  // 256 and 512 (256 dims per wavefront): 16-key units

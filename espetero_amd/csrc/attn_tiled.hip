@@ -42,8 +42,6 @@
 
 namespace esp {
 
-constexpr unsigned kComputeUnits = 256;  // of one MI355X
-
 template <int DT, int HD, int OCC>
 __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int n_tiles) {
   constexpr int KS = HD / 16, NT = HD / 32;
@@ -108,7 +106,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   // keys, 32 / 4 heads of 128, whole step: 117.7 us before, 109 so, 73 with the plan that counts on it.) Where every workgroup of the
   // grid has a compute unit to itself nothing is gained, and the second load of the rows behind the tree's record is 1.6 us
   // of an 18.5 us step of short prompts: such passes keep one head per workgroup.
-  const bool packed = rows_live * a.G <= 128 && gridDim.x > kComputeUnits;
+  const bool packed = rows_live * a.G <= 128 && gridDim.x > unsigned(kComputeUnits);
   int m = m_row;
   if (packed && a.G > 1) {
     if (hg != 0) return;
@@ -877,9 +875,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
 }
 
 // Workgroups per compute unit and the largest tile each variant takes.
-constexpr int tiled_occ(int HD) { return HD == 128 ? 2 : 1; }
 int tiled_max_rows(int HD) { return HD == 512 ? 64 : 128; }  // 512: attn_tiled512_kernel's 2 row groups x 2 dim halves
-int tiled_workgroups_per_cu(int HD) { return tiled_occ(HD); }
 size_t tiled_smem_bytes(int HD) { return size_t(4) * 64 * HD * 2 + 64; }  // two stages of K (64 rows) and V^T (64 keys), 16 ints
 
 template <int DT, int HD>

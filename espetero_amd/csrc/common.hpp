@@ -10,6 +10,7 @@
 #include <atomic>
 
 #include "../../include/espetero_attn.h"
+#include "launch_shape.hpp"
 
 namespace esp {
 

@@ -1,0 +1,24 @@
+// How a pass's shape becomes workgroups: the facts of the attention kernels that the host planner counts with too. No device
+// code and no HIP header: the kernels, the C ABI and espetero_amd/engine/planner.hpp read the same lines.
+#pragma once
+
+namespace esp {
+
+constexpr int kComputeUnits = 256;  // of one MI355X
+
+// Which kernel serves rows_per_tile x G packed rows: 1 or 2, the streaming kernel with that many column tiles; -1, the tiled
+// kernel. (Two column tiles: in one wavefront's registers at head dim 128, as two wavefront pairs of one workgroup at head dim 512.)
+constexpr int kernel_family(int head_dim, int rows_per_tile, int G) {
+  const int nc = (rows_per_tile * G + 15) / 16;
+  return nc == 1 || (nc == 2 && (head_dim == 128 || head_dim == 512)) ? nc : -1;
+}
+
+// Resident workgroups per compute unit of each variant: the single-column-tile head_dim-128 kernel fits two; the wider ones
+// need more than 256 VGPRs and run one.
+constexpr int stream_occ(int HD, int NC) { return (HD == 128 && NC == 1) ? 2 : 1; }  // wavefronts per SIMD
+// Head dim 512: workgroups of one wavefront pair per column tile, one wavefront per SIMD: two pairs fill a compute unit.
+constexpr int stream_workgroups_per_cu(int HD, int NC) { return HD >= 512 ? 2 / NC : stream_occ(HD, NC); }
+constexpr int tiled_occ(int HD) { return HD == 128 ? 2 : 1; }
+constexpr int tiled_workgroups_per_cu(int HD) { return tiled_occ(HD); }
+
+}  // namespace esp

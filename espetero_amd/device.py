@@ -56,7 +56,7 @@ def plan_hint3(params, device=0):
     err = C.create_string_buffer(_ERRLEN)
     n, g, r = C.c_int32(0), C.c_int32(0), C.c_int32(0)
     abi.check(abi.attn_lib().esp_attn_plan_hint(C.byref(params), device, C.byref(n), C.byref(g), C.byref(r), err, _ERRLEN), err)
-    return n.value, g.value, r.value
+    return n.value, abi.PlanGroups(g.value, params), r.value
 
 
 def workspace_bytes(params, n_rows, n_parts):

@@ -68,6 +68,12 @@ void esp_plan_options_mi355x(esp_plan_options* o, int32_t rows, int32_t workgrou
 int esp_plan_tiles(const esp_tree* trees, int32_t n_trees, int32_t groups, int32_t window, const int32_t* pos,
                    const esp_plan_options* o, esp_tile* tiles, int32_t tiles_cap, int32_t* n_tiles, esp_combine* jobs,
                    int32_t jobs_cap, int32_t* n_jobs, int32_t* n_parts, char* err, size_t errlen) {
+  return esp_plan_tiles_for(nullptr, trees, n_trees, groups, window, pos, o, tiles, tiles_cap, n_tiles, jobs, jobs_cap, n_jobs, n_parts, err, errlen);
+}
+
+int esp_plan_tiles_for(const esp_attn_params* p, const esp_tree* trees, int32_t n_trees, int32_t groups, int32_t window, const int32_t* pos,
+                       const esp_plan_options* o, esp_tile* tiles, int32_t tiles_cap, int32_t* n_tiles, esp_combine* jobs,
+                       int32_t jobs_cap, int32_t* n_jobs, int32_t* n_parts, char* err, size_t errlen) {
   if (!o || (n_trees > 0 && !trees) || !n_tiles || !n_jobs || !n_parts) return put_err(err, errlen, ESP_EINVAL, "NULL argument");
   if (n_trees < 0 || groups <= 0) return put_err(err, errlen, ESP_EINVAL, "n_trees / groups");
   if (o->rows_per_tile <= 0 || o->groups_target <= 0 || o->granule <= 0 || o->max_splits <= 0 || o->min_chunk <= 0)
@@ -77,7 +83,7 @@ int esp_plan_tiles(const esp_tree* trees, int32_t n_trees, int32_t groups, int32
   try {
     AttnPlan A;
     A.trees.assign(trees, trees + n_trees);
-    plan_tiles(A, groups, window, pos, to_cpp(*o));
+    plan_tiles(A, groups, window, pos, to_cpp(*o), p);
     *n_tiles = int32_t(A.tiles.size());
     *n_jobs = int32_t(A.combine.size());
     *n_parts = A.parts;

@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "../../include/espetero_attn.h"
+#include "../csrc/launch_shape.hpp"
 
 namespace espetero::engine {
 
@@ -84,6 +85,21 @@ struct AttnPlan {
   int rows_per_tile = 8;
 };
 
+// The kernel a pass is planned for, as far as a plan depends on it. family 0: not known.
+struct PlanShape {
+  int family = 0;      // kernel_family()
+  int head_dim = 0;
+  int Hkv = 0, G = 0;  // KV heads, query heads per KV head
+};
+
+// Of the layer's parameters; not known (also) where `groups` is not that kernel's count of workgroups per tile.
+inline PlanShape plan_shape(const esp_attn_params* p, int groups, int rows_per_tile) {
+  if (!p || p->Hkv <= 0 || p->H <= 0 || p->H % p->Hkv) return {};
+  const int G = p->H / p->Hkv, family = esp::kernel_family(p->head_dim, rows_per_tile, G);
+  if (groups != (family > 0 ? p->Hkv : p->H)) return {};
+  return {family, p->head_dim, p->Hkv, G};
+}
+
 struct RowTile {
   int tree, r, k0, b0, span;
   int batch;   // batch keys the tile scans after its cached range (balanced rule: part of its work)
@@ -96,16 +112,30 @@ struct RowTile {
 // What a split costs is worked out by running it: the tiles go to the compute units in the order the hardware will
 // start them, two workgroups on one compute unit share what it can pull (36 GB/s, whether one or two ask), all of them
 // together what memory gives (0.75 of that per unit), every workgroup has a fixed set-up and end, and a pass with any
-// split tile a merge behind it. Those two are kFixed and kMerge, in keys of head dim 128 (two workgroups per compute
-// unit: 512 bytes per key and head) or 256 (one: 1024 bytes): 60 KB and 4.6 us at 36 GB/s. Against 61 measured passes
-// (16 to 96 ragged sequences, head dims 128 and 256, 24 to 258 tiles) this is right within 10 %. Before, a pass that filled more than half of the chip with whole sequences was not split at
-// all: 48 sequences of 60 .. 3000 keys on 8 KV heads 72.5 us (62.6 at 74 tiles), 24 of 300 .. 6000 at head dim 256 175
-// us (114 at 53 tiles).
+// split tile a merge behind it: 60 KB and 4.6 us at 36 GB/s, here in keys. Against 61
+// measured passes (16 to 96 ragged sequences, head dims 128 and 256, 24 to 258 tiles) this is right within 10 %. A pass
+// that fills more than half of the chip with whole sequences gains from a split too: 48 sequences of 60 .. 3000 keys on
+// 8 KV heads 72.5 us whole, 62.6 at 74 tiles.
+// Where the kernel is not known neither is what a key costs: a pass that whole sequences fill less than half is then cut
+// as evenly as fits, without weighing, and for the others the split target has to stand for the key.
 template <typename PartsOf>
-inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const PlanOptions& o, int room, const PartsOf& parts_of) {
+inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const PlanOptions& o, const PlanShape& shape, int room,
+                                     const PartsOf& parts_of) {
   const int n = int(rts.size());
-  const int per_cu = o.groups_target >= 512 ? 2 : 1, cus = std::max(1, room / per_cu);
-  const double kFixed = per_cu == 2 ? 117 : 58, kMerge = per_cu == 2 ? 323 : 161;
+  const bool known = shape.family != 0;
+  const int per_cu = !known              ? (o.groups_target >= 512 ? 2 : 1)
+                     : shape.family > 0 ? esp::stream_workgroups_per_cu(shape.head_dim, shape.family)
+                                        : esp::tiled_workgroups_per_cu(shape.head_dim);
+  const int cus = std::max(1, room / per_cu);
+  // Two column tiles of 128 dims: a key takes its workgroup about twice as long as its bytes do. (One sequence of 300 keys,
+  // 4 rows at 32 / 4 heads: 11.3 us in five parts, which keys of 512 bytes would refuse, 11.8 whole.)
+  const int key_bytes = !known ? (per_cu == 2 ? 512 : 1024) : 4 * shape.head_dim * (shape.head_dim == 128 && shape.family == 2 ? 2 : 1);
+  const double kFixed = 60000 / key_bytes, kMerge = 165600 / key_bytes;
+  // Wavefront pairs of 512 dims reach less of memory together, and a record of theirs is four times a 128-dim one's: no
+  // halves of a resident tile's share. (16 / 2 heads of 512: 130 sequences of 1000 .. 1500 keys 138 us at 255 tiles, 137 at
+  // 385, 141 at 580; 100 of 60 .. 3000 111 us at 247 tiles, 126 at 369; 200 of them 238 us at 256, 285 whole.)
+  const bool wide = known && shape.head_dim == 512;
+  const double kMemory = wide ? 0.6 : 0.75;
   long long total = 0;
   for (const RowTile& rt : rts) total += rt.span + rt.batch;
   std::vector<int> ns(size_t(n), 1), best(size_t(n), 1);
@@ -172,7 +202,7 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
     double t = 0, was = 0;
     size_t pulling = idle.size();
     for (double at : idle) {  // ascending: the queue hands events out in time order
-      t += (at - was) / std::min(1.0, 0.75 * cus / double(pulling--));
+      t += (at - was) / std::min(1.0, kMemory * cus / double(pulling--));
       was = at;
     }
     return t + (split ? kMerge : 0);
@@ -197,6 +227,7 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
       else lo = mid + 1;
     }
     consider(lo * o.granule, 0);
+    if (!known && n <= room / 2) return best;
     consider(whole, 0.95);
   } else {
     consider(whole, 0);
@@ -204,14 +235,17 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
   // Where the compute units end together no other split does better; within 10 % of that none is tried.
   long long n_best = 0;
   for (int k : best) n_best += k;
-  if (least > 1.1 * ((double(total) + kFixed * double(n_best)) / (0.75 * cus) + kMerge))
-    for (const double share : {1.5, 0.75, 0.5}) consider((long long)(double(total) / room * share), 0.95);
+  if (least > 1.1 * ((double(total) + kFixed * double(n_best)) / (kMemory * cus) + kMerge))
+    for (const double share : {1.5, 0.75, 0.5})
+      if (!wide || share > 0.5) consider((long long)(double(total) / room * share), 0.95);
   return best;
 }
 
 // groups: workgroups per tile (KV heads, or KV heads x head splits).
 // window > 0 needs pos (4 ints per row, pos[4 * row] = position).
-inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, const PlanOptions& o) {
+// params: the layer the pass is planned for (may be null: a plan that holds for any).
+inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, const PlanOptions& o, const esp_attn_params* params = nullptr) {
+  const PlanShape shape = plan_shape(params, groups, o.rows_per_tile);
   A.tiles.clear();
   A.combine.clear();
   A.parts = 0;
@@ -327,7 +361,7 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
       }
     }
   } else if (o.balanced && n_tiles > 0) {
-    ns_of = stream_split(rts, o, std::max(1, o.groups_target / std::max(1, groups)), parts_of);
+    ns_of = stream_split(rts, o, shape, std::max(1, o.groups_target / std::max(1, groups)), parts_of);
   }
   // Tiled kernel, a pass with short tiles: records are handed out last to first, and trees in the order of the pass put a
   // long chunk's parts behind short ones, beside which they end alone. By the length of their parts instead, longest

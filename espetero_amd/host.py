@@ -22,6 +22,7 @@ class TreeSpec(C.Structure):
 
 
 _V, _I = C.c_void_p, C.c_int32
+_AP = C.POINTER(abi.AttnParams)
 _ERR = (C.c_char_p, C.c_size_t)
 _PO = C.POINTER(PlanOptions)
 _TS = C.POINTER(TreeSpec)
@@ -30,6 +31,7 @@ ENGINE_SYMBOLS = {
     "esp_plan_options_reference": (None, (_PO,)),
     "esp_plan_options_mi355x": (None, (_PO, _I, _I)),
     "esp_plan_tiles": (C.c_int, (_V, _I, _I, _I, _V, _PO, _V, _I, _IP, _V, _I, _IP, _IP) + _ERR),
+    "esp_plan_tiles_for": (C.c_int, (_AP, _V, _I, _I, _I, _V, _PO, _V, _I, _IP, _V, _I, _IP, _IP) + _ERR),
     "esp_engine_create": (_V, (_I, _I, _I, _I)),
     "esp_engine_destroy": (None, (_V,)),
     "esp_engine_slot_alloc": (C.c_int, (_V,)),
@@ -97,10 +99,16 @@ def options_mi355x(rows, workgroups):
 
 
 def plan_tiles(trees, groups, window, pos, options):
-    """trees: TREE_DT array. Returns (tiles TILE_DT, jobs COMBINE_DT, n_parts)."""
+    """trees: TREE_DT array. groups: plan_hint's, which plans for that layer, or a number, which plans for any.
+    Returns (tiles TILE_DT, jobs COMBINE_DT, n_parts)."""
     lib = engine_lib()
     trees = np.ascontiguousarray(trees, dtype=abi.TREE_DT)
     pos_a = None if pos is None else np.ascontiguousarray(pos, dtype=np.int32)
+    layer = getattr(groups, "layer", None)
+    p = None
+    if layer is not None:
+        p = abi.AttnParams()
+        p.H, p.Hkv, p.head_dim = layer
     err = C.create_string_buffer(256)
     nt, nj, npart = C.c_int32(0), C.c_int32(0), C.c_int32(0)
     # Room for one tile per row group and three resident rounds of parts (of a chip as large as any) serves nearly every plan in one
@@ -111,9 +119,9 @@ def plan_tiles(trees, groups, window, pos, options):
     while True:
         tiles = np.empty(n_tiles, abi.TILE_DT)
         jobs = np.empty(n_jobs, abi.COMBINE_DT)
-        rc = lib.esp_plan_tiles(trees.ctypes.data, len(trees), groups, window, None if pos_a is None else pos_a.ctypes.data,
-                                C.byref(options), tiles.ctypes.data, n_tiles, C.byref(nt), jobs.ctypes.data, n_jobs, C.byref(nj),
-                                C.byref(npart), err, 256)
+        rc = lib.esp_plan_tiles_for(p, trees.ctypes.data, len(trees), groups, window, None if pos_a is None else pos_a.ctypes.data,
+                                    C.byref(options), tiles.ctypes.data, n_tiles, C.byref(nt), jobs.ctypes.data, n_jobs, C.byref(nj),
+                                    C.byref(npart), err, 256)
         if rc != abi.ESP_EWORKSPACE or (nt.value <= n_tiles and nj.value <= n_jobs):
             break
         n_tiles, n_jobs = max(n_tiles, nt.value), max(n_jobs, nj.value)

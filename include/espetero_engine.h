@@ -57,6 +57,13 @@ int esp_plan_tiles(const esp_tree* trees, int32_t n_trees, int32_t groups, int32
                    const esp_plan_options* o, esp_tile* tiles, int32_t tiles_cap, int32_t* n_tiles, esp_combine* jobs,
                    int32_t jobs_cap, int32_t* n_jobs, int32_t* n_parts, char* err, size_t errlen);
 
+/* The same for the layer `p` (its H, Hkv and head_dim are read; NULL: esp_plan_tiles): how much a key weighs and which
+ * tiles the kernel packs into one workgroup per KV head follow from them. With esp_plan_tiles alone, and where groups is
+ * not what esp_attn_plan_hint reports for p at these rows_per_tile, the plan is one that suits any layer. */
+int esp_plan_tiles_for(const esp_attn_params* p, const esp_tree* trees, int32_t n_trees, int32_t groups, int32_t window, const int32_t* pos,
+                       const esp_plan_options* o, esp_tile* tiles, int32_t tiles_cap, int32_t* n_tiles, esp_combine* jobs,
+                       int32_t jobs_cap, int32_t* n_jobs, int32_t* n_parts, char* err, size_t errlen);
+
 /* ---- KV engine: pool + slots + pass builder ---- */
 typedef struct esp_engine esp_engine;
 

@@ -5,7 +5,7 @@ properties those formulas must keep. Integer work: every comparison is exact.
 import numpy as np
 import pytest
 
-from espetero_amd import abi, host
+from espetero_amd import abi, host, synth
 from oracle import host_oracle as ho
 
 
@@ -743,3 +743,44 @@ def test_a_split_target_of_any_size_is_planned_in_the_memory_of_its_tiles():
     assert r.returncode == 0, r.stderr
     n, jobs, parts = (int(x) for x in r.stdout.split())
     assert jobs == 2 and parts == n > 200
+
+
+def _layer_groups(H, Hkv, HD, rows):
+    """What device.plan_hint reports as groups for such a layer (the device is not asked: the count follows from the shape)."""
+    packed = -(-rows * (H // Hkv) // 16)
+    stream = packed == 1 or (packed == 2 and HD in (128, 512))
+    return abi.PlanGroups(Hkv if stream else H, synth.make_params(H, Hkv, HD, abi.ESP_F16, 16, rows_per_tile=rows))
+
+
+@pytest.mark.parametrize("H,Hkv,HD,rows,lens,slots,tiles", [
+    (16, 2, 512, 1, [300], 512, 5),          # a 512-dim key weighs four 128-dim ones: short sequences are worth cutting
+    (16, 2, 512, 1, [150], 512, 3),
+    (16, 2, 512, 1, [350] * 4, 512, 24),
+    (16, 2, 512, 4, [300], 256, 5),          # two wavefront pairs
+    (32, 4, 128, 1, [300], 512, 1),          # a 128-dim one is not,
+    (32, 4, 128, 1, [300], 64, 1),           # nor on a share of the chip
+    (32, 4, 128, 4, [300], 256, 5),          # two column tiles: a key takes twice as long
+    (16, 8, 256, 1, [300], 256, 5),
+])
+def test_streaming_split_weighs_the_keys_of_its_layer(H, Hkv, HD, rows, lens, slots, tiles):
+    """Tiles of short decodes and verify passes, as measured best on the device, through the groups of plan_hint."""
+    trees = np.array([(rows * i, L, 0, rows) for i, L in enumerate(lens)], abi.TREE_DT)
+    got, jobs, parts = host.plan_tiles(trees, _layer_groups(H, Hkv, HD, rows), 0, None, host.options_mi355x(rows, slots))
+    assert len(got) == tiles and parts == (tiles if tiles > len(lens) else 0)
+
+
+def test_streaming_split_for_any_layer_cuts_what_whole_sequences_fill_less_than_half():
+    """Groups as a number: the layer, so the weight of a key, is not known."""
+    o = host.options_mi355x(1, 512)
+    assert [len(host.plan_tiles(np.array([(0, L, 0, 1)], abi.TREE_DT), 2, 0, None, o)[0]) for L in (100, 300, 700)] == [1, 5, 11]
+    g = _layer_groups(16, 2, 512, 1)
+    assert g == 2 and isinstance(g, int) and g.layer == (16, 2, 512) and getattr(g + 0, "layer", None) is None
+
+
+def test_groups_of_another_kernel_are_planned_for_any_layer():
+    """A layer whose kernel has another count of workgroups per tile than `groups` says nothing about the pass."""
+    trees = np.array([(0, 300, 0, 1)], abi.TREE_DT)
+    o = host.options_mi355x(1, 512)
+    odd = abi.PlanGroups(16, synth.make_params(16, 2, 512, abi.ESP_F16, 16))
+    for a, b in zip(host.plan_tiles(trees, odd, 0, None, o), host.plan_tiles(trees, 16, 0, None, o)):
+        assert np.array_equal(a, b)
