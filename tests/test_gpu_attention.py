@@ -222,6 +222,74 @@ def test_sharp_softmax_with_a_moving_maximum(kw, dtype):
     assert err <= 2e-3
 
 
+def _packed_case_errors(c):
+    """(error beyond the stored output's rounding, bound) of every output of a tiled pass against the float64 closed form.
+    What a correct kernel may add: each probability rounded to the storage type before P.V, a relative u of every term
+    (2^-9 bf16, 2^-12 fp16), and the row's sum, of the probabilities before that rounding: together at most
+    u (sum p |v| + |o|). fp16 probabilities below 2^-14 lose more than a relative 2^-12, but no more than 2^-25 each, at a
+    reference up to 2^8 below the row's maximum: 1e-3 covers 2000 keys of |v| < 4; fp32 sums and exponentials are far below."""
+    import copy
+    from gpu_utils import run_case
+    dtype = c.params.dtype
+    got = f32(run_case(c), dtype).astype(np.float64)
+    want = brute(c)
+    a = copy.copy(c)
+    a.Vb, a.pool_ref = c.Vb & 0x7fff, c.pool_ref.copy()
+    a.pool_ref.reshape(c.n_blocks, 2, -1)[:, 1] &= 0x7fff
+    u = 2.0 ** (-9 if dtype == abi.ESP_BF16 else -12)
+    stored = np.abs(want) * u + 2.0 ** -25
+    return np.abs(got - want) - stored, u * (brute(a) + np.abs(want)) + 1e-3
+
+
+@pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
+@pytest.mark.parametrize("kw", [
+    dict(seqs=((700, 1),), H=16),                              # G = 8: one row's eight heads move their reference together
+    dict(seqs=((333, 7),), H=10),                              # G = 5
+    dict(seqs=((0, 16),), H=16),                               # batch keys only, 128 places
+    dict(seqs=((1000, 130),), H=16),                           # a whole tile and a packed remainder of two rows
+    dict(seqs=((700, 5), (200, 1)), H=8, HD=256),              # G = 4, head dim 256
+    dict(seqs=((500, 131),), H=16, HD=256),
+])
+def test_sharp_softmax_of_short_tiles(kw, dtype):
+    """The scores of the test above on tiles whose query heads share a workgroup (a grid of more than a workgroup per compute
+    unit): the rows of several heads move their reference at one moment, each by what it needs. Every output is held to
+    what rounding can have done to it; the 2e-3 of single tests is no bound for the largest of so many bf16 outputs (the
+    kernel reads up to 3.1e-3 on them with and without packed tiles)."""
+    spread = dict(sigma_q=2.0, k_hi=4.0) if dtype == abi.ESP_F16 else dict(sigma_q=1.5, k_hi=3.0)
+    tiles = sum(-(-M // 128) for _, M in kw["seqs"])
+    kw = dict(kw, seqs=kw["seqs"] * -(-257 // (kw["H"] * tiles)))
+    c = sharp_case(53, dtype, **spread, **kw)
+    print(f"case sharp short tiles seqs={c.meta['seqs'][:2]} x {len(c.trees)} HD={c.params.head_dim} dtype={dtype}", flush=True)
+    err, bound = _packed_case_errors(c)
+    worst = float((err / bound).max())
+    print(f"  largest error {err.max():.2e}, {worst:.2f} of its bound", flush=True)
+    assert worst <= 1.0
+
+
+@pytest.mark.parametrize("kw", [dict(seqs=((300, 1), (60, 130)), H=16), dict(seqs=((200, 3), (1100, 1)), H=8, HD=256, dtype=abi.ESP_BF16)])
+@pytest.mark.parametrize("split", [False, True])
+def test_short_tiles_with_a_head_wise_gate(kw, split):
+    """The gate's head is the row's own, whichever workgroup does the tile's work, in the epilogue and in the merge."""
+    import torch
+    from gpu_utils import run_case
+    kw = dict(kw, seqs=kw["seqs"] * -(-257 // (kw["H"] * 2)))
+    c = small_case(seed=47, rows_per_tile=128, **kw)
+    p = c.params
+    g = np.ascontiguousarray(np.random.default_rng(2).standard_normal((c.n_rows, p.H)).astype(np.float32))
+    gd = torch.from_numpy(g).cuda()
+    p.gate, p.gate_ld, p.gate_hs, p.gate_off, p.gate_headwise = gd.data_ptr(), p.H, 1, 0, 1
+    opts = None
+    if split:
+        opts = host.options_mi355x(128, 8192)
+        opts.min_chunk, opts.min_span, opts.item_steps, opts.part_steps = 64, 128, 1, 0
+    print(f"case gated short tiles seqs={c.meta['seqs'][:2]} x {len(c.trees)} HD={p.head_dim} split={split}", flush=True)
+    got = run_case(c, opts)
+    p.gate = g.ctypes.data                # the checker reads the same values from host memory
+    want = oracle_direct(c, threads=8)
+    p.gate, p.gate_headwise = None, 0
+    assert max_abs(got, want, p.dtype) <= tol_for(p.dtype)
+
+
 # ---- head dim 512 prefill: 64-row tiles, wavefront pairs split the dims
 @pytest.mark.parametrize("kw", [
     dict(seqs=((0, 200),), H=4, Hkv=2),                                 # first chunk: batch keys only

@@ -58,6 +58,28 @@ def test_tiled_kernel_reads_its_rows_from_the_pool(kw):
 
 
 @pytest.mark.parametrize("kw", [
+    dict(seqs=((96, 130), (130, 1), (2175, 1)), H=16),                             # G = 8: a remainder of 2 rows, decode rows; the staging ahead of the rows' facts
+    dict(seqs=((32, 16), (48, 16), (80, 144)), H=10, dtype=abi.ESP_BF16),          # G = 5, whole groups of 16 rows
+    dict(seqs=((1024, 128), (128, 144)), H=8, Hkv=2, HD=256),                      # G = 4, head dim 256
+])
+@pytest.mark.parametrize("split", [False, True])
+def test_short_tiles_read_their_rows_from_the_pool(kw, split):
+    """Tiles whose query heads share a workgroup: enough sequences that the grid is more than a workgroup per compute unit."""
+    seqs, base, H = [], 0, kw["H"]
+    while sum(-(-M // 128) for _, M in seqs) * H <= 256:
+        for P, M in kw["seqs"]:
+            P += (base - P) % 16                                                   # P - base a multiple of 16
+            seqs.append((P, M))
+            base += M
+    c = pool_case(64, **{"rows_per_tile": 128, **kw, "seqs": tuple(seqs)})
+    opts = None
+    if split:
+        opts = host.options_mi355x(128, 8192)
+        opts.min_chunk, opts.min_span, opts.item_steps, opts.part_steps = 64, 128, 1, 0
+    _both(c, opts)
+
+
+@pytest.mark.parametrize("kw", [
     dict(seqs=((70, 1), (33, 1), (0, 1), (16, 1)), rows_per_tile=1),               # decode rows at any position of a page
     dict(seqs=((1030, 4), (90, 4)), rows_per_tile=4, desc_fn=lambda M: synth.verify_desc(M, 1)),   # a root and its chain
     dict(seqs=((777, 1), (100, 1)), H=4, Hkv=2, HD=256, rows_per_tile=1),
