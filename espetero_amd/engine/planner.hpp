@@ -102,8 +102,7 @@ inline PlanShape plan_shape(const esp_attn_params* p, int groups, int rows_per_t
 
 struct RowTile {
   int tree, r, k0, b0, span;
-  int batch;   // batch keys the tile scans after its cached range (balanced rule: part of its work)
-  int groups;  // workgroups that work on one part of it
+  int batch;  // batch keys the tile scans after its cached range (balanced rule: part of its work)
 };
 
 // Streaming kernel, balanced rule: the parts of every row tile of a pass. `room`: tiles resident at once (all the KV
@@ -266,12 +265,7 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
       }
       // A causal tile scans the batch rows up to its own last row; one split part takes them all.
       const int batch = o.balanced ? std::max(0, std::min(t.M, r + R) - b0) : 0;
-      // The 128-row tiled kernel gives a short tile - all its query heads' rows together fit one workgroup - one
-      // workgroup per KV head instead of one per query head. How many query heads share a KV head is not known here:
-      // up to 16 rows are taken for short, at four heads per KV head. (The 64-row kernel does not pack. 512 prompt rows
-      // beside 12 decoding sequences, 32 / 4 heads of 128, whole step: 109 us planned as before, 81 so.)
-      const bool packed = o.item_steps > 0 && R > 64 && t.M - r <= 16;
-      rts.push_back({ti, r, k0, b0, t.P - k0, batch, packed ? std::max(1, groups / 4) : groups});
+      rts.push_back({ti, r, k0, b0, t.P - k0, batch});
     }
   }
   const int n_tiles = int(rts.size());
@@ -282,6 +276,8 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
     return cuttable(rt) ? std::clamp<long long>((rt.span + rt.batch + chunk - 1) / chunk, 1, o.max_splits) : 1;
   };
   std::vector<int> ns_of;  // balanced rule: parts of every row tile, once chosen
+  std::vector<int> emit(size_t(n_tiles), 0);  // row tiles in the order their records are written
+  for (int i = 0; i < n_tiles; ++i) emit[size_t(i)] = i;
   if (o.balanced && o.item_steps > 0) {
     // Tiled kernel. A pass is tiles x groups workgroups of unequal length (a causal chunk's later tiles
     // see more keys) on groups_target slots; the hardware hands the next workgroup to the first free slot,
@@ -293,19 +289,63 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
     long long max_work = 1;
     for (const RowTile& rt : rts) max_work = std::max<long long>(max_work, rt.span + rt.batch);
     const long long c_lo = std::max(1, o.min_chunk / o.granule), c_hi = (max_work + o.granule - 1) / o.granule;
+    // A mixed pass: decoding sequences or drafts ride with prompt chunks, in a grid that fills the slots or whose short tiles
+    // the kernel packs. It is run as the kernel runs it: workgroups by the kernel's own rule (the others of a packed tile end at
+    // once), records in an order of their own, and each part at what the merge dispatch costs for its record, 0.6 steps
+    // (passes of chunks alone have few). Of 26 such passes on 2 to 32 KV heads, each timed whole and in ten cuts, this picks a
+    // cut that takes 4 % (head dim 128) and 2 % (256) longer than the pass's best, in geometric mean; without what the merge
+    // costs 8 and 10 %. 512 rows over 2048 keys beside 12 sequences of 200 .. 6000, attention and merge: 90 us whole -> 63
+    // (32 / 4 heads), 90 -> 58 (40 / 8), 130 -> 84 (32 / 32, where nothing is packed). Passes below that fill the chip less
+    // than once and are cut for that already (322 and 124 rows beside 13 sequences, 8 / 2 heads of 256: 56 us, 63 as mixed), and
+    // a chunk's short remainder counted as packed was 2 % slower (eight chunks of 1032 rows over 15360 keys at 16 / 8 heads of
+    // 256: 2577 -> 2630 us): everything else is planned as if nothing were packed, as is every pass whose layer is not known.
+    const long long grid = 1LL * n_tiles * groups;
+    auto live_rows = [&](const RowTile& rt) { return std::min(R, A.trees[size_t(rt.tree)].M - rt.r); };
+    const bool mixed = shape.family < 0 && (grid >= slots || grid > esp::kComputeUnits) &&
+                       std::any_of(rts.begin(), rts.end(), [&](const RowTile& rt) {
+                         return rt.r == 0 && live_rows(rt) <= 16 && esp::tiled_packs(shape.head_dim, live_rows(rt), shape.G, LLONG_MAX);
+                       });
+    // Workgroups that work on one part of a tile in a pass of so many records.
+    auto groups_of = [&](const RowTile& rt, long long records) {
+      return mixed && esp::tiled_packs(shape.head_dim, live_rows(rt), shape.G, records * groups) ? shape.Hkv : groups;
+    };
+    // Records are handed out last to first, and trees in the order of the pass put a long chunk's parts behind those of
+    // decoding sequences, beside which they end alone. In a mixed pass trees go by their longest part, longest last; the tiles
+    // of a tree stay together in their order, since those that run side by side share the tree's keys. (The first three passes
+    // above in the pass's order: 70, 55 and 89 us. Records sorted one by one, in a pass of the eight chunks: 2577 -> 2943 us.)
+    std::vector<int> longest(A.trees.size(), 0);
+    auto order_records = [&](const std::vector<int>& ns_v) {
+      if (!mixed) return;
+      std::fill(longest.begin(), longest.end(), 0);
+      for (int i = 0; i < n_tiles; ++i) {
+        int& part = longest[size_t(rts[size_t(i)].tree)];
+        part = std::max(part, (rts[size_t(i)].span + rts[size_t(i)].batch) / ns_v[size_t(i)]);
+        emit[size_t(i)] = i;
+      }
+      std::stable_sort(emit.begin(), emit.end(), [&](int x, int y) {
+        const int tx = rts[size_t(x)].tree, ty = rts[size_t(y)].tree;
+        return longest[size_t(tx)] != longest[size_t(ty)] ? longest[size_t(tx)] < longest[size_t(ty)] : tx < ty;
+      });
+    };
+    // In tenths of a step.
     auto finish_time = [&](const std::vector<int>& ns_v) {
+      order_records(ns_v);
+      long long records = 0, parts = 0;
+      for (int ns : ns_v) records += ns, parts += ns > 1 ? ns : 0;
       std::priority_queue<long long, std::vector<long long>, std::greater<long long>> free_at;
       for (int i = 0; i < slots; ++i) free_at.push(0);
       long long end = 0;
       for (int i = n_tiles - 1; i >= 0; --i) {
-        const RowTile& rt = rts[size_t(i)];
+        const int at = emit[size_t(i)];
+        const RowTile& rt = rts[size_t(at)];
         const long long work = rt.span + rt.batch;
-        const long long ns = ns_v[size_t(i)];
+        const long long ns = ns_v[size_t(at)];
         const long long per = (work + ns - 1) / ns;
+        const int workgroups = groups_of(rt, records);
         for (long long p = ns - 1; p >= 0; --p) {  // a record's parts in reverse too
           const long long keys = std::min(per, work - p * per);
           const long long cost = o.item_steps + (ns > 1 ? o.part_steps : 0) + (std::max<long long>(keys, 0) + o.granule - 1) / o.granule;
-          for (int g = 0; g < rt.groups; ++g) {
+          for (int g = 0; g < workgroups; ++g) {
             const long long t = free_at.top() + cost;
             free_at.pop();
             free_at.push(t);
@@ -313,19 +353,19 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
           }
         }
       }
-      return end;
+      return 10 * end + (mixed ? 6 * parts : 0);
     };
     std::vector<int> cand(size_t(n_tiles), 1);
     ns_of = cand;
     long long best = finish_time(cand);
     long long items = 0;
-    for (const RowTile& rt : rts) items += rt.groups;
+    for (const RowTile& rt : rts) items += groups_of(rt, n_tiles);
     const long long rounds = items / slots;
     // Fewer workgroups than slots (with cut_batch: no more than slots): one chunk for every tile, the chunks that cut the longest tile into 2 .. 8
     // parts (fewer parts first: ties keep them). With a round or more of whole workgroups such a split was
     // measured slower than none (two workgroups share a compute unit and the older one is served first, so the
-    // slots are less alike than this hand-out takes them to be).
-    for (int parts = 2; parts <= 8 && (rounds == 0 || (o.cut_batch && items <= slots)); ++parts) {
+    // slots are less alike than this hand-out takes them to be); a mixed pass may end on one long sequence all the same.
+    for (int parts = 2; parts <= 8 && (rounds == 0 || mixed || (o.cut_batch && items <= slots)); ++parts) {
       const long long c = std::max(c_lo, (c_hi + parts - 1) / parts) * o.granule;
       for (int i = 0; i < n_tiles; ++i) cand[size_t(i)] = int(parts_of(rts[size_t(i)], c));
       const long long t = finish_time(cand);
@@ -343,7 +383,8 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
       std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
         return rts[size_t(x)].span + rts[size_t(x)].batch < rts[size_t(y)].span + rts[size_t(y)].batch;
       });
-      const int n_tail = int((items - rounds * slots + groups - 1) / groups);
+      int n_tail = 0;
+      for (long long over = items - rounds * slots; over > 0; ++n_tail) over -= groups_of(rts[size_t(order[size_t(n_tail)])], n_tiles);
       for (int most = 3; most <= 6; ++most) {  // parts of the tile with the least work; the others one fewer each, down to 2
         std::fill(cand.begin(), cand.end(), 1);
         bool any = false;
@@ -360,21 +401,9 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
         if (t < best) best = t, ns_of = cand;
       }
     }
+    order_records(ns_of);
   } else if (o.balanced && n_tiles > 0) {
     ns_of = stream_split(rts, o, shape, std::max(1, o.groups_target / std::max(1, groups)), parts_of);
-  }
-  // Tiled kernel, a pass with short tiles: records are handed out last to first, and trees in the order of the pass put a
-  // long chunk's parts behind short ones, beside which they end alone. By the length of their parts instead, longest
-  // last. (Decoding sequences beside prompt chunks, attention alone: 512 rows + 12 sequences at 32 / 4 heads of 128
-  // 70.9 -> 64.8 us; 322 and 124 rows + 13 at 8 / 2 heads of 256 64.2 -> 48.6; 225 rows + 6 64.5 -> 54.4; 81 rows + 6, a pass
-  // that does not fill the chip, 34.9 -> 35.6.)
-  std::vector<int> emit(size_t(n_tiles), 0);
-  for (int i = 0; i < n_tiles; ++i) emit[size_t(i)] = i;
-  if (std::any_of(rts.begin(), rts.end(), [&](const RowTile& rt) { return rt.groups < groups; })) {
-    std::stable_sort(emit.begin(), emit.end(), [&](int x, int y) {
-      auto part = [&](int i) { return (rts[size_t(i)].span + rts[size_t(i)].batch) / std::max(1, ns_of.empty() ? 1 : ns_of[size_t(i)]); };
-      return part(x) < part(y);
-    });
   }
   for (const int index : emit) {
     const RowTile& rt = rts[size_t(index)];

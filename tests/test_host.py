@@ -784,3 +784,79 @@ def test_groups_of_another_kernel_are_planned_for_any_layer():
     odd = abi.PlanGroups(16, synth.make_params(16, 2, 512, abi.ESP_F16, 16))
     for a, b in zip(host.plan_tiles(trees, odd, 0, None, o), host.plan_tiles(trees, 16, 0, None, o)):
         assert np.array_equal(a, b)
+
+
+def _pass_of(seqs):
+    out, base, used = [], 0, 0
+    for P, M in seqs:
+        out.append((base, P, used, M))
+        base += M
+        used += -(-(P + M) // 16)
+    return np.array(out, abi.TREE_DT)
+
+
+def _ones(*cached):
+    return tuple((P, 1) for P in cached)
+
+
+_RIDERS = _ones(*(200 + 480 * i for i in range(12)))
+
+
+@pytest.mark.parametrize("layer,slots,seqs", [
+    ((16, 8, 256), 256, ((15360, 1032),) * 8),                       # chunks with a short remainder
+    ((32, 4, 128), 512, ((3000, 1032),) * 8),
+    ((32, 32, 128), 512, ((3000, 1032),) * 8),
+    ((8, 2, 256), 256, ((2048, 81),) + _RIDERS[:6]),                 # grids of at most 256 workgroups
+    ((8, 2, 256), 256, ((2048, 322), (2048, 124)) + _RIDERS),
+    ((16, 8, 128), 512, ((2048, 256),) + _RIDERS),
+    ((32, 4, 128), 512, ((0, 900), (0, 40), (0, 333))),              # prompts alone
+    ((16, 2, 512), 512, ((2048, 512),) + _RIDERS * 2),               # the kernel of 512 dims packs nothing
+])
+def test_passes_without_packed_riders_are_planned_as_if_nothing_were_packed(layer, slots, seqs):
+    """As a plan for any layer: the same cuts, records tree by tree in the pass's order."""
+    H, Hkv, HD = layer
+    rows, trees = 64 if HD == 512 else 128, _pass_of(seqs)
+    o = host.options_mi355x(rows, slots)
+    got, want = host.plan_tiles(trees, _layer_groups(H, Hkv, HD, rows), 0, None, o), host.plan_tiles(trees, H, 0, None, o)
+    assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    assert (np.diff(want[0]["tree"]) >= 0).all()
+
+
+@pytest.mark.parametrize("layer,slots", [((32, 32, 128), 512), ((32, 16, 128), 512), ((40, 8, 128), 512), ((32, 4, 128), 512), ((24, 4, 256), 256),
+                                         ((16, 16, 256), 256)])
+@pytest.mark.parametrize("seqs", [((2048, 512),) + _RIDERS, _RIDERS[:4] + ((3000, 600),) + _RIDERS[4:] + ((700, 333),), ((1200, 300),) + ((2400, 4), (8400, 16)) * 8,
+                                  ((900, 530),) + _RIDERS])
+def test_mixed_passes_put_the_tree_with_the_longest_part_last(layer, slots, seqs):
+    """Decoding sequences beside chunks, 1 to 8 query heads per KV head: valid records; a tree's records together and in its
+    order; trees by their longest part, which the kernel starts first."""
+    from espetero_amd import device
+    H, Hkv, HD = layer
+    trees = _pass_of(seqs)
+    o = host.options_mi355x(128, slots)
+    tiles, jobs, parts = host.plan_tiles(trees, _layer_groups(H, Hkv, HD, 128), 0, None, o)
+    n_blocks = int(sum(-(-(P + M) // 16) for P, M in seqs))
+    p = synth.make_params(H, Hkv, HD, abi.ESP_F16, 16, rows_per_tile=128)
+    device.validate(p, tiles, trees, jobs, parts, sum(M for _, M in seqs), np.arange(n_blocks, dtype=np.int32), n_blocks)
+    order = [int(t) for i, t in enumerate(tiles["tree"]) if i == 0 or t != tiles["tree"][i - 1]]
+    assert len(order) == len(seqs)                                   # no tree in two pieces
+    def longest(t):
+        x = tiles[tiles["tree"] == t]
+        assert (np.diff(x["r0"]) >= 0).all()
+        work = [(seqs[t][0] + min(seqs[t][1], r - int(trees[t]["base"]) + 128)) // int((x["r0"] == r).sum()) for r in sorted(set(x["r0"].tolist()))]
+        return max(work)
+    by = [longest(t) for t in order]
+    assert by == sorted(by)
+
+
+@pytest.mark.parametrize("layer,slots,seqs,tiles,parts", [
+    # nothing to pack, but one round that ends on its longest sequence: 130 us whole, 84 so
+    ((32, 32, 128), 512, ((2048, 512),) + _ones(3091, 3122, 1154, 528, 240, 736, 802, 233, 236, 5983, 1839, 444), 19, 6),
+    # the chip is full as it is: 184 us whole, 216 .. 278 in cuts
+    ((24, 4, 256), 256, ((4000, 512),) + _ones(*(200 + 190 * i for i in range(30))), 34, 0),
+    # exactly a round of 256: 164 us whole, 66 so
+    ((16, 8, 256), 256, ((60, 700), (900, 333)) + _ones(745, 500, 856, 1247, 502, 807, 5865), 23, 9),
+])
+def test_mixed_passes_are_cut_as_measured(layer, slots, seqs, tiles, parts):
+    """Counted by the kernel's own rule, a part at what its merge costs."""
+    got, jobs, n = host.plan_tiles(_pass_of(seqs), _layer_groups(*layer, 128), 0, None, host.options_mi355x(128, slots))
+    assert (len(got), n) == (tiles, parts)
