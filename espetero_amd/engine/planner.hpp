@@ -116,7 +116,8 @@ struct RowTile {
 // that fills more than half of the chip with whole sequences gains from a split too: 48 sequences of 60 .. 3000 keys on
 // 8 KV heads 72.5 us whole, 62.6 at 74 tiles.
 // Where the kernel is not known neither is what a key costs: a pass that whole sequences fill less than half is then cut
-// as evenly as fits, without weighing, and for the others the split target has to stand for the key.
+// as evenly as fits, without weighing, and for the others the split target has to stand for the key. A target below what the
+// chip holds of the kernel asks for so many tiles: such a pass is cut without weighing too.
 template <typename PartsOf>
 inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const PlanOptions& o, const PlanShape& shape, int room,
                                      const PartsOf& parts_of) {
@@ -125,6 +126,7 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
   const int per_cu = !known              ? (o.groups_target >= 512 ? 2 : 1)
                      : shape.family > 0 ? esp::stream_workgroups_per_cu(shape.head_dim, shape.family)
                                         : esp::tiled_workgroups_per_cu(shape.head_dim);
+  const bool even = !known || o.groups_target < esp::kComputeUnits * per_cu;
   const int cus = std::max(1, room / per_cu);
   // Two column tiles of 128 dims: a key takes its workgroup about twice as long as its bytes do. (One sequence of 300 keys,
   // 4 rows at 32 / 4 heads: 11.3 us in five parts, which keys of 512 bytes would refuse, 11.8 whole.)
@@ -226,7 +228,7 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
       else lo = mid + 1;
     }
     consider(lo * o.granule, 0);
-    if (!known && n <= room / 2) return best;
+    if (even && n <= room / 2) return best;
     consider(whole, 0.95);
   } else {
     consider(whole, 0);

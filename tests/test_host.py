@@ -758,7 +758,8 @@ def _layer_groups(H, Hkv, HD, rows):
     (16, 2, 512, 1, [350] * 4, 512, 24),
     (16, 2, 512, 4, [300], 256, 5),          # two wavefront pairs
     (32, 4, 128, 1, [300], 512, 1),          # a 128-dim one is not,
-    (32, 4, 128, 1, [300], 64, 1),           # nor on a share of the chip
+    (32, 4, 128, 1, [300], 64, 5),           # unless the target is a number of the caller's own
+    (4, 2, 128, 1, [255, 255], 64, 8),
     (32, 4, 128, 4, [300], 256, 5),          # two column tiles: a key takes twice as long
     (16, 8, 256, 1, [300], 256, 5),
 ])
