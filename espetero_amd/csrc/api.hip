@@ -77,21 +77,9 @@ int family(const esp_attn_params* p) {
   return esp::kernel_family(p->head_dim, p->rows_per_tile, p->H / p->Hkv);
 }
 
-struct Carve {
-  size_t parts_o, parts_ml, vt_stage, total;
-};
+using esp::Carve;
 Carve carve(const esp_attn_params* p, int n_rows, int n_parts) {
-  const size_t cols = size_t(p->rows_per_tile) * size_t(p->H / p->Hkv);
-  const size_t recs = size_t(n_parts > 0 ? n_parts : 0) * p->Hkv * cols;
-  auto up = [](size_t x) { return (x + 255) & ~size_t(255); };
-  Carve c;
-  c.parts_o = 0;
-  c.parts_ml = up(recs * p->head_dim * sizeof(float));
-  c.vt_stage = c.parts_ml + up(recs * 2 * sizeof(float));
-  const size_t groups = size_t(n_rows > 0 ? (n_rows + 15) / 16 : 0);
-  c.total = c.vt_stage + (family(p) < 0 ? up(groups * 16 * p->Hkv * p->head_dim * sizeof(uint16_t)) : 0);
-  if (c.total == 0) c.total = 256;
-  return c;
+  return esp::carve_workspace(p->H, p->Hkv, p->head_dim, p->rows_per_tile, n_rows, n_parts);
 }
 
 esp::KArgs make_args(const esp_attn_params* p, const Carve& c, void* workspace, int n_rows) {

@@ -2,6 +2,9 @@
 // code and no HIP header: the kernels, the C ABI and espetero_amd/engine/planner.hpp read the same lines.
 #pragma once
 
+#include <cstddef>
+#include <cstdint>
+
 namespace esp {
 
 constexpr int kComputeUnits = 256;  // of one MI355X
@@ -25,5 +28,23 @@ constexpr int tiled_workgroups_per_cu(int HD) { return tiled_occ(HD); }
 // per query head? Where they fit its 128 places, of a grid that is more than a workgroup per compute unit; why the line lies
 // there: at the kernel. (Head dim 512 has a kernel of its own, which does not.)
 constexpr bool tiled_packs(int HD, int rows, int G, long long grid) { return HD != 512 && rows * G <= 128 && grid > kComputeUnits; }
+
+// Where a pass's partial records and, for the tiled kernels, its transposed batch V lie in the workspace.
+struct Carve {
+  size_t parts_o, parts_ml, vt_stage, total;
+};
+constexpr Carve carve_workspace(int H, int Hkv, int head_dim, int rows_per_tile, int n_rows, int64_t n_parts) {
+  const size_t cols = size_t(rows_per_tile) * size_t(H / Hkv);
+  const size_t recs = size_t(n_parts > 0 ? n_parts : 0) * Hkv * cols;
+  auto up = [](size_t x) { return (x + 255) & ~size_t(255); };
+  Carve c{};
+  c.parts_o = 0;
+  c.parts_ml = up(recs * head_dim * sizeof(float));
+  c.vt_stage = c.parts_ml + up(recs * 2 * sizeof(float));
+  const size_t groups = size_t(n_rows > 0 ? (n_rows + 15) / 16 : 0);
+  c.total = c.vt_stage + (kernel_family(head_dim, rows_per_tile, H / Hkv) < 0 ? up(groups * 16 * Hkv * head_dim * sizeof(uint16_t)) : 0);
+  if (c.total == 0) c.total = 256;
+  return c;
+}
 
 }  // namespace esp

@@ -24,6 +24,7 @@
 #include <climits>
 #include <cstdint>
 #include <functional>
+#include <limits>
 #include <queue>
 #include <vector>
 
@@ -106,7 +107,8 @@ struct RowTile {
 };
 
 // Streaming kernel, balanced rule: the parts of every row tile of a pass. `room`: tiles resident at once (all the KV
-// heads of a tile run side by side, so a tile stands for one workgroup on each of `groups` shares of the chip).
+// heads of a tile run side by side, so a tile stands for one workgroup on each of `groups` shares of the chip). `most_parts`:
+// what esp_attn_forward_static has room for.
 //
 // What a split costs is worked out by running it: the tiles go to the compute units in the order the hardware will
 // start them, two workgroups on one compute unit share what it can pull (36 GB/s, whether one or two ask), all of them
@@ -120,7 +122,7 @@ struct RowTile {
 // chip holds of the kernel asks for so many tiles: such a pass is cut without weighing too.
 template <typename PartsOf>
 inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const PlanOptions& o, const PlanShape& shape, int room,
-                                     const PartsOf& parts_of) {
+                                     long long most_parts, const PartsOf& parts_of) {
   const int n = int(rts.size());
   const bool known = shape.family != 0;
   const int per_cu = !known              ? (o.groups_target >= 512 ? 2 : 1)
@@ -212,12 +214,21 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
   // round for them), or no split where whole sequences already overfill the chip; any other candidate has to win by 5 %,
   // a margin for kernels whose workgroups pull less alone than the model's (two column tiles, wavefront pairs): no
   // split, and chunks of one and a half, three quarters and half of the pass's keys per resident tile.
-  double least = 0;
+  double least = std::numeric_limits<double>::infinity();
   auto consider = [&](long long chunk, double win) {
     chunk = std::max<long long>(chunk, std::max(1, o.min_chunk));
     chunk = (chunk + o.granule - 1) / o.granule * o.granule;
+    // Sequences that fill less than half of the chip are cut into as many tiles as are resident whatever their records take;
+    // any other split (134 sequences at 16 / 2 heads of 512, 4 rows: 268 parts, 34 MB) stays within the library's own array.
+    long long tiles = 0, parts = 0;
+    for (const RowTile& rt : rts) {
+      const long long k = parts_of(rt, chunk);
+      tiles += k;
+      parts += k > 1 ? k : 0;
+    }
+    if ((n > room / 2 || tiles > room) && parts > most_parts) return;
     const double t = time_at(chunk);
-    if (win == 0 || t < win * least) least = t, best = ns;
+    if (t < win * least) least = t, best = ns;
   };
   const long long whole = total + o.min_chunk;
   if (n <= room) {
@@ -227,11 +238,11 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
       if (count_at(mid * o.granule) <= room) hi = mid;
       else lo = mid + 1;
     }
-    consider(lo * o.granule, 0);
+    consider(lo * o.granule, 1);
     if (even && n <= room / 2) return best;
     consider(whole, 0.95);
   } else {
-    consider(whole, 0);
+    consider(whole, 1);
   }
   // Where the compute units end together no other split does better; within 10 % of that none is tried.
   long long n_best = 0;
@@ -277,6 +288,23 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
     // (at least one: with min_span <= 0 a tile that sees no key at all may be asked for)
     return cuttable(rt) ? std::clamp<long long>((rt.span + rt.batch + chunk - 1) / chunk, 1, o.max_splits) : 1;
   };
+  // Parts whose records fit esp_attn_forward_static's array beside what else such a pass keeps there. Where the layer is not
+  // known (only the streaming rule asks then): of the largest records there are, 32 columns of 512 dims on every KV head.
+  auto most_static_parts = [&] {
+    int n_rows = 0;
+    for (const esp_tree& t : A.trees) n_rows = std::max(n_rows, t.base + t.M);
+    if (!shape.family) return (long long)(ESP_STATIC_SCRATCH_BYTES) / (32LL * 514 * 4 * std::max(1, groups));
+    auto fits = [&](long long parts) {
+      return esp::carve_workspace(shape.G * shape.Hkv, shape.Hkv, shape.head_dim, R, n_rows, parts).total <= ESP_STATIC_SCRATCH_BYTES;
+    };
+    long long lo = 0, hi = 1 << 20;
+    while (lo < hi) {
+      const long long mid = (lo + hi + 1) / 2;
+      if (fits(mid)) lo = mid;
+      else hi = mid - 1;
+    }
+    return lo;
+  };
   std::vector<int> ns_of;  // balanced rule: parts of every row tile, once chosen
   std::vector<int> emit(size_t(n_tiles), 0);  // row tiles in the order their records are written
   for (int i = 0; i < n_tiles; ++i) emit[size_t(i)] = i;
@@ -294,46 +322,52 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
     // A mixed pass: decoding sequences or drafts ride with prompt chunks, in a grid that fills the slots or whose short tiles
     // the kernel packs. It is run as the kernel runs it: workgroups by the kernel's own rule (the others of a packed tile end at
     // once), records in an order of their own, and each part at what the merge dispatch costs for its record, 0.6 steps
-    // (passes of chunks alone have few). Of 26 such passes on 2 to 32 KV heads, each timed whole and in ten cuts, this picks a
-    // cut that takes 4 % (head dim 128) and 2 % (256) longer than the pass's best, in geometric mean; without what the merge
-    // costs 8 and 10 %. 512 rows over 2048 keys beside 12 sequences of 200 .. 6000, attention and merge: 90 us whole -> 63
-    // (32 / 4 heads), 90 -> 58 (40 / 8), 130 -> 84 (32 / 32, where nothing is packed). Passes below that fill the chip less
+    // (passes of chunks alone have few). Of 19 such passes on 4 to 32 KV heads, each timed whole and in up to 21 cuts, this picks
+    // one that takes 5 % longer than the best that fits the library's own array, in geometric mean, 21 % at worst (it does not
+    // know that two workgroups slow each other on a compute unit). 512 rows over 2048 keys beside 12 sequences of 200 .. 6000,
+    // attention and merge: 90 us whole -> 60 (32 / 4 heads), 90 -> 61 (40 / 8; 56 in 20 parts, which do not fit), 130 -> 79
+    // (32 / 32, where nothing is packed). Passes below that fill the chip less
     // than once and are cut for that already (322 and 124 rows beside 13 sequences, 8 / 2 heads of 256: 56 us, 63 as mixed), and
     // a chunk's short remainder counted as packed was 2 % slower (eight chunks of 1032 rows over 15360 keys at 16 / 8 heads of
     // 256: 2577 -> 2630 us): everything else is planned as if nothing were packed, as is every pass whose layer is not known.
     const long long grid = 1LL * n_tiles * groups;
     auto live_rows = [&](const RowTile& rt) { return std::min(R, A.trees[size_t(rt.tree)].M - rt.r); };
-    const bool mixed = shape.family < 0 && (grid >= slots || grid > esp::kComputeUnits) &&
-                       std::any_of(rts.begin(), rts.end(), [&](const RowTile& rt) {
-                         return rt.r == 0 && live_rows(rt) <= 16 && esp::tiled_packs(shape.head_dim, live_rows(rt), shape.G, LLONG_MAX);
-                       });
+    bool mixed = shape.family < 0 && (grid >= slots || grid > esp::kComputeUnits) &&
+                 std::any_of(rts.begin(), rts.end(), [&](const RowTile& rt) {
+                   return rt.r == 0 && live_rows(rt) <= 16 && esp::tiled_packs(shape.head_dim, live_rows(rt), shape.G, LLONG_MAX);
+                 });
     // Workgroups that work on one part of a tile in a pass of so many records.
     auto groups_of = [&](const RowTile& rt, long long records) {
       return mixed && esp::tiled_packs(shape.head_dim, live_rows(rt), shape.G, records * groups) ? shape.Hkv : groups;
     };
     // Records are handed out last to first, and trees in the order of the pass put a long chunk's parts behind those of
     // decoding sequences, beside which they end alone. In a mixed pass trees go by their longest part, longest last; the tiles
-    // of a tree stay together in their order, since those that run side by side share the tree's keys. (The first three passes
-    // above in the pass's order: 70, 55 and 89 us. Records sorted one by one, in a pass of the eight chunks: 2577 -> 2943 us.)
+    // of a tree stay together in their order, since those that run side by side share the tree's keys. (Those three passes,
+    // in 20 parts, trees by length and in the pass's order: 60 and 70, 52 and 55, 85 and 98 us. Records sorted one by one, in a pass of the eight chunks: 2577 -> 2943 us.)
     std::vector<int> longest(A.trees.size(), 0);
     auto order_records = [&](const std::vector<int>& ns_v) {
+      for (int i = 0; i < n_tiles; ++i) emit[size_t(i)] = i;
       if (!mixed) return;
       std::fill(longest.begin(), longest.end(), 0);
       for (int i = 0; i < n_tiles; ++i) {
         int& part = longest[size_t(rts[size_t(i)].tree)];
         part = std::max(part, (rts[size_t(i)].span + rts[size_t(i)].batch) / ns_v[size_t(i)]);
-        emit[size_t(i)] = i;
       }
       std::stable_sort(emit.begin(), emit.end(), [&](int x, int y) {
         const int tx = rts[size_t(x)].tree, ty = rts[size_t(y)].tree;
         return longest[size_t(tx)] != longest[size_t(ty)] ? longest[size_t(tx)] < longest[size_t(ty)] : tx < ty;
       });
     };
+    auto parts_in = [](const std::vector<int>& ns_v) {
+      long long k = 0;
+      for (int ns : ns_v) k += ns > 1 ? ns : 0;
+      return k;
+    };
     // In tenths of a step.
     auto finish_time = [&](const std::vector<int>& ns_v) {
       order_records(ns_v);
-      long long records = 0, parts = 0;
-      for (int ns : ns_v) records += ns, parts += ns > 1 ? ns : 0;
+      long long records = 0;
+      for (int ns : ns_v) records += ns;
       std::priority_queue<long long, std::vector<long long>, std::greater<long long>> free_at;
       for (int i = 0; i < slots; ++i) free_at.push(0);
       long long end = 0;
@@ -355,57 +389,75 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
           }
         }
       }
-      return 10 * end + (mixed ? 6 * parts : 0);
+      return 10 * end + (mixed ? 6 * parts_in(ns_v) : 0);
     };
-    std::vector<int> cand(size_t(n_tiles), 1);
-    ns_of = cand;
-    long long best = finish_time(cand);
-    long long items = 0;
-    for (const RowTile& rt : rts) items += groups_of(rt, n_tiles);
-    const long long rounds = items / slots;
-    // Fewer workgroups than slots (with cut_batch: no more than slots): one chunk for every tile, the chunks that cut the longest tile into 2 .. 8
-    // parts (fewer parts first: ties keep them). With a round or more of whole workgroups such a split was
-    // measured slower than none (two workgroups share a compute unit and the older one is served first, so the
-    // slots are less alike than this hand-out takes them to be); a mixed pass may end on one long sequence all the same.
-    for (int parts = 2; parts <= 8 && (rounds == 0 || mixed || (o.cut_batch && items <= slots)); ++parts) {
-      const long long c = std::max(c_lo, (c_hi + parts - 1) / parts) * o.granule;
-      for (int i = 0; i < n_tiles; ++i) cand[size_t(i)] = int(parts_of(rts[size_t(i)], c));
-      const long long t = finish_time(cand);
-      if (t < best) best = t, ns_of = cand;
-    }
-    // A round or more, and some workgroups over (640 on 512 slots): those would run nearly alone at the end.
-    // Only the tiles with the least work are split, just enough of them that the whole ones fill whole rounds,
-    // and their parts fill the slots beside and behind those; the tile dispatched last gets the most parts, so
-    // that the pass ends on short workgroups. (Measured on 2048-row causal chunks over 2048 .. 6144 cached keys:
-    // 5 to 8 % faster than unsplit; splitting fewer tiles than that, so that some whole ones still spill into
-    // another round, was 3 to 6 % slower.)
-    if (rounds >= 1 && items % slots != 0) {
-      std::vector<int> order(size_t(n_tiles), 0);  // tiles by work, least first (ties: dispatched last first)
-      for (int i = 0; i < n_tiles; ++i) order[size_t(i)] = i;
-      std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-        return rts[size_t(x)].span + rts[size_t(x)].batch < rts[size_t(y)].span + rts[size_t(y)].batch;
-      });
-      int n_tail = 0;
-      for (long long over = items - rounds * slots; over > 0; ++n_tail) over -= groups_of(rts[size_t(order[size_t(n_tail)])], n_tiles);
-      for (int most = 3; most <= 6; ++most) {  // parts of the tile with the least work; the others one fewer each, down to 2
-        std::fill(cand.begin(), cand.end(), 1);
-        bool any = false;
-        for (int j = 0; j < n_tail; ++j) {
-          const RowTile& rt = rts[size_t(order[size_t(j)])];
-          const long long cap = std::min<long long>((rt.span + rt.batch) / std::max(1, o.min_chunk), o.max_splits);
-          const int want = std::max(2, most - j);
-          const int ns = rt.span >= o.min_span ? int(std::min<long long>(want, cap)) : 1;
-          cand[size_t(order[size_t(j)])] = std::max(1, ns);
-          any = any || ns > 1;
-        }
-        if (!any) break;
+    // The split that finishes first, of those with no more than `most` parts.
+    std::vector<int> cand;
+    auto choose = [&](long long most) {
+      cand.assign(size_t(n_tiles), 1);
+      ns_of = cand;
+      long long best = finish_time(cand);
+      auto consider = [&] {
+        if (parts_in(cand) > most) return;
         const long long t = finish_time(cand);
         if (t < best) best = t, ns_of = cand;
+      };
+      long long items = 0;
+      for (const RowTile& rt : rts) items += groups_of(rt, n_tiles);
+      const long long rounds = items / slots;
+      // Fewer workgroups than slots (with cut_batch: no more than slots): one chunk for every tile, the chunks that cut the longest tile into 2 .. 8
+      // parts (fewer parts first: ties keep them). With a round or more of whole workgroups such a split was
+      // measured slower than none (two workgroups share a compute unit and the older one is served first, so the
+      // slots are less alike than this hand-out takes them to be).
+      auto cut_at = [&](long long c) {
+        for (int i = 0; i < n_tiles; ++i) cand[size_t(i)] = int(parts_of(rts[size_t(i)], std::max(c_lo, c) * o.granule));
+        consider();
+      };
+      for (int parts = 2; parts <= 8 && !mixed && (rounds == 0 || (o.cut_batch && items <= slots)); ++parts) cut_at((c_hi + parts - 1) / parts);
+      // A mixed pass may end on one long sequence whatever the rounds, and between two of those chunks lie many cuts of it.
+      for (int part = 15; part >= 2 && mixed; --part) cut_at((c_hi * part + 15) / 16);
+      // A round or more, and some workgroups over (640 on 512 slots): those would run nearly alone at the end.
+      // Only the tiles with the least work are split, just enough of them that the whole ones fill whole rounds,
+      // and their parts fill the slots beside and behind those; the tile dispatched last gets the most parts, so
+      // that the pass ends on short workgroups. (Measured on 2048-row causal chunks over 2048 .. 6144 cached keys:
+      // 5 to 8 % faster than unsplit; splitting fewer tiles than that, so that some whole ones still spill into
+      // another round, was 3 to 6 % slower.)
+      if (rounds >= 1 && items % slots != 0) {
+        std::vector<int> order(size_t(n_tiles), 0);  // tiles by work, least first (ties: dispatched last first)
+        for (int i = 0; i < n_tiles; ++i) order[size_t(i)] = i;
+        std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+          return rts[size_t(x)].span + rts[size_t(x)].batch < rts[size_t(y)].span + rts[size_t(y)].batch;
+        });
+        int n_tail = 0;
+        for (long long over = items - rounds * slots; over > 0; ++n_tail) over -= groups_of(rts[size_t(order[size_t(n_tail)])], n_tiles);
+        for (int most = 3; most <= 6; ++most) {  // parts of the tile with the least work; the others one fewer each, down to 2
+          std::fill(cand.begin(), cand.end(), 1);
+          bool any = false;
+          for (int j = 0; j < n_tail; ++j) {
+            const RowTile& rt = rts[size_t(order[size_t(j)])];
+            const long long cap = std::min<long long>((rt.span + rt.batch) / std::max(1, o.min_chunk), o.max_splits);
+            const int want = std::max(2, most - j);
+            const int ns = rt.span >= o.min_span ? int(std::min<long long>(want, cap)) : 1;
+            cand[size_t(order[size_t(j)])] = std::max(1, ns);
+            any = any || ns > 1;
+          }
+          if (!any) break;
+          consider();
+        }
       }
+    };
+    choose(LLONG_MAX);
+    // A mixed pass leaves slots for more parts than it would be cut into with nothing packed, and a part's record has room for a
+    // whole tile (22 parts at 32 / 4 heads: 47 MB). What esp_attn_forward_static took that way it still takes.
+    if (const long long room = most_static_parts(); mixed && parts_in(ns_of) > room) {
+      mixed = false;
+      choose(LLONG_MAX);
+      mixed = true;
+      choose(std::max(room, parts_in(ns_of)));
     }
     order_records(ns_of);
   } else if (o.balanced && n_tiles > 0) {
-    ns_of = stream_split(rts, o, shape, std::max(1, o.groups_target / std::max(1, groups)), parts_of);
+    ns_of = stream_split(rts, o, shape, std::max(1, o.groups_target / std::max(1, groups)), most_static_parts(), parts_of);
   }
   for (const int index : emit) {
     const RowTile& rt = rts[size_t(index)];

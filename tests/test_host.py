@@ -850,14 +850,43 @@ def test_mixed_passes_put_the_tree_with_the_longest_part_last(layer, slots, seqs
 
 
 @pytest.mark.parametrize("layer,slots,seqs,tiles,parts", [
-    # nothing to pack, but one round that ends on its longest sequence: 130 us whole, 84 so
-    ((32, 32, 128), 512, ((2048, 512),) + _ones(3091, 3122, 1154, 528, 240, 736, 802, 233, 236, 5983, 1839, 444), 19, 6),
-    # the chip is full as it is: 184 us whole, 216 .. 278 in cuts
-    ((24, 4, 256), 256, ((4000, 512),) + _ones(*(200 + 190 * i for i in range(30))), 34, 0),
-    # exactly a round of 256: 164 us whole, 66 so
-    ((16, 8, 256), 256, ((60, 700), (900, 333)) + _ones(745, 500, 856, 1247, 502, 807, 5865), 23, 9),
+    # 90 us whole, 60 so, 63 .. 69 in 15 to 32 parts
+    ((32, 4, 128), 512, ((2048, 512),) + _ones(3091, 3122, 1154, 528, 240, 736, 802, 233, 236, 5983, 1839, 444), 20, 7),
+    # nothing to pack, but one round that ends on its longest sequence: 130 us whole, 79 so
+    ((32, 32, 128), 512, ((2048, 512),) + _ones(3091, 3122, 1154, 528, 240, 736, 802, 233, 236, 5983, 1839, 444), 20, 7),
+    # exactly a round of 256: 164 us whole, 63 so
+    ((16, 8, 256), 256, ((60, 700), (900, 333)) + _ones(745, 500, 856, 1247, 502, 807, 5865), 24, 10),
 ])
 def test_mixed_passes_are_cut_as_measured(layer, slots, seqs, tiles, parts):
     """Counted by the kernel's own rule, a part at what its merge costs."""
     got, jobs, n = host.plan_tiles(_pass_of(seqs), _layer_groups(*layer, 128), 0, None, host.options_mi355x(128, slots))
     assert (len(got), n) == (tiles, parts)
+
+
+def _static_scratch(layer, rows, trees, parts):
+    import ctypes as C
+    p = synth.make_params(*layer, abi.ESP_F16, 16, rows_per_tile=rows)
+    return abi.attn_lib().esp_attn_workspace_bytes(C.byref(p), int((trees["base"] + trees["M"]).max()), parts)
+
+
+@pytest.mark.parametrize("layer,rows,slots", [((16, 2, 512), 4, 256), ((16, 2, 512), 2, 512), ((16, 2, 512), 1, 512), ((32, 4, 128), 4, 256), ((16, 8, 256), 8, 256),
+                                              ((40, 8, 128), 1, 512)])
+@pytest.mark.parametrize("known", [True, False])
+def test_streaming_splits_fit_the_static_scratch_array(layer, rows, slots, known):
+    """Default plans of decode and verify passes around and above a full chip: esp_attn_forward_static takes them."""
+    rng = np.random.default_rng(rows)
+    groups = _layer_groups(*layer, rows) if known else layer[1]
+    for lens in [[623] * 134, [38839] * 185, [1404] * 259, [3000] * 100] + [rng.integers(60, hi, n) for n in (20, 65, 100, 130, 200, 260, 400) for hi in (700, 3000, 40000)]:
+        trees = _pass_of([(int(L), rows) for L in lens])
+        parts = host.plan_tiles(trees, groups, 0, None, host.options_mi355x(rows, slots))[2]
+        assert _static_scratch(layer, rows, trees, parts) <= abi.ESP_STATIC_SCRATCH_BYTES, (len(lens), max(lens), parts)
+
+
+@pytest.mark.parametrize("layer,slots", [((32, 4, 128), 512), ((40, 8, 128), 512), ((32, 32, 128), 512), ((24, 4, 256), 256), ((16, 8, 256), 256)])
+@pytest.mark.parametrize("seqs", [((2048, 512),) + _RIDERS, ((2048, 512),) + _RIDERS * 2, ((3000, 600), (700, 333)) + _RIDERS, ((500, 100),) + _RIDERS * 3])
+def test_mixed_passes_fit_the_static_scratch_array_where_they_did(layer, slots, seqs):
+    """Cut for their packed tiles, they take no more than the array or what the plan without such tiles takes."""
+    trees, o = _pass_of(seqs), host.options_mi355x(128, slots)
+    plain = _static_scratch(layer, 128, trees, host.plan_tiles(trees, layer[0], 0, None, o)[2])
+    mixed = _static_scratch(layer, 128, trees, host.plan_tiles(trees, _layer_groups(*layer, 128), 0, None, o)[2])
+    assert mixed <= max(plain, abi.ESP_STATIC_SCRATCH_BYTES)
