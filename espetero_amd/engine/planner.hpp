@@ -96,6 +96,7 @@ struct PlanShape {
 // Of the layer's parameters; not known (also) where `groups` is not that kernel's count of workgroups per tile.
 inline PlanShape plan_shape(const esp_attn_params* p, int groups, int rows_per_tile) {
   if (!p || p->Hkv <= 0 || p->H <= 0 || p->H % p->Hkv) return {};
+  if (p->head_dim != 128 && p->head_dim != 256 && p->head_dim != 512) return {};  // no kernel serves it
   const int G = p->H / p->Hkv, family = esp::kernel_family(p->head_dim, rows_per_tile, G);
   if (groups != (family > 0 ? p->Hkv : p->H)) return {};
   return {family, p->head_dim, p->Hkv, G};

@@ -796,6 +796,17 @@ def _pass_of(seqs):
     return np.array(out, abi.TREE_DT)
 
 
+def test_a_layer_that_no_kernel_serves_is_planned_for_any_layer():
+    """Such parameters are refused when a pass is run; planned, they say nothing of what a key weighs."""
+    trees = np.array([(0, 3000, 0, 1), (1, 900, 0, 1)], abi.TREE_DT)
+    o = host.options_mi355x(1, 512)
+    for head_dim in (0, -128, 64, 100000):
+        g = abi.PlanGroups(4)
+        g.layer = (32, 4, head_dim)
+        for a, b in zip(host.plan_tiles(trees, g, 0, None, o), host.plan_tiles(trees, 4, 0, None, o)):
+            assert np.array_equal(a, b)
+
+
 def _ones(*cached):
     return tuple((P, 1) for P in cached)
 
