@@ -159,7 +159,10 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
   };
   std::vector<Cu> cu;
   std::vector<double> idle;
-  auto time_at = [&](long long chunk) {
+  constexpr double kNever = std::numeric_limits<double>::infinity();
+  double least = kNever;
+  // kNever for a split that is the best so far once more, or cannot end early enough by its keys or by its longest part alone.
+  auto time_at = [&](long long chunk, double win) {
     items.clear();
     bool split = false;
     for (int i = 0; i < n; ++i) {
@@ -171,6 +174,10 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
       for (int p = 0; p + 1 < k && p * step < rt.span; ++p) items.push_back({false, std::min(step, rt.span - p * step)});
       items.push_back({true, std::max(0, work - (k - 1) * step)});
     }
+    long long keys = 0, most = 0;
+    for (const Item& x : items) keys += x.keys, most = std::max<long long>(most, x.keys);
+    const double bound = std::max((double(keys) + kFixed * double(items.size())) / (kMemory * cus), double(most) + kFixed) + (split ? kMerge : 0);
+    if (bound >= win * least || (least < kNever && ns == best)) return kNever;
     const bool one_round = int(items.size()) <= room;
     std::stable_sort(items.begin(), items.end(), [&](const Item& x, const Item& y) {
       if (one_round && x.last != y.last) return x.last;
@@ -215,7 +222,6 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
   // round for them), or no split where whole sequences already overfill the chip; any other candidate has to win by 5 %,
   // a margin for kernels whose workgroups pull less alone than the model's (two column tiles, wavefront pairs): no
   // split, and chunks of one and a half, three quarters and half of the pass's keys per resident tile.
-  double least = std::numeric_limits<double>::infinity();
   auto consider = [&](long long chunk, double win) {
     chunk = std::max<long long>(chunk, std::max(1, o.min_chunk));
     chunk = (chunk + o.granule - 1) / o.granule * o.granule;
@@ -228,7 +234,7 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
       parts += k > 1 ? k : 0;
     }
     if ((n > room / 2 || tiles > room) && parts > most_parts) return;
-    const double t = time_at(chunk);
+    const double t = time_at(chunk, win);
     if (t < win * least) least = t, best = ns;
   };
   const long long whole = total + o.min_chunk;
@@ -243,6 +249,11 @@ inline std::vector<int> stream_split(const std::vector<RowTile>& rts, const Plan
     if (even && n <= room / 2) return best;
     consider(whole, 0.95);
   } else {
+    // Handed out one by one, whole sequences end at most a full unit's last ones after an even share: often near enough as it is.
+    long long most = 0;
+    for (const RowTile& rt : rts) most = std::max<long long>(most, rt.span + rt.batch);
+    const double even_share = (double(total) + kFixed * n) / cus;
+    if (even_share + per_cu * (double(most) + kFixed) <= 1.1 * (even_share + kMemory * kMerge)) return best;
     consider(whole, 1);
   }
   // Where the compute units end together no other split does better; within 10 % of that none is tried.
@@ -369,8 +380,10 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
       order_records(ns_v);
       long long records = 0;
       for (int ns : ns_v) records += ns;
-      std::priority_queue<long long, std::vector<long long>, std::greater<long long>> free_at;
-      for (int i = 0; i < slots; ++i) free_at.push(0);
+      // (when, how many slots): the workgroups of a record are alike and mostly take slots that are.
+      using Free = std::pair<long long, int>;
+      std::priority_queue<Free, std::vector<Free>, std::greater<Free>> free_at;
+      free_at.push({0, slots});
       long long end = 0;
       for (int i = n_tiles - 1; i >= 0; --i) {
         const int at = emit[size_t(i)];
@@ -382,11 +395,14 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
         for (long long p = ns - 1; p >= 0; --p) {  // a record's parts in reverse too
           const long long keys = std::min(per, work - p * per);
           const long long cost = o.item_steps + (ns > 1 ? o.part_steps : 0) + (std::max<long long>(keys, 0) + o.granule - 1) / o.granule;
-          for (int g = 0; g < workgroups; ++g) {
-            const long long t = free_at.top() + cost;
+          for (int left = workgroups; left > 0;) {
+            const Free f = free_at.top();
+            const int take = std::min(left, f.second);
             free_at.pop();
-            free_at.push(t);
-            end = std::max(end, t);
+            if (f.second > take) free_at.push({f.first, f.second - take});
+            free_at.push({f.first + cost, take});
+            end = std::max(end, f.first + cost);
+            left -= take;
           }
         }
       }
