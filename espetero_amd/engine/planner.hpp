@@ -344,22 +344,24 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
     // 256: 2577 -> 2630 us): everything else is planned as if nothing were packed, as is every pass whose layer is not known.
     const long long grid = 1LL * n_tiles * groups;
     auto live_rows = [&](const RowTile& rt) { return std::min(R, A.trees[size_t(rt.tree)].M - rt.r); };
-    bool mixed = shape.family < 0 && (grid >= slots || grid > esp::kComputeUnits) &&
-                 std::any_of(rts.begin(), rts.end(), [&](const RowTile& rt) {
-                   return rt.r == 0 && live_rows(rt) <= 16 && esp::tiled_packs(shape.head_dim, live_rows(rt), shape.G, LLONG_MAX);
-                 });
+    auto is_short = [&](const RowTile& rt) { return live_rows(rt) <= 16 && esp::tiled_packs(shape.head_dim, live_rows(rt), shape.G, LLONG_MAX); };
+    const bool fills = shape.family < 0 && (grid >= slots || grid > esp::kComputeUnits);
+    const bool by_tree = fills && std::any_of(rts.begin(), rts.end(), is_short);
+    bool mixed = fills && std::any_of(rts.begin(), rts.end(), [&](const RowTile& rt) { return rt.r == 0 && is_short(rt); });
     // Workgroups that work on one part of a tile in a pass of so many records.
     auto groups_of = [&](const RowTile& rt, long long records) {
       return mixed && esp::tiled_packs(shape.head_dim, live_rows(rt), shape.G, records * groups) ? shape.Hkv : groups;
     };
     // Records are handed out last to first, and trees in the order of the pass put a long chunk's parts behind those of
-    // decoding sequences, beside which they end alone. In a mixed pass trees go by their longest part, longest last; the tiles
-    // of a tree stay together in their order, since those that run side by side share the tree's keys. (Those three passes,
-    // in 20 parts, trees by length and in the pass's order: 60 and 70, 52 and 55, 85 and 98 us. Records sorted one by one, in a pass of the eight chunks: 2577 -> 2943 us.)
+    // decoding sequences, beside which they end alone. In a pass with short tiles trees go by their longest part, longest last;
+    // the tiles of a tree stay together in their order, since those that run side by side share the tree's keys. (Those three
+    // passes, in 20 parts, by tree and in the pass's order: 60 and 70, 52 and 55, 85 and 98 us. Chunks of 445, 453 and 396 rows on a
+    // period of five sliding layers and a full one, 24 / 4 heads of 256: 609 and 633 us. Records sorted one by one, in a pass of
+    // the eight chunks: 2577 -> 2943 us.)
     std::vector<int> longest(A.trees.size(), 0);
     auto order_records = [&](const std::vector<int>& ns_v) {
       for (int i = 0; i < n_tiles; ++i) emit[size_t(i)] = i;
-      if (!mixed) return;
+      if (!by_tree) return;
       std::fill(longest.begin(), longest.end(), 0);
       for (int i = 0; i < n_tiles; ++i) {
         int& part = longest[size_t(rts[size_t(i)].tree)];

@@ -821,7 +821,7 @@ _RIDERS = _ones(*(200 + 480 * i for i in range(12)))
     ((8, 2, 256), 256, ((2048, 81),) + _RIDERS[:6]),                 # grids of at most 256 workgroups
     ((8, 2, 256), 256, ((2048, 322), (2048, 124)) + _RIDERS),
     ((16, 8, 128), 512, ((2048, 256),) + _RIDERS),
-    ((32, 4, 128), 512, ((0, 900), (0, 40), (0, 333))),              # prompts alone
+    ((32, 4, 128), 512, ((0, 920), (0, 40), (0, 333))),              # prompts alone
     ((16, 2, 512), 512, ((2048, 512),) + _RIDERS * 2),               # the kernel of 512 dims packs nothing
 ])
 def test_passes_without_packed_riders_are_planned_as_if_nothing_were_packed(layer, slots, seqs):
@@ -837,9 +837,10 @@ def test_passes_without_packed_riders_are_planned_as_if_nothing_were_packed(laye
 @pytest.mark.parametrize("layer,slots", [((32, 32, 128), 512), ((32, 16, 128), 512), ((40, 8, 128), 512), ((32, 4, 128), 512), ((24, 4, 256), 256),
                                          ((16, 16, 256), 256)])
 @pytest.mark.parametrize("seqs", [((2048, 512),) + _RIDERS, _RIDERS[:4] + ((3000, 600),) + _RIDERS[4:] + ((700, 333),), ((1200, 300),) + ((2400, 4), (8400, 16)) * 8,
-                                  ((900, 530),) + _RIDERS])
-def test_mixed_passes_put_the_tree_with_the_longest_part_last(layer, slots, seqs):
-    """Decoding sequences beside chunks, 1 to 8 query heads per KV head: valid records; a tree's records together and in its
+                                  ((900, 530),) + _RIDERS,
+                                  ((0, 1400), (0, 40), (0, 333), (0, 900))])     # no sequence decoding, a remainder of 4 rows
+def test_passes_with_short_tiles_put_the_tree_with_the_longest_part_last(layer, slots, seqs):
+    """Decoding sequences or remainders beside chunks, 1 to 8 query heads per KV head: valid records; a tree's records together and in its
     order; trees by their longest part, which the kernel starts first."""
     from espetero_amd import device
     H, Hkv, HD = layer
