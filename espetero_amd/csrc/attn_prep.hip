@@ -32,10 +32,10 @@ namespace esp {
 constexpr int kPrepRows = 8;
 
 template <int DT, int HD>
-__global__ __launch_bounds__(256) void attn_prep_kernel(const PrepArgs a, int n_rows) {
+__global__ __launch_bounds__(256) void attn_prep_kernel(const PrepArgs a, int n_rows, bool deal) {
   constexpr int R = kPrepRows;
   constexpr int LPH = HD / kPrepDims;  // lanes per head
-  constexpr int HPP = 256 / LPH;       // heads of the workgroup
+  constexpr int HPW = 64 / LPH;        // heads of a wavefront
   __shared__ __attribute__((aligned(16))) float2 cs[R][HD / 2];  // (cos, sin) per row and frequency
   const esp_prep_params& p = a.p;
   const int row0 = blockIdx.x * R;
@@ -43,7 +43,8 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(const PrepArgs a, int n_
   const int tid = threadIdx.x;
   const int half = p.rope_dims / 2;
   const int n_slots = p.H + 2 * p.Hkv;
-  const int slot = blockIdx.y * HPP + tid / LPH;  // this lane's head: queries, then keys, then values
+  // This lane's head: queries, then keys, then values
+  const int slot = (deal ? (tid / 64) * int(gridDim.y) + int(blockIdx.y) : 4 * int(blockIdx.y) + tid / 64) * HPW + tid % 64 / LPH;
   const bool live = slot < n_slots;
   const int kind = slot < p.H ? 0 : (slot < p.H + p.Hkv ? 1 : 2);  // q, k, v
   const int h = kind == 0 ? slot : (kind == 1 ? slot - p.H : slot - p.H - p.Hkv);
@@ -163,14 +164,21 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(const PrepArgs a, int n_
 
 hipError_t launch_attn_prep(const PrepArgs& a, int n_rows, hipStream_t st) {
   const int dt = a.p.dtype, HD = a.p.head_dim;
-  const int hpp = 256 / (HD / kPrepDims), n_slots = a.p.H + 2 * a.p.Hkv;
+  const int hpp = 4 * (64 / (HD / kPrepDims)), n_slots = a.p.H + 2 * a.p.Hkv;  // heads of a workgroup's four wavefronts
+  // Few rows, and value heads that are more than one wavefront: the heads are dealt to the rows' workgroups a wavefront at a time.
+  // A value row that goes to a block of its own takes an element store per dim, which consecutive heads put into one workgroup:
+  // 16 decode rows of 16 + 8 + 8 heads of 256 dims 14.1 us, dealt 7.6; 4 rows of 40 + 8 + 8 of 128 5.8 and 5.1. With many rows a
+  // workgroup's consecutive 8 KB of each row read faster: 2048 rows in whole groups 22.8 us, dealt 30.1; the two meet between
+  // 500 and 1000 rows (524: 11.6 and 10.6; 40 + 8 + 8 heads of 128 7.9 and 8.2). Value heads of one wavefront gain nothing
+  // (16 rows of 32 + 4 + 4 of 128 6.4 us, dealt 6.8).
+  const bool deal = n_rows <= 512 && a.p.Hkv > 64 / (HD / kPrepDims);
   const dim3 grid((n_rows + kPrepRows - 1) / kPrepRows, (n_slots + hpp - 1) / hpp), block(256);
-  if (dt == ESP_F16 && HD == 128) launch_timed(attn_prep_kernel<ESP_F16, 128>, grid, block, 0, st, a, n_rows);
-  else if (dt == ESP_F16 && HD == 256) launch_timed(attn_prep_kernel<ESP_F16, 256>, grid, block, 0, st, a, n_rows);
-  else if (dt == ESP_BF16 && HD == 128) launch_timed(attn_prep_kernel<ESP_BF16, 128>, grid, block, 0, st, a, n_rows);
-  else if (dt == ESP_BF16 && HD == 256) launch_timed(attn_prep_kernel<ESP_BF16, 256>, grid, block, 0, st, a, n_rows);
-  else if (dt == ESP_F16 && HD == 512) launch_timed(attn_prep_kernel<ESP_F16, 512>, grid, block, 0, st, a, n_rows);
-  else if (dt == ESP_BF16 && HD == 512) launch_timed(attn_prep_kernel<ESP_BF16, 512>, grid, block, 0, st, a, n_rows);
+  if (dt == ESP_F16 && HD == 128) launch_timed(attn_prep_kernel<ESP_F16, 128>, grid, block, 0, st, a, n_rows, deal);
+  else if (dt == ESP_F16 && HD == 256) launch_timed(attn_prep_kernel<ESP_F16, 256>, grid, block, 0, st, a, n_rows, deal);
+  else if (dt == ESP_BF16 && HD == 128) launch_timed(attn_prep_kernel<ESP_BF16, 128>, grid, block, 0, st, a, n_rows, deal);
+  else if (dt == ESP_BF16 && HD == 256) launch_timed(attn_prep_kernel<ESP_BF16, 256>, grid, block, 0, st, a, n_rows, deal);
+  else if (dt == ESP_F16 && HD == 512) launch_timed(attn_prep_kernel<ESP_F16, 512>, grid, block, 0, st, a, n_rows, deal);
+  else if (dt == ESP_BF16 && HD == 512) launch_timed(attn_prep_kernel<ESP_BF16, 512>, grid, block, 0, st, a, n_rows, deal);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }

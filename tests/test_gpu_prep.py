@@ -129,6 +129,26 @@ def test_prep_folded_append_of_a_prefill_chunk(kind, H, Hkv, HD, dtype, first):
     assert torch.equal(pool.view(torch.int16), want.view(torch.int16)) and bool(pool.any())
 
 
+@pytest.mark.parametrize("kind,H,Hkv,HD", [("gemma", 16, 8, 256), ("omni", 40, 8, 128), ("omni", 5, 5, 128), ("gemma", 3, 3, 256), ("gemma", 16, 2, 512)])
+def test_prep_of_few_rows_deals_its_heads_to_the_workgroups(kind, H, Hkv, HD):
+    """More value heads than a wavefront holds, whole and ragged numbers of heads per workgroup: 512 rows, which deal them a
+    wavefront at a time, give the bits of the first 512 of 513, which do not, in the rows and in the pool (rows in blocks of their
+    own, in whole groups of 8, and nowhere)."""
+    device.init(0)
+    n, bt = 513, 16
+    p, a = synth.make_prep(kind, H, Hkv, HD, abi.ESP_F16, n, seed=14, bt=bt)
+    table = np.full((n, 4), -1, np.int32)
+    table[:200, 0], table[:200, 1] = np.arange(200), (7 * np.arange(200) + 3) % bt
+    table[200:400, 0], table[200:400, 1] = 200 + np.arange(200) // bt, np.arange(200) % bt
+    table[400:500, 2], table[400:500, 3] = 220 + np.arange(100), 5
+    got = []
+    for rows in (512, 513):
+        pool = torch.zeros(320 * 2 * bt * p.kv_ld, dtype=torch.float16, device="cuda")
+        cut = {k: v[:rows] if k in ("X", "pos") else v for k, v in a.items()}
+        got.append([x[:512] for x in _run_gpu(p, cut, rows, table[:rows], pool)] + [pool.view(torch.int16).cpu().numpy()])
+    assert all(np.array_equal(x, y) for x, y in zip(*got)) and all(x.any() for x in got[0])
+
+
 def test_prep_rejects_bad_arguments():
     device.init(0)
     p, a = synth.make_prep("omni", 4, 2, 128, abi.ESP_F16, 4)
