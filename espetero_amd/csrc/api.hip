@@ -570,7 +570,7 @@ static int check_prep(const esp_prep_params* p, bool with_table, const void* kv_
   if (p->q_ld < p->H * HD || p->q_ld % 4 || p->kv_ld < p->Hkv * HD || p->kv_ld % 4)
     return fail(err, errlen, ESP_EINVAL, "q_ld %d / kv_ld %d", p->q_ld, p->kv_ld);
   if (HD == 512 && (p->q_ld % 8 || p->kv_ld % 8)) return fail(err, errlen, ESP_EINVAL, "q_ld %d / kv_ld %d: multiples of 8 at head_dim 512", p->q_ld, p->kv_ld);
-  const int rd = p->rope_dims, rd_min = HD == 512 ? 16 : 8;  // half of rope_dims is a multiple of a lane's 4 consecutive dims (of 8 at head_dim 512)
+  const int rd = p->rope_dims, rd_min = HD == 512 ? 16 : 8;  // as the header states them: half of rope_dims in whole chunks of a lane's 4 dims; of 8 (and strides of 8) at head_dim 512, which this kernel does not need
   if (rd < 0 || rd > HD || (rd != 0 && (rd < rd_min || (rd & (rd - 1)))))
     return fail(err, errlen, ESP_EINVAL, "rope_dims %d: 0 or a power of two in [%d, head_dim]", rd, rd_min);
   if (with_table) {

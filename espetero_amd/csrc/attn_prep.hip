@@ -86,8 +86,9 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(const PrepArgs a, int n_
       xv[r][1] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(xr + pd.b));
     }
   }
-  // Do the 8 rows go to positions ps0 .. ps0 + 7 (ps0 a multiple of 8) of one block, nowhere else? (The table is never
-  // written by a kernel: the same entries for the whole workgroup, read through the scalar cache.)
+  // Do the 8 rows go to positions ps0 .. ps0 + 7 (ps0 a multiple of 8) of one block, nowhere else? (The same entries for the
+  // whole workgroup, read through the scalar cache, as some of the positions below: no kernel writes either while this one
+  // runs. chain_advance_kernel does between the steps of a chain, in a dispatch of its own.)
   using const_int = const int __attribute__((address_space(4)));
   const_int* ents = (const_int*)(a.row_table + row0);
   bool run = a.row_table && rows == R;
