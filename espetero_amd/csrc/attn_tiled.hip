@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   // chunks, a prompt's remainder - is one workgroup per KV head: place x of it is row x / G, query head x % G, and the
   // workgroups of the other heads end here. One head at a time such a tile streams its keys through LDS and the matrix
   // cores G times for a few live rows of 128. (512 prompt rows behind 2048 keys with 12 decoding sequences of 200 .. 6000
-  // keys, 32 / 4 heads of 128, whole step: 117.7 us before, 109 so, 73 with the plan that counts on it.) Where every workgroup of the
+  // keys, 32 / 4 heads of 128, whole step: 122.8 us before, 109 so, 66 with the plan that counts on it.) Where every workgroup of the
   // grid has a compute unit to itself nothing is gained, and the second load of the rows behind the tree's record is 1.6 us
   // of an 18.5 us step of short prompts: such passes keep one head per workgroup.
   const bool packed = tiled_packs(HD, rows_live, a.G, gridDim.x);

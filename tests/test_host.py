@@ -875,6 +875,19 @@ def test_mixed_passes_are_cut_as_measured(layer, slots, seqs, tiles, parts):
     assert (len(got), n) == (tiles, parts)
 
 
+@pytest.mark.parametrize("layer,n,hi,slots", [((40, 8, 128), 48, 3000, 512), ((16, 8, 128), 65, 3000, 512), ((16, 8, 256), 24, 6000, 256),
+                                              ((16, 8, 256), 33, 6000, 256)])
+def test_streaming_split_cuts_ragged_passes_that_nearly_fill_or_overfill_the_chip(layer, n, hi, slots):
+    """On the layer's own kernel: the longest sequence of a ragged batch never ends alone."""
+    lens = np.random.default_rng(n).integers(hi // 40, hi + 1, n)
+    lens[0] = hi
+    tiles, jobs, parts = host.plan_tiles(_pass_of([(int(L), 1) for L in lens]), _layer_groups(*layer, 1), 0, None, host.options_mi355x(1, slots))
+    share = lens.sum() / (slots // layer[1])
+    longest = max(int(x["k1"] - x["k0"]) for x in tiles)
+    assert parts > 0 and longest < hi and longest <= 2.2 * share
+    assert len(tiles) == n + parts - len(jobs)
+
+
 def _static_scratch(layer, rows, trees, parts):
     import ctypes as C
     p = synth.make_params(*layer, abi.ESP_F16, 16, rows_per_tile=rows)
