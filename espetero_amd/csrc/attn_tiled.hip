@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   // keys, 32 / 4 heads of 128, whole step: 122.8 us before, 109 so, 66 with the plan that counts on it.) Where every workgroup of the
   // grid has a compute unit to itself nothing is gained, and the second load of the rows behind the tree's record is 1.6 us
   // of an 18.5 us step of short prompts: such passes keep one head per workgroup.
-  const bool packed = tiled_packs(HD, rows_live, a.G, gridDim.x);
+  const bool packed = tiled_fits(rows_live, a.G) && tiled_packs_grid(gridDim.x);  // tiled_packs of this head dim
   int m = m_row;
   if (packed && a.G > 1) {
     if (hg != 0) return;

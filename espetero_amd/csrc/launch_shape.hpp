@@ -25,9 +25,14 @@ constexpr int tiled_occ(int HD) { return HD == 128 ? 2 : 1; }
 constexpr int tiled_workgroups_per_cu(int HD) { return tiled_occ(HD); }
 
 // Does the tiled kernel give a tile of `rows` live rows one workgroup per KV head, all G query heads' rows in it, instead of one
-// per query head? Where they fit its 128 places, of a grid that is more than a workgroup per compute unit; why the line lies
-// there: at the kernel. (Head dim 512 has a kernel of its own, which does not.)
-constexpr bool tiled_packs(int HD, int rows, int G, long long grid) { return HD != 512 && rows * G <= 128 && grid > kComputeUnits; }
+// per query head? Where they fit its 128 places, and the grid is more than a workgroup per compute unit; why the line lies there:
+// at the kernel. (Head dim 512 has a kernel of its own, which does not.)
+constexpr bool tiled_fits(int rows, int G) { return rows * G <= 128; }
+template <typename N>
+constexpr bool tiled_packs_grid(N grid) {
+  return grid > N(kComputeUnits);
+}
+constexpr bool tiled_packs(int HD, int rows, int G, long long grid) { return HD != 512 && tiled_fits(rows, G) && tiled_packs_grid(grid); }
 
 // Where a pass's partial records and, for the tiled kernels, its transposed batch V lie in the workspace.
 struct Carve {
