@@ -428,22 +428,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
     }
     return;
   }
-  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  uint16_t* op = a.O + size_t(row) * a.q_ld + size_t(h) * kHD + dw;
-  const float* gp = a.gate ? a.gate + size_t(row) * a.gate_ld + size_t(h) * a.gate_hs + a.gate_off + dw * a.gate_ds : nullptr;
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const int dd = 32 * nt + 8 * i4 + 4 * hb;
-      float o[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        o[j] = acc[nt][4 * i4 + j] * inv;
-        if (gp) o[j] = o[j] / (1.0f + __expf(-gp[(dd + j) * a.gate_ds]));
-      }
-      *reinterpret_cast<u32x2*>(op + dd) = u32x2{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])};
-    }
+  store_output<DT>(a, acc, l > 0.0f ? 1.0f / l : 0.0f, row, h, size_t(h) * kHD, dw, hb);
 }
 
 // The dynamic LDS limit of both variants on the current device, ahead of the first launch.

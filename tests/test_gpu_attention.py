@@ -290,6 +290,31 @@ def test_short_tiles_with_a_head_wise_gate(kw, split):
     assert max_abs(got, want, p.dtype) <= tol_for(p.dtype)
 
 
+@pytest.mark.parametrize("HD", [128, 256, 512])
+@pytest.mark.parametrize("headwise", [0, 1])
+def test_tiled_kernels_gate_of_odd_strides(HD, headwise):
+    """A tile's epilogue reads the gate where the caller's strides put it, four dims at a time or one value per head, on full tiles and
+    remainders; gates beyond what exp can hold close the output."""
+    import torch
+    from gpu_utils import run_case
+    c = small_case(seed=48, HD=HD, seqs=((40, 150), (0, 1), (33, 20)), H=4, Hkv=2, rows_per_tile=64 if HD == 512 else 128)
+    p = c.params
+    hs = 3 if headwise else HD + 3
+    ld, off = p.H * hs + 5, 1
+    g = np.random.default_rng(3).standard_normal((c.n_rows, ld)).astype(np.float32)
+    g[::7] = -200.0
+    gd = torch.from_numpy(g).cuda()
+    p.gate, p.gate_ld, p.gate_hs, p.gate_off, p.gate_headwise = gd.data_ptr(), ld, hs, off, headwise
+    print(f"case gate HD={HD} headwise={headwise}", flush=True)
+    got = f32(run_case(c), p.dtype)
+    p.gate, p.gate_headwise = None, 0
+    dims = np.zeros(HD, int) if headwise else np.arange(HD)
+    at = off + hs * np.arange(p.H)[:, None] + dims
+    with np.errstate(over="ignore"):
+        want = brute(c) / (1.0 + np.exp(-g.astype(np.float64)[:, at].reshape(c.n_rows, -1)))
+    assert np.abs(got - want).max() <= 2e-3 and (got[::7] == 0).all()
+
+
 # ---- head dim 512 prefill: 64-row tiles, wavefront pairs split the dims
 @pytest.mark.parametrize("kw", [
     dict(seqs=((0, 200),), H=4, Hkv=2),                                 # first chunk: batch keys only
