@@ -10,26 +10,33 @@
 //
 // Mapping to gfx950. A 512-dim head does not fit one wavefront (32 rows x 512 dims
 // of fp32 accumulators alone are 256 registers), so a workgroup is one tile of up to
-// 64 query rows x one query head, and its 4 wavefronts are 2 row groups x 2 dim
-// halves: wavefront (rg, dh) owns rows 32 rg .. and dims 256 dh .. of them. Keys
-// advance in steps of 32 (two 16-key sub-blocks). Per step a wavefront computes
-//   S^T[32 keys][32 rows] over its 256 dims    v_mfma_f32_32x32x16, A = K from LDS, B = Q^T in registers
-//   the two halves of a row group meet in LDS and are added in one order on both sides
-//   (the reference sums its per-simdgroup score partials the same way, 80_:272-282)
-//   P^T = exp2(S^T - m)                         identical in both wavefronts of the pair
-//   O^T[256 dims][32 rows] += V^T . P^T         A = V^T (its 256 dims) from LDS
-// The next step travels global memory -> the other LDS stage with global_load_lds_dwordx4
-// (no staging registers) while the current step is in the matrix cores.
+// 64 query rows x one query head, and its 4 wavefronts are 2 row groups of 32 rows x 2.
+// Keys advance in steps of 32 (two 16-key sub-blocks). The two wavefronts of a row group
+// share a step's scores by keys and its output by dims: wavefront (rg, w) computes
+//   S^T[16 keys][32 rows] of sub-block w over all 512 dims   v_mfma_f32_16x16x32, A = K from LDS, B = Q^T in registers
+//   P^T = exp2(S^T - m)                                      of its 16 keys, left in LDS in 16 bits
+//   O^T[256 dims][32 rows] += V^T . P^T                      its 256 dims, all 32 keys; A = V^T and B = P^T from LDS
+// (The reference's simdgroups split the dims of the scores and sum partials through threadgroup memory, 80_:272-282. So did
+// this kernel: 4 KB of fp32 partials there and back per wavefront and step and the whole softmax in both wavefronts of a pair,
+// 370 issued instructions around 1024 clocks of matrix work. By keys, 1 KB of P goes through LDS and each score has one owner.)
+// Steps overlap: iteration i multiplies Q K^T of step i and P V of step i - 1, so that one barrier per step publishes the
+// staged data and the P at once and the softmax of step i stands beside P V instructions that do not depend on it. K runs
+// one step ahead of V in the staging (global_load_lds_dwordx4, no staging registers).
+// The row's reference m moves only where a lane's share of a step's sum says so, and in the whole workgroup at once: the two
+// wavefronts of a row group multiply each other's P.
+// What bounds it: one wavefront per SIMD (accumulators 128 registers, Q 128, the rest 130), which issues in order, and the 64 KB a
+// step brings through the compute unit's vector memory path at 64 B per clock. A step of whole cached sub-blocks takes 2150 clocks:
+// 1010 in the 32 instructions of Q K^T (512 clocks) with 12 of a wavefront's 16 loads between them, 690 in 12 of P V (384) with
+// the softmax, 170 in the wait and the barrier, 280 in the last 4 of P V with the other 4 loads; with all 16 loads in a row behind
+// the barrier that stretch alone was 990, with four of them beside P V they landed too late (a wait of 440). Two prompt
+// chunks of 700 .. 1024 rows over 3000 .. 7000 keys, 16 / 2 heads: kernel 412 us before, 325 so (the step's scores by dims halves 3340
+// clocks; a lone branch that moved the reference inside the step's matrix instructions cost 70 register moves in every step).
 //
 // LDS layout: K of stage 0, K of stage 1, V^T of stage 0, V^T of stage 1 (an operand read is a per-lane base
-// register plus an immediate, which takes 16 bits: with a stage's K and V^T side by side the second stage would lie
-// beyond it and every read of it would cost an addition). K of a stage: 32 rows of 1024 bytes, unpadded; the 16-byte chunk c of row r
-// lies at chunk position c ^ (pi(r) & 15), pi = swap of row bits 2 and 3. The lane with S^T
-// row l reads key row pi(l) at position c ^ (l & 15): 16 consecutive lanes hit 16 different
-// positions, and with the rows permuted by pi the 8 P values a lane packs for one P.V
-// instruction are 8 consecutive keys, which is how V^T lies in memory. V^T per sub-block:
-// [dim][2 halves of 8 keys], the two 16-byte halves of dim d swapped when bit 3 of d is set
-// (lanes d and d + 8 of an operand read would otherwise share banks).
+// register plus an immediate, which takes 16 bits), P. K of a stage: 32 rows of 1024 bytes, unpadded; the 16-byte chunk c of
+// row r of a sub-block lies at chunk position c ^ r: the 16 lanes that read a chunk of 16 rows hit 16 different positions.
+// V^T per sub-block: [dim][2 halves of 8 keys], the two 16-byte halves of dim d swapped when bit 3 of d is set
+// (lanes d and d + 8 of an operand read would otherwise share banks). P: [row][32 keys], rows 80 bytes apart.
 #include <utility>
 
 #include "common.hpp"
@@ -38,23 +45,23 @@
 namespace esp {
 
 namespace {
-constexpr int kHD = 512, kHW = 256;                  // dims of a head; dims one wavefront multiplies and accumulates
+constexpr int kHD = 512, kHW = 256;                  // dims of a head; dims one wavefront accumulates
 constexpr int kKStage = 32 * kHD * 2;                // K of one stage: 32 rows
 constexpr int kVSub = kHD * 32;                      // V^T of one sub-block
 constexpr int kVStage = 2 * kVSub;                   // V^T of one stage: two sub-blocks
-constexpr int kVBase = 2 * kKStage;                  // layout: K stage 0, K stage 1, V^T stage 0, V^T stage 1 - every operand read is
-                                                     // a per-lane base plus an immediate below 64 KB, whichever the stage
-constexpr int kStage = kKStage + kVStage;
-constexpr int kXch = 4 * 4 * 64 * 16;                // partial S^T: [wavefront][4][lane] 16-byte pieces
-constexpr int kLds = 2 * kStage + kXch + 64;         // two stages, the exchange, 16 ints
+constexpr int kVBase = 2 * kKStage;                  // layout: K stage 0, K stage 1, V^T stage 0, V^T stage 1
+constexpr int kPRow = 80, kPBuf = 2 * 32 * kPRow;    // P of one step: 2 row groups x 32 rows
+constexpr int kPBase = kVBase + 2 * kVStage;
+constexpr int kMax = kPBase + 2 * kPBuf;             // a row's maximum in either wavefront: [row group][wavefront][32] floats
+constexpr int kFlags = kMax + 2 * 2 * 32 * 4;        // [buffer][wavefront] ints
+constexpr int kLds = kFlags + 2 * 4 * 4;
 }  // namespace
 
 template <int DT>
 __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, int n_tiles) {
-  constexpr int KS = kHW / 16, NT = kHW / 32;
+  constexpr int NT = kHW / 32, KK = kHD / 32;
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  f32x4* xch = reinterpret_cast<f32x4*>(lds + 2 * kStage);
-  int(*red)[4] = reinterpret_cast<int(*)[4]>(lds + 2 * kStage + kXch);
+  int(*flags)[4] = reinterpret_cast<int(*)[4]>(lds + kFlags);
 
   // Workgroup -> (KV head, head in group, tile): consecutive ids differ in KV head first, the heads
   // sharing a KV head land on the same XCD's L2; tiles run last to first (longest key ranges first).
@@ -66,8 +73,9 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rg = wave >> 1, dw = (wave & 1) * kHW;
-  const int l32 = lane & 31, hb = lane >> 5;
+  const int rg = wave >> 1, half = wave & 1, dw = half * kHW;
+  const int l32 = lane & 31, hb = lane >> 5;   // P V: this lane's row of the group, half of a sub-block's keys
+  const int c16 = lane & 15, q4 = lane >> 4;   // scores: rows c16 and 16 + c16 of the group, keys 4 q4 .. + 3 of sub-block `half`
   esp_tile tile = a.tiles[tile_i];
   const esp_tree tree = a.trees[tile.tree];
   if (tile.k1 == INT32_MAX) tile.k1 = tree.P;  // open-ended range: up to the tree's cached length as it is now
@@ -76,29 +84,33 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
   const int rows_live = min(a.R, end - tile.r0);
   const int rr0 = tile.r0 - tree.base;
 
-  // ---- this lane's row and its Q fragments (this wavefront's dims)
-  const int m_row = 32 * rg + l32;
-  const bool row_ok = m_row < rows_live;
-  const int row = row_ok ? tile.r0 + m_row : tile.r0;
-  const int rr = rr0 + m_row;
-  const int4 d = a.desc ? a.desc[row] : make_int4(0, 0, 0, 0);
-  const int qpos = a.window > 0 ? a.pos[row].x : 0;
-  u32x4 qf[KS];
-  {
-    const uint16_t* qp = a.Q + size_t(row) * a.q_ld + size_t(h) * kHD + dw + 8 * hb;
+  // ---- this lane's two rows of the scores and their Q fragments
+  int rr[2], qpos[2];
+  int4 d[2];
+  u32x4 qf[2][KK];
+  int kl = -1;  // the last batch key they see
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = row_ok ? *reinterpret_cast<const u32x4*>(qp + 16 * ks) : u32x4{0, 0, 0, 0};
+  for (int rt = 0; rt < 2; ++rt) {
+    const int m = 32 * rg + 16 * rt + c16;
+    const bool ok = m < rows_live;
+    const int row = ok ? tile.r0 + m : tile.r0;
+    rr[rt] = rr0 + m;
+    d[rt] = a.desc ? a.desc[row] : make_int4(0, 0, 0, 0);
+    qpos[rt] = a.window > 0 ? a.pos[row].x : 0;
+    const uint16_t* qp = a.Q + size_t(row) * a.q_ld + size_t(h) * kHD + 8 * q4;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) qf[rt][kk] = ok ? *reinterpret_cast<const u32x4*>(qp + 32 * kk) : u32x4{0, 0, 0, 0};
+    if (ok) kl = max(kl, max(rr[rt], max(d[rt].z - 1, a.bidi ? d[rt].w - 1 : -1)));
   }
 
   // ---- the last batch key any row of the tile sees
   int k_last = -1;
   {
-    int kl = row_ok ? max(rr, max(d.z - 1, a.bidi ? d.w - 1 : -1)) : -1;
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) kl = max(kl, __shfl_xor(kl, o));
-    if (lane == 0) red[wave][0] = kl;
+    for (int o = 8; o >= 1; o >>= 1) kl = max(kl, __shfl_xor(kl, o));  // the lanes of a quarter hold all rows
+    if (lane == 0) flags[0][wave] = kl;
     __syncthreads();
-    k_last = max(max(red[0][0], red[1][0]), max(red[2][0], red[3][0]));
+    k_last = max(flags[0][0], flags[0][2]);
     k_last = __builtin_amdgcn_readfirstlane(min(min(k_last, tree.M - 1), tile.last >= 2 ? tile.last - 2 : INT32_MAX));  // last >= 2: the part's batch range ends at row last - 2
   }
 
@@ -116,8 +128,8 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
   const int pool_shift = tree.P - tree.base;
 
   // ---- staging, 16 bytes per lane straight into LDS. K: this wavefront brings rows 4 wave .. + 3 of each
-  // sub-block; the lane that fills chunk position `lane` of row r brings chunk lane ^ (pi(r) & 15), and
-  // pi(4 wave + q) = pi(4 wave) + q. V^T: this wavefront brings pieces 256 wave .. + 255 of each sub-block's
+  // sub-block; the lane that fills chunk position `lane` of row r brings chunk lane ^ r.
+  // V^T: this wavefront brings pieces 256 wave .. + 255 of each sub-block's
   // 1024 (piece c: keys 8 (c % 2) .. + 7 of dim c / 2); position p holds piece p ^ ((p >> 4) & 1).
   const uint32_t lds_base = uint32_t(uintptr_t(lds));
   // Pool addresses of the sub-blocks, 64 at a time: lane l holds the byte address of the K rows of sub-block adr0 + l
@@ -143,38 +155,54 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
     const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(kadr_lo), idx)), hi = uint32_t(__builtin_amdgcn_readlane(int(kadr_hi), idx));
     return reinterpret_cast<const char*>(uint64_t(lo) | (uint64_t(hi) << 32));
   };
-  const uint32_t kx = uint32_t(swap23(4 * wave));
+  const uint32_t kx = uint32_t(4 * wave);
   const uint32_t voff = uint32_t((lane ^ ((lane >> 4) & 1)) << 4);
-  // plain: the caller knows that both sub-blocks of the step are cached keys.
-  auto fill = [&](int step, int stage, auto plain) __attribute__((always_inline)) {
+  // Staging of a step whose sub-blocks the pool holds: where this wavefront's share of the K of sub-block t lies (and, bt rows' worth
+  // of bytes behind it, of its V^T: kept for an iteration later), and two of its four loads of either. fill_k and fill_v: all four, whatever
+  // the sub-block (v_src null: past the range).
+  const char* k_src = nullptr;
+  const char* v_src[2] = {nullptr, nullptr};
+  auto locate_k = [&](int t, int step) __attribute__((always_inline)) {
+    k_src = pool_k(2 * step + t) + wave * 4096;
+    v_src[t] = k_src + size_t(a.bt) * 1024;  // the 16-token sub-block: 16 KB contiguous
+  };
+  auto load_k = [&]<int H>(int t, int stage) __attribute__((always_inline)) {
+    const uint32_t kl = uint32_t(lane);
+    load_to_lds16_x2<H>(k_src, (kl ^ (kx + 2 * H)) << 4, (kl ^ (kx + 2 * H + 1)) << 4, lds_base + stage * kKStage + (16 * t + 4 * wave) * 1024);
+  };
+  auto load_v = [&]<int H>(int t, int stage) __attribute__((always_inline)) {
+    load_to_lds16_x2<H>(v_src[t], voff, voff, lds_base + kVBase + stage * kVStage + t * kVSub + wave * 4096);
+  };
+  auto fill_k = [&](int t, int step, int stage) __attribute__((always_inline)) {
+    const int sidx = 2 * step + t;
+    if (sidx < n_c || (in_pool && sidx < n_sb)) {
+      locate_k(t, step);
+      load_k.template operator()<0>(t, stage);
+      load_k.template operator()<1>(t, stage);
+    } else if (sidx < n_sb) {
+      const int g = a0 + (sidx - n_c);
+      const int lim = a.n_rows - 1 - 16 * g;  // batch rows past the pass's last row do not exist: repeat the last (masked)
+      const char* kb = reinterpret_cast<const char*>(a.Kb + size_t(16 * g) * a.kv_ld + size_t(kvh) * kHD);
+      v_src[t] = reinterpret_cast<const char*>(a.vt_stage + (size_t(kvh) * n_groups + g) * size_t(kHD) * 16) + wave * 4096;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int sidx = 2 * step + t;
-      const uint32_t kdst = lds_base + stage * kKStage + (16 * t + 4 * wave) * 1024;
-      const uint32_t vdst = lds_base + kVBase + stage * kVStage + t * kVSub + wave * 4096;
-      const uint32_t kl = uint32_t(lane);
-      if (decltype(plain)::value || sidx < n_c || (in_pool && sidx < n_sb)) {
-        const char* kb = pool_k(sidx) + wave * 4096;
-        const char* vb = kb + size_t(a.bt) * 1024;  // the 16-token sub-block: 16 KB contiguous
-        load_to_lds16_x4(kb, (kl ^ kx) << 4, (kl ^ (kx + 1)) << 4, (kl ^ (kx + 2)) << 4, (kl ^ (kx + 3)) << 4, kdst);
-        load_to_lds16_x4(vb, voff, voff, voff, voff, vdst);
-      } else if (sidx < n_sb) {
-        const int g = a0 + (sidx - n_c);
-        const int lim = a.n_rows - 1 - 16 * g;  // batch rows past the pass's last row do not exist: repeat the last (masked)
-        const char* kb = reinterpret_cast<const char*>(a.Kb + size_t(16 * g) * a.kv_ld + size_t(kvh) * kHD);
-        const char* vb = reinterpret_cast<const char*>(a.vt_stage + (size_t(kvh) * n_groups + g) * size_t(kHD) * 16) + wave * 4096;
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          load_to_lds16(kb + size_t(min(4 * wave + q, lim)) * size_t(a.kv_ld) * 2, (kl ^ (kx + q)) << 4, kdst + q * 1024);
-        load_to_lds16_x4(vb, voff, voff, voff, voff, vdst);
-      } else {  // past the range: K stays whatever it was (S is masked), V^T must be finite
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          *reinterpret_cast<u32x4*>(lds + kVBase + stage * kVStage + t * kVSub + wave * 4096 + q * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
-      }
+      for (int q = 0; q < 4; ++q)
+        load_to_lds16(kb + size_t(min(4 * wave + q, lim)) * size_t(a.kv_ld) * 2, (uint32_t(lane) ^ (kx + q)) << 4,
+                      lds_base + stage * kKStage + (16 * t + 4 * wave + q) * 1024);
+    } else {
+      v_src[t] = nullptr;  // past the range: K stays whatever it was (S is masked)
     }
   };
-  // After this wavefront's loads of `step` have landed: cached keys outside [k0, k1) may be memory
+  auto fill_v = [&](int t, int stage) __attribute__((always_inline)) {
+    if (v_src[t]) {
+      load_v.template operator()<0>(t, stage);
+      load_v.template operator()<1>(t, stage);
+    } else {  // V^T must be finite
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<u32x4*>(lds + kVBase + stage * kVStage + t * kVSub + wave * 4096 + q * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+    }
+  };
+  // After this wavefront's loads of V^T of `step` have landed: cached keys outside [k0, k1) may be memory
   // never written; their V must not reach the products.
   auto fix = [&](int step, int stage) __attribute__((always_inline)) {
 #pragma unroll
@@ -214,205 +242,280 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
   // ---- operand reads: LDS byte addresses (base register + immediate)
   using lds_u32x4 = const __attribute__((address_space(3))) u32x4;
   auto lds_ptr = [](uint32_t addr) __attribute__((always_inline)) { return reinterpret_cast<lds_u32x4*>(addr); };
-  // K slice ks = 8 g + j of this wavefront's dims is chunk dw / 8 + 16 g + 2 j + hb of key row pi(l32).
-  uint32_t kaddr[8];
-  {
-    const int prow = (l32 & 0x13) | ((l32 & 4) << 1) | ((l32 & 8) >> 1);  // pi(l32)
+  // K slice kk is chunk 4 kk + q4 of key row c16 of sub-block `half`.
+  uint32_t kaddr[4];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) kaddr[j] = lds_base + uint32_t(prow * 1024 + dw * 2 + (((2 * j + hb) ^ (l32 & 15)) << 4));
-  }
+  for (int j = 0; j < 4; ++j) kaddr[j] = lds_base + uint32_t((16 * half + c16) * 1024 + (((4 * j + q4) ^ c16) << 4));
   // V^T operand nt of sub-block t: keys 8 hb .. + 7 of dim dw + 32 nt + l32.
   const uint32_t vaddr = lds_base + uint32_t(kVBase + (dw + l32) * 32 + ((hb ^ ((l32 >> 3) & 1)) << 4));
+  // P operand of sub-block t: keys 8 hb .. + 7 of row l32. This lane's own P: keys 4 q4 .. + 3 of sub-block `half`, rows c16 and 16 + c16.
+  const uint32_t paddr = lds_base + uint32_t(kPBase + (32 * rg + l32) * kPRow + 16 * hb);
+  char* const p_own = lds + kPBase + (32 * rg + c16) * kPRow + 32 * half + 8 * q4;
 
   f32x16 acc[NT];
-  float m_run = -INFINITY, l_run = 0.0f;  // l_run: this lane's share (16 of every 32 keys) of the row's sum
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[nt][i] = 0.0f;
+  // Per score row of this lane: the running reference in log2 units of the scaled score (-inf: no key seen yet), what is
+  // subtracted for it, and this lane's share of the row's sum. Without a reference kUnset is subtracted: the first visible score
+  // gives an infinite P and with it a sum that asks for one, and keys the row does not see give 0 as always. ps: the lane's share of the
+  // sum of the step whose P is in LDS, not yet in l_run.
+  constexpr float kUnset = -1e30f;
+  float m_run[2], m_sub[2], l_run[2], ps[2];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    m_run[rt] = -INFINITY;
+    m_sub[rt] = kUnset;
+    l_run[rt] = ps[rt] = 0.0f;
+  }
+  f32x4 s[2];        // scores of the step: s[rt][e] is key 4 q4 + e of sub-block `half`, row 16 rt + c16
+  u32x4 ring[2][4];  // operands on their way from LDS
+  int out_of_range = 0;  // did any lane of the workgroup find its share of the last step's sum beyond 2^8?
 
-  // A step's matrix work is 32 operand reads from LDS, each feeding one matrix instruction, in 4 groups of 8
-  // through two register buffers: K slices 0..7, K slices 8..15, V^T of sub-block 0, V^T of sub-block 1.
-  // The reads of a group are in flight while the matrix cores consume the group before it; the V^T reads
-  // do not depend on the softmax and cover the exchange of the partial scores.
-  //
-  // At the top of iteration i stage i % 2 holds step i, step i + 1 is on its way into the other stage and
-  // the first group of K slices of step i is being read. The iteration: both score groups, the exchange,
-  // the softmax - its second sub-block's share laid between the first sub-block's P V instructions - then,
-  // every operand of the step now in registers, the wait for the own loads of step i + 1, the barrier that
-  // publishes them, the request for step i + 2 into the stage just left, the first reads of step i + 1, and
-  // only then the second sub-block's P V instructions: they cover the barrier, the address arithmetic of the
-  // loads and the first read latency. (A wavefront issues in order: a matrix instruction hides only what
-  // stands right behind it.)
-  u32x4 ring[2][8];
-  auto read_k0 = [&]<int S>(std::integral_constant<int, S>) __attribute__((always_inline)) {
+  // P of the step's scores into buffer `buf`, and this lane's shares of its sums. The row sum is that of the rounded P the products
+  // use: under a lazily moved reference the dominant P is not exactly 1, and O = sum(P~ v) / sum(P~) keeps its rounding out of
+  // a row that one key dominates. No maximum is taken: all P >= 0, so a share of the sum <= 2^8 bounds every one of them.
+  auto exp_pack = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) ring[0][j] = *lds_ptr(kaddr[j] + uint32_t(S * kKStage));
-  };
-  // plain: steps `step` .. `step + 2` are cached keys wholly inside [k0, k1) of a layer without a window: every key is
-  // visible to every row, nothing staged needs fixing up, one kind of load.
-  auto iter = [&]<int S>(int step, std::integral_constant<int, S>, auto plain) __attribute__((always_inline)) {
+    for (int rt = 0; rt < 2; ++rt) {
+      float p[4];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) ring[1][j] = *lds_ptr(kaddr[j] + uint32_t(S * kKStage + 256));
-    __builtin_amdgcn_sched_barrier(0);
-    // s[4 i + j] is S^T row 8 i + 4 hb + j, which is key 16 (i / 2) + 8 hb + 4 (i % 2) + j of the step:
-    // s[8 t + e] is key 8 hb + e of sub-block t.
-    f32x16 s;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s = mfma32x16<DT>(ring[0][j], qf[j], s);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) ring[0][j] = *lds_ptr(vaddr + uint32_t(S * kVStage + j * 1024));
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s = mfma32x16<DT>(ring[1][j], qf[8 + j], s);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) ring[1][j] = *lds_ptr(vaddr + uint32_t(S * kVStage + kVSub + j * 1024));
-    // The other half of the dims: through LDS, added in the same order in both wavefronts of the pair.
-#pragma unroll
-    for (int v = 0; v < 4; ++v) xch[(wave * 4 + v) * 64 + lane] = f32x4{s[4 * v], s[4 * v + 1], s[4 * v + 2], s[4 * v + 3]};
-    __syncthreads();
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const f32x4 o = xch[((wave ^ 1) * 4 + v) * 64 + lane];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) s[4 * v + j] = (wave & 1) ? o[j] + s[4 * v + j] : s[4 * v + j] + o[j];
+      for (int e = 0; e < 4; ++e) p[e] = fast_exp2(__builtin_fmaf(s[rt][e], a.scale_log2, -m_sub[rt]));
+      const u32x2 w = {pack2<DT>(p[0], p[1]), pack2<DT>(p[2], p[3])};
+      ps[rt] = sum2<DT>(w.y, sum2<DT>(w.x, 0.0f));
+      *reinterpret_cast<u32x2*>(p_own + buf * kPBuf + 16 * rt * kPRow) = w;
     }
-    // ---- visibility
+  };
+  // Some lane of the workgroup found a reference too low for the step whose P is in buffer `buf` (or not set): every row takes
+  // the maximum of that step over both wavefronts of its group, moves its reference, rescales what is accumulated, and the step's P is
+  // written again. Every wavefront of the workgroup comes through here together.
+  auto settle = [&](int buf) __attribute__((always_inline)) {
+    asm volatile("s_nop 0");  // a real branch: this block must not be speculated into the loop body
+    float* mx_sh = reinterpret_cast<float*>(lds + kMax) + rg * 64;
+    float mx[2];
 #pragma unroll
-    for (int t = 0; t < (decltype(plain)::value ? 0 : 2); ++t) {
-      const int sidx = 2 * step + t;
-      const bool cached = sidx < n_c, batch = !cached && sidx < n_sb;
-      const int j0 = cached ? (c0 + sidx) << 4 : ((a0 + sidx - n_c) << 4) - tree.base;
-      if (cached && a.window == 0 && j0 >= tile.k0 && j0 + 16 <= tile.k1) continue;  // every key visible to every row
-      // Visible keys of the sub-block for this lane's row: j in [lo, hi], or 0 <= j < anc.
+    for (int rt = 0; rt < 2; ++rt) {
+      mx[rt] = fmaxf(fmaxf(s[rt][0], s[rt][1]), fmaxf(s[rt][2], s[rt][3]));
+      mx[rt] = fmaxf(mx[rt], __shfl_xor(mx[rt], 16));
+      mx[rt] = fmaxf(mx[rt], __shfl_xor(mx[rt], 32));
+      if (q4 == 0) mx_sh[half * 32 + 16 * rt + c16] = mx[rt];
+    }
+    __syncthreads();
+    float corr[2];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      const float other = mx_sh[(half ^ 1) * 32 + 16 * rt + c16];
+      const float m_new = fmaxf(m_run[rt], fmaxf(mx[rt], other) * a.scale_log2);  // scale > 0: the max commutes with it
+      corr[rt] = (m_run[rt] == -INFINITY) ? 1.0f : fast_exp2(m_run[rt] - m_new);  // nothing accumulated without a reference
+      m_run[rt] = m_new;
+      m_sub[rt] = (m_new == -INFINITY) ? kUnset : m_new;
+      l_run[rt] *= corr[rt];
+    }
+    const float c = (lane & 16) ? corr[1] : corr[0];  // of row l32
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[nt] *= c;
+    exp_pack(buf);
+    __syncthreads();
+  };
+  // Visibility of the step's keys of this wavefront's sub-block.
+  auto mask = [&](int step) __attribute__((always_inline)) {
+    const int sidx = 2 * step + half;
+    const bool cached = sidx < n_c, batch = !cached && sidx < n_sb;
+    const int j0 = cached ? (c0 + sidx) << 4 : ((a0 + sidx - n_c) << 4) - tree.base;
+    if (cached && a.window == 0 && j0 >= tile.k0 && j0 + 16 <= tile.k1) return;  // every key visible to every row
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      // Visible keys of the sub-block for this row: j in [lo, hi], or b0 <= j < anc.
       int lo, hi, anc = 0;
       if (cached) {
         lo = tile.k0;
         hi = tile.k1 - 1;
-        if (a.window > 0) lo = max(lo, qpos - a.window + 1);
+        if (a.window > 0) lo = max(lo, qpos[rt] - a.window + 1);
       } else if (batch) {
-        lo = max(d.x, tile.b0);  // below b0 (the window's lower edge over the tile's rows) nothing is visible
-        hi = min(k_last, (a.bidi && d.w > 0) ? max(rr, d.w - 1) : rr);
-        anc = min(d.z, k_last + 1);
+        lo = max(d[rt].x, tile.b0);  // below b0 (the window's lower edge over the tile's rows) nothing is visible
+        hi = min(k_last, (a.bidi && d[rt].w > 0) ? max(rr[rt], d[rt].w - 1) : rr[rt]);
+        anc = min(d[rt].z, k_last + 1);
       } else {
         lo = 1;
         hi = 0;
       }
-      const int jb = j0 + 8 * hb;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int j = jb + e;
+      for (int e = 0; e < 4; ++e) {
+        const int j = j0 + 4 * q4 + e;
         bool vis = (j >= lo && j <= hi) || (j >= tile.b0 && j < anc);
-        if (batch && a.window > 0 && vis) vis = qpos - a.pos[tree.base + j].x < a.window;
-        s[8 * t + e] = vis ? s[8 * t + e] : -INFINITY;
+        if (batch && a.window > 0 && vis) vis = qpos[rt] - a.pos[tree.base + j].x < a.window;
+        s[rt][e] = vis ? s[rt][e] : -INFINITY;
       }
     }
-    // ---- online softmax; the two lanes of a row (hb = 0, 1) agree on the maximum. The running reference
-    // m_run only moves when some row's maximum exceeds it by more than 8 (log2 units): P stays below
-    // 2^8 and the 128 accumulator registers are rescaled a handful of times per row.
-    float mx = -INFINITY;
+  };
+  auto mul_v = [&](const u32x4 (&buf)[4], int nt0, u32x4 p) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
-    mx *= a.scale_log2;  // scale > 0: the max commutes with it
-    if (__any(mx > m_run + 8.0f)) {
-      const float m_new = fmaxf(m_run, fmaxf(mx, __shfl_xor(mx, 32)));
-      const float corr = (m_new == -INFINITY) ? 1.0f : fast_exp2(m_run - m_new);  // m_run = -inf -> 0: nothing accumulated yet
-      l_run *= corr;
+    for (int j = 0; j < 4; ++j) acc[nt0 + j] = mfma32x16<DT>(buf[j], p, acc[nt0 + j]);
+  };
+
+  // Iteration i. At its top the barrier has been passed that publishes K of step i, V^T and P of step i - 1; the first sub-block of V^T
+  // of step i is on its way, and so are the first K operands. It requests the rest of V^T of step i and K of step i + 1, multiplies
+  // Q K^T of step i, then P V of step i - 1 but for four instructions, with the softmax of step i between them, and leaves P of step i.
+  // Those four instructions stand behind the barrier that publishes it and cover the first reads and requests of the next.
+  // plain: every key of steps i and i + 1 is a cached key inside [k0, k1) of a layer without a window, i >= 1, and no reference has to
+  // move. The loads stand between the matrix instructions there, two at a time.
+  auto iter = [&](int i, auto plain) __attribute__((always_inline)) {
+    constexpr bool PLAIN = decltype(plain)::value;
+    const int S = i & 1;
+    auto read_k = [&](u32x4 (&buf)[4], uint32_t off) __attribute__((always_inline)) {
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) acc[nt] *= corr;
-      m_run = m_new;
-    }
-    const float m_safe = (m_run == -INFINITY) ? 0.0f : m_run;
-    u32x4 pb[2];
-    float ps = 0.0f;
-    // The row sum is that of the rounded P the products use: under a lazily moved reference the dominant P is
-    // not exactly 1, and O = sum(P~ v) / sum(P~) keeps its rounding out of a row that one key dominates.
-    auto exp_pack = [&]<int T>(std::integral_constant<int, T>) __attribute__((always_inline)) {
-      float p[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) p[e] = fast_exp2(__builtin_fmaf(s[8 * T + e], a.scale_log2, -m_safe));
-      pb[T] = u32x4{pack2<DT>(p[0], p[1]), pack2<DT>(p[2], p[3]), pack2<DT>(p[4], p[5]), pack2<DT>(p[6], p[7])};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ps = sum2<DT>(pb[T][e], ps);
+      for (int j = 0; j < 4; ++j) buf[j] = *lds_ptr(kaddr[j] + off);
     };
-    exp_pack(std::integral_constant<int, 0>{});
-    __builtin_amdgcn_sched_barrier(0);
-    // ---- O^T += V^T . P^T over this wavefront's dims: the first sub-block's products, the second sub-block's
-    // exponentials between them
+    const uint32_t koff = uint32_t(S * kKStage);
+    const uint32_t va = vaddr + uint32_t((S ^ 1) * kVStage), pa = paddr + uint32_t((S ^ 1) * kPBuf);
+    auto read_v = [&](u32x4 (&buf)[4], int t, int nt0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma32x16<DT>(ring[0][nt], pb[0], acc[nt]);
-    exp_pack(std::integral_constant<int, 1>{});
-    asm volatile("" : "+v"(pb[1]), "+v"(ps));  // worked out here, not where pb[1] is first used
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+      for (int j = 0; j < 4; ++j) buf[j] = *lds_ptr(va + uint32_t(t * kVSub + (nt0 + j) * 1024));
+    };
+    if constexpr (!PLAIN) {
+      if (i > 0 && out_of_range) settle(S ^ 1);
+      fill_v(1, S);
+      if (i + 1 < n_steps) {
+        fill_k(0, i + 1, S ^ 1);
+        fill_k(1, i + 1, S ^ 1);
+      }
     }
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      l_run[rt] += ps[rt];
+      s[rt] = f32x4{0, 0, 0, 0};
+    }
+    u32x4 pf[2], carry[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      if (g < 3) {
+        read_k(ring[(g + 1) & 1], koff + uint32_t(256 * (g + 1)));
+      } else {
+        read_v(ring[0], 0, 0);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) pf[t] = *lds_ptr(pa + uint32_t(32 * t));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) s[rt] = mfma16x32<DT>(ring[g & 1][j], qf[rt][4 * g + j], s[rt]);
+        if (PLAIN && (j & 1)) {
+          const int slot = 2 * g + (j >> 1);
+          __builtin_amdgcn_sched_barrier(0);
+          if (slot == 0) load_v.template operator()<0>(1, S);
+          if (slot == 1) load_v.template operator()<1>(1, S);
+          if (slot == 2) locate_k(0, i + 1), load_k.template operator()<0>(0, S ^ 1);
+          if (slot == 3) load_k.template operator()<1>(0, S ^ 1);
+          if (slot == 4) locate_k(1, i + 1), load_k.template operator()<0>(1, S ^ 1);
+          if (slot == 5) load_k.template operator()<1>(1, S ^ 1);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    read_v(ring[1], 0, 4);
     __builtin_amdgcn_sched_barrier(0);
-    l_run += ps;
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // own loads of step + 1 landed, own reads of stage S done
-    if constexpr (decltype(plain)::value) {
-      __syncthreads();
-      fill(step + 2, S, plain);
-      read_k0(std::integral_constant<int, S ^ 1>{});
+    if constexpr (!PLAIN) {
+      mfma_settle(s[0]);
+      mfma_settle(s[1]);
+      mask(i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (PLAIN || i > 0) {
+      mul_v(ring[0], 0, pf[0]);
+      read_v(ring[0], 1, 0);
+      mul_v(ring[1], 4, pf[0]);
+      read_v(carry, 1, 4);
+      if constexpr (PLAIN) exp_pack(S);
+      mul_v(ring[0], 0, pf[1]);
+    }
+    if constexpr (PLAIN) {
+#pragma unroll
+      for (int j = 0; j < 12; ++j) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
     } else {
-      if (step + 1 < n_steps) fix(step + 1, S ^ 1);
-      __syncthreads();
-      if (step + 2 < n_steps) fill(step + 2, S, plain);
-      if (step + 1 < n_steps) read_k0(std::integral_constant<int, S ^ 1>{});
+      exp_pack(S);
+    }
+    const int mine = __any(!(ps[0] <= 256.0f) || !(ps[1] <= 256.0f));
+    if (lane == 0) flags[S][wave] = mine;
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // own loads landed, own reads of this iteration's stages done
+    if constexpr (!PLAIN) fix(i, S);
+    __syncthreads();
+    const u32x4 fl = *lds_ptr(lds_base + uint32_t(kFlags + S * 16));
+    read_k(ring[0], koff ^ uint32_t(kKStage));
+    __builtin_amdgcn_sched_barrier(0);
+    auto left = [&](int j) __attribute__((always_inline)) {
+      if (PLAIN || i > 0) acc[4 + j] = mfma32x16<DT>(carry[j], pf[1], acc[4 + j]);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    left(0);
+    left(1);
+    if constexpr (PLAIN) {
+      load_v.template operator()<0>(0, S ^ 1);
+    } else {
+      if (i + 1 < n_steps) fill_v(0, S ^ 1);
     }
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma32x16<DT>(ring[1][nt], pb[1], acc[nt]);
+    left(2);
+    left(3);
+    if constexpr (PLAIN) load_v.template operator()<1>(0, S ^ 1);
     __builtin_amdgcn_sched_barrier(0);
+    out_of_range = __builtin_amdgcn_readfirstlane(int(fl.x | fl.y | fl.z | fl.w));
   };
   constexpr std::false_type general{};
   constexpr std::true_type plain{};
   if (n_steps > 0) {
-    fill(0, 0, general);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) fill_k(t, 0, 0);
     wait_loads();
-    fix(0, 0);
-  }
-  __syncthreads();
-  if (n_steps > 1) fill(1, 1, general);
-  if (n_steps > 0) read_k0(std::integral_constant<int, 0>{});
-  {
-    // Plain iterations: pairs of steps i, i + 1 whose steps up to i + 3 are sub-blocks wholly inside the cached range.
-    int p0 = 0, p1 = 0;  // iterations [p0, p1), both even
-    if (a.window == 0 && n_c > 0) {
-      const int sb_lo = (tile.k0 & 15) ? 1 : 0, sb_hi = n_c - ((tile.k1 & 15) ? 1 : 0);  // sub-blocks [sb_lo, sb_hi) are whole
-      p0 = (((sb_lo + 1) >> 1) + 1) & ~1;
-      const int last = (sb_hi >> 1) - 3;  // last iteration i with 2 (i + 2) + 1 < sb_hi
-      p1 = last >= p0 ? p0 + ((last + 1 - p0) & ~1) : p0;
-    }
-    int i = 0;
+    fill_v(0, 0);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ring[0][j] = *lds_ptr(kaddr[j]);
+    // Plain iterations lie below p1: steps up to i + 1 are sub-blocks wholly inside the cached range.
+    const int p1 = a.window == 0 && n_c > 0 ? ((n_c - ((tile.k1 & 15) ? 1 : 0)) >> 1) - 1 : 0;
+    for (int i = 0; i < n_steps;) {
+      iter(i++, general);
 #pragma nounroll
-    for (; i + 2 <= min(p0, n_steps); i += 2) {
-      iter(i, std::integral_constant<int, 0>{}, general);
-      iter(i + 1, std::integral_constant<int, 1>{}, general);
+      for (; i < p1 && !out_of_range; ++i) iter(i, plain);
     }
-    if (i == p0) {
-#pragma nounroll
-      for (; i + 2 <= p1; i += 2) {
-        iter(i, std::integral_constant<int, 0>{}, plain);
-        iter(i + 1, std::integral_constant<int, 1>{}, plain);
+    // ---- what is left: P V of the last step
+    const int S = (n_steps - 1) & 1;
+    if (out_of_range) settle(S);
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) l_run[rt] += ps[rt];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const u32x4 p = *lds_ptr(paddr + uint32_t(S * kPBuf + 32 * t));
+#pragma unroll
+      for (int nt0 = 0; nt0 < NT; nt0 += 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ring[0][j] = *lds_ptr(vaddr + uint32_t(S * kVStage + t * kVSub + (nt0 + j) * 1024));
+        mul_v(ring[0], nt0, p);
       }
     }
-#pragma nounroll
-    for (; i + 2 <= n_steps; i += 2) {
-      iter(i, std::integral_constant<int, 0>{}, general);
-      iter(i + 1, std::integral_constant<int, 1>{}, general);
-    }
-    if (i < n_steps) iter(i, std::integral_constant<int, 0>{}, general);
   }
 
-  // ---- output: lane (row l32, half hb) holds dims dw + 32 nt + 8 i + 4 hb + j at acc[nt][4 i + j]
-  const float l = l_run + __shfl_xor(l_run, 32);
-  if (!row_ok) return;
+  // ---- output: lane (row l32, half hb) holds dims dw + 32 nt + 8 i + 4 hb + j at acc[nt][4 i + j]. Its row's sum: over the
+  // lanes that share the row, then over both wavefronts of the group.
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    l_run[rt] += __shfl_xor(l_run[rt], 16);
+    l_run[rt] += __shfl_xor(l_run[rt], 32);
+  }
+  float* l_sh = reinterpret_cast<float*>(lds + kMax) + rg * 64;
+  const float l_mine = (lane & 16) ? l_run[1] : l_run[0], m_mine = (lane & 16) ? m_run[1] : m_run[0];
+  __syncthreads();
+  if (hb == 0) l_sh[half * 32 + l32] = l_mine;
+  __syncthreads();
+  const float l = half ? l_sh[l32] + l_mine : l_mine + l_sh[32 + l32];
+  const int m_row = 32 * rg + l32;
+  const int row = tile.r0 + m_row;
+  if (m_row >= rows_live) return;
   if (tile.part >= 0) {
     const size_t rec = (size_t(tile.part) * a.Hkv + kvh) * a.cols + size_t(m_row) * a.G + hg;
     float* po = a.parts_o + rec * kHD + dw;
@@ -423,7 +526,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
         *reinterpret_cast<f32x4*>(po + 32 * nt + 8 * i4 + 4 * hb) =
             f32x4{acc[nt][4 * i4], acc[nt][4 * i4 + 1], acc[nt][4 * i4 + 2], acc[nt][4 * i4 + 3]};
     if (hb == 0 && dw == 0) {
-      a.parts_ml[rec * 2] = m_run;
+      a.parts_ml[rec * 2] = m_mine;
       a.parts_ml[rec * 2 + 1] = l;
     }
     return;

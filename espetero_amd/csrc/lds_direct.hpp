@@ -41,6 +41,31 @@ __device__ __forceinline__ void load_to_lds16_x4(const void* base, uint32_t o0, 
       : "s"(lds_addr), "v"(o0), "v"(o1), "v"(o2), "v"(o3), "s"(base)
       : "memory");
 }
+// Two of the four: the first pair (H = 0) or the second, for code that lays them between other instructions.
+template <int H>
+__device__ __forceinline__ void load_to_lds16_x2(const void* base, uint32_t o0, uint32_t o1, uint32_t lds_addr) {
+  lds_addr = uint32_t(__builtin_amdgcn_readfirstlane(int(lds_addr)));
+  const uint64_t b64 = reinterpret_cast<uint64_t>(base);
+  const uint32_t b_lo = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(b64))));
+  const uint32_t b_hi = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(b64 >> 32))));
+  base = reinterpret_cast<const void*>(uint64_t(b_lo) | (uint64_t(b_hi) << 32));
+  if constexpr (H == 0)
+    asm volatile(
+        "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %3\n\t"
+        "global_load_lds_dwordx4 %2, %3 offset:1024"
+        :
+        : "s"(lds_addr), "v"(o0), "v"(o1), "s"(base)
+        : "memory");
+  else
+    asm volatile(
+        "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %3 offset:2048\n\t"
+        "global_load_lds_dwordx4 %2, %3 offset:3072"
+        :
+        : "s"(lds_addr), "v"(o0), "v"(o1), "s"(base)
+        : "memory");
+}
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // s_waitcnt immediates (gfx9 layout): only the LDS / scalar-memory counter, at most 8 or 0 outstanding.

@@ -335,6 +335,34 @@ def test_tiled_kernel_head_dim_512(kw):
     _check(small_case(seed=44, HD=512, **{"rows_per_tile": 64, **kw}))
 
 
+@pytest.mark.parametrize("kw", [
+    dict(seqs=((0, 1), (16, 1), (31, 2), (33, 40))),                    # one to three steps: no overlap yet, then the first of each kind
+    dict(seqs=((64, 64), (96, 33), (130, 64))),                         # even and odd counts of steps, whole and partial ones
+    dict(seqs=((400, 64), (333, 40)), window=40),                       # rows that see nothing of their tile's first steps
+    dict(seqs=((0, 150),), window=17),
+])
+@pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
+def test_tiled_kernel_head_dim_512_few_steps(kw, dtype):
+    """A step's scores and the P V products of the step before run side by side: what begins and ends that."""
+    _check(small_case(seed=49, HD=512, H=4, Hkv=2, rows_per_tile=64, dtype=dtype, **kw))
+
+
+@pytest.mark.parametrize("HD,rows", [(128, 128), (512, 64)])
+def test_tiled_kernel_scores_far_below_zero(HD, rows):
+    """Every score is near -650 log2 units: nothing of it survives an exponential before the row has a reference. Equal queries of -20 against
+    keys near 1 leave weights that the brute force works out from the same storage values."""
+    from gpu_utils import run_case
+    c = small_case(seed=50, HD=HD, H=4, Hkv=2, seqs=((100, 70),), rows_per_tile=rows, scale=HD ** -0.5)
+    rng = np.random.default_rng(51)
+    near_one = lambda shape: synth._bits((1.0 + 0.05 * rng.standard_normal(shape)).astype(np.float32), c.params.dtype)  # noqa: E731
+    c.Q[:] = synth._bits(np.full(c.Q.shape, -20.0 * (512 / HD) ** 0.5, np.float32), c.params.dtype)
+    c.Kb[:] = near_one(c.Kb.shape)
+    pv = c.pool_ref.reshape(c.n_blocks, 2, c.params.bt, -1)
+    pv[:, 0] = near_one(pv[:, 0].shape)
+    print(f"case far below zero HD={HD}", flush=True)
+    assert np.abs(f32(run_case(c), c.params.dtype) - brute(c)).max() <= 2e-3
+
+
 def test_tiled_kernel_head_dim_512_split_and_gate():
     """Split tiles merged by the combine kernel at head dim 512, with a head-wise gate in the epilogue."""
     import torch
