@@ -302,12 +302,28 @@ __global__ __launch_bounds__(HD >= 512 ? 128 * NC : 256, OCC) void attn_stream_k
   // A sub-block past the range's last page re-reads that page.
   const int last_js = (max(tile.k1, tile.k0 + 1) - 1) & ~15;
   const int lane_k = (c16 * HD + dw + 8 * q4), lane_v = (dw + c16) * kVtDim + 4 * q4;
+  // The block ids of a unit's sub-blocks, asked for together: behind one another each is a trip of its own in front of the
+  // workgroup's first key page. With the lane reduction that plain rows no longer make for k_last (below), one row over 1024 keys
+  // (32 query heads of 128 dims) takes 7.62 us a pass in place of 7.88, replayed as a graph, and 48 rows over 60 to 3000 keys 60.3
+  // in place of 60.8.
+  auto blocks_of = [&](int u, int (&blk)[SBU]) {
+    const int j0 = u << USH;
+    if (a.ring) {
+#pragma unroll
+      for (int sb = 0; sb < SBU; ++sb) blk[sb] = table + min(j0 + 16 * sb, last_js) / bt % a.ring;
+    } else {
+#pragma unroll
+      for (int sb = 0; sb < SBU; ++sb) blk[sb] = list_entry(a, table + min(j0 + 16 * sb, last_js) / bt);
+    }
+  };
   auto load_cached = [&](int u, Unit<HW, SBU>& U) {
     const int j0 = u << USH;
+    int blk[SBU];
+    blocks_of(u, blk);
 #pragma unroll
     for (int sb = 0; sb < SBU; ++sb) {
       const int js = min(j0 + 16 * sb, last_js);  // first key of the sub-block
-      const int b = block_of(a, table, js);
+      const int b = blk[sb];
       const int t0 = js % bt;
       const uint16_t* hb = a.pool + head_base(a, HD, b, kvh);
       const uint16_t* kp = hb + t0 * HD + lane_k;
@@ -567,7 +583,9 @@ __global__ __launch_bounds__(HD >= 512 ? 128 * NC : 256, OCC) void attn_stream_k
       // Last batch key any row of the tile sees: its last row, a root it sees whole
       // (anc_len), the end of its image (bidi).
       int kl = -1;
-      if constexpr (PAIR && NC > 1) {  // over all rows of the tile: every pair scans the same batch units
+      if (!a.desc) {
+        kl = rr0 + rows_live - 1;  // plain rows: the tile's last one sees furthest
+      } else if constexpr (PAIR && NC > 1) {  // over all rows of the tile: every pair scans the same batch units
         for (int m = lane; m < rows_live; m += 64) {
           const int4 dm = a.desc ? a.desc[tile.r0 + m] : make_int4(0, 0, 0, 0);
           kl = max(kl, max(rr0 + m, max(dm.z - 1, a.bidi ? dm.w - 1 : -1)));
@@ -577,8 +595,10 @@ __global__ __launch_bounds__(HD >= 512 ? 128 * NC : 256, OCC) void attn_stream_k
         for (int c = 0; c < NCW; ++c)
           if (ok[c]) kl = max(kl, max(rr[c], max(dsc[c].z - 1, a.bidi ? dsc[c].w - 1 : -1)));
       }
+      if (a.desc) {
 #pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) kl = max(kl, __shfl_xor(kl, o));
+        for (int o = 32; o >= 1; o >>= 1) kl = max(kl, __shfl_xor(kl, o));
+      }
       // fused: the batch keys are the tile's own rows in LDS, never more than the tile holds
       k_last = __builtin_amdgcn_readfirstlane(min(kl, (FUSED ? min(tree.M, rows_live) : tree.M) - 1));
       if (tile.last >= 2) k_last = min(k_last, tile.last - 2);  // a part whose batch range ends at row last - 2 of the tree

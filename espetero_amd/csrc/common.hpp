@@ -159,10 +159,13 @@ __host__ __device__ __forceinline__ size_t vt_elem(int bt, int HD, int t, int d)
 // The block list is read through the constant address space: no kernel writes it, and a kernel that
 // stores to the pool (the fused prologue's append) would otherwise have to assume its stores reach the
 // list and fetch every entry with a vector load whose wait drains the key and value loads in flight.
-__device__ __forceinline__ int block_of(const KArgs& a, int table, int j) {
+__device__ __forceinline__ int list_entry(const KArgs& a, int i) {
   using const_i32 = const int32_t __attribute__((address_space(4)));
+  return ((const_i32*)a.blocks)[i];
+}
+__device__ __forceinline__ int block_of(const KArgs& a, int table, int j) {
   const int bi = j / a.bt;
-  return a.ring ? table + bi % a.ring : ((const_i32*)a.blocks)[table + bi];
+  return a.ring ? table + bi % a.ring : list_entry(a, table + bi);
 }
 
 // The tiled kernels' last step for one lane: dims d0 + 32 nt + 8 i + 4 hb + j of one (row, query head) at acc[nt][4 i + j], times
