@@ -50,6 +50,29 @@ def test_gate_matches_checker(H, HD, D, n_rows, dtype):
         assert np.abs(ob.to_f32(_bits(O), dtype) - ob.to_f32(want, dtype)).max() <= 2e-3
 
 
+@pytest.mark.parametrize("H,D,n_rows", [(1, 8, 1), (16, 64, 16), (17, 72, 17), (16, 520, 33), (32, 576, 5), (33, 1032, 31), (48, 1600, 16),
+                                        (49, 2056, 3), (64, 4104, 18)])
+@pytest.mark.parametrize("skew", [0, 1])
+def test_gate_dots_alone(H, D, n_rows, skew):
+    """The dots-only call where its split of the model dims can go wrong: fewer pieces of 64 dims than wavefronts, one more than
+    they share evenly, a partial last piece, partial row and head blocks; skew 1: rows that start two bytes off a 16-byte
+    boundary. Infinities beside the rows are not read. The bound is test_gate_matches_checker's."""
+    device.init(0)
+    print(f"gate dots H={H} D={D} rows={n_rows} skew={skew}", flush=True)
+    p, a = synth.make_gate(H, 64, D, abi.ESP_F16, n_rows, seed=H + D)
+    _, want = ob.head_gate(p, a["O"], a["X"], a["Wg"], n_rows, want_dots=True)
+    ld = D + 16
+    X = torch.full((n_rows * ld + 8,), 0x7C00, dtype=torch.int16, device="cuda")
+    X[skew:skew + n_rows * ld].view(n_rows, ld)[:, :D] = _dev(a["X"].view(np.int16))[:, :D]
+    dots = torch.full((n_rows + 1, H), 7.0, dtype=torch.float32, device="cuda")
+    p.x_ld = ld
+    device.head_gate(p, None, X[skew:], _dev(a["Wg"].view(np.int16)), dots, n_rows)
+    torch.cuda.synchronize()
+    got = dots.cpu().numpy()
+    assert np.abs(got[:n_rows] - want).max() <= 2e-5 * np.sqrt(D)
+    assert (got[n_rows] == 7.0).all()
+
+
 def test_gate_strides_padding_and_modes():
     """Row strides wider than the data; columns past H * head_dim stay as they were; O alone, dots alone."""
     device.init(0)
