@@ -42,6 +42,36 @@
 
 namespace esp {
 
+// A wavefront's 32 output rows of RB bytes on their way through LDS: written by row (lane % 32), stored 1 KB of consecutive rows at a
+// time. The 16-byte parts of a row are turned by its number, which spreads both sides over the banks.
+template <int RB>
+struct RowsOut {
+  static constexpr int P = RB / 16, RPI = 64 / P;  // parts of a row; rows one store instruction takes
+  static __device__ __forceinline__ char* at(char* ob, int r, int p) { return ob + r * RB + (p ^ (r & (P < 16 ? P - 1 : 15))) * 16; }
+  // dst: where this lane's row (lane % 32) goes, 0 where there is none
+  static __device__ __forceinline__ void store(char* ob, uint64_t dst, int lane) {
+    using out16 = uint32_t __attribute__((ext_vector_type(4), aligned(8)));  // a row of O starts at any multiple of 8 bytes
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");  // the rows are written: one wavefront's LDS accesses keep their order
+    const int lo = int(uint32_t(dst)), hi = int(uint32_t(dst >> 32));
+    constexpr int N = 32 / RPI, B = N < 8 ? N : 8;
+#pragma unroll
+    for (int j0 = 0; j0 < N; j0 += B) {
+      u32x4 v[B];
+      uint64_t d[B];
+#pragma unroll
+      for (int j = 0; j < B; ++j) {
+        const int r = (j0 + j) * RPI + lane / P;
+        v[j] = *reinterpret_cast<const u32x4*>(at(ob, r, lane % P));
+        d[j] = uint64_t(uint32_t(__shfl(lo, r))) | uint64_t(uint32_t(__shfl(hi, r))) << 32;
+      }
+#pragma unroll
+      for (int j = 0; j < B; ++j)
+        if (d[j]) *(__attribute__((address_space(1))) out16*)(d[j] + uint64_t(lane % P) * 16) = v[j];
+    }
+  }
+};
+
 template <int DT, int HD, int OCC>
 __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int n_tiles) {
   constexpr int KS = HD / 16, NT = HD / 32;
@@ -810,7 +840,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   // Where the loops' instructions lie in the 32 bytes of a fetch is worth 3 % where workgroups run one to a compute unit (512 rows
   // behind 2048 keys beside 12 decoding sequences: 65.0 us here and 8 bytes ahead, 66.2 8 bytes on, 67.2 16 bytes on; a 2048-row chunk
   // at 6144 313 and 315.7): pinned, so that code in front of them does not shift it.
-  asm volatile(".p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
+  asm volatile(".p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
   int i = 0;
 #pragma nounroll
   for (int seg = 0; seg < 3; ++seg) {
@@ -840,27 +870,44 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
     if (i + 2 < n_steps) fill(i + 2, i & 1, general);
   }
 
-  // ---- output: lane (row l32, half hb) holds dims 32 nt + 8 i + 4 hb + j at acc[nt][4 i + j]
+  // ---- output: lane (row l32, half hb) holds dims 32 nt + 8 i + 4 hb + j at acc[nt][4 i + j]. The wavefront's 32 rows go
+  // through its quarter of the stages, which all four have read, so that neighbouring lanes store one row's bytes: a store whose
+  // neighbouring lanes are different rows takes the memory path a clock per lane, 1.7 us of a workgroup at D = 128. Six prompts of 40 to
+  // 900 rows, prep to attention, 65.1 us -> 62.7; 8 x 1024 rows at 15360, 256 dims, 3913 -> 3885.
   const float l = l_run + __shfl_xor(l_run, 32);
-  if (!row_ok) return;
   const int h_in_group = packed ? m_row % a.G : hg;
+  // The lane's number anew: addresses made from it before the loop would be carried through it, in registers it has not got.
+  int ln;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+  const int r32 = ln & 31, half = ln >> 5;
+  char* ob = lds + wave * KBUF;
+  // A packed tile's part: one wavefront's rows, few of them, and nothing beside it to hide a trip through LDS.
+  const bool direct = packed && tile.part >= 0;
+  if (!direct) __syncthreads();
   if (tile.part >= 0) {
     const size_t rec = (size_t(tile.part) * a.Hkv + kvh) * a.cols + size_t(rr - rr0) * a.G + h_in_group;
     float* po = a.parts_o + rec * HD;
+    if (row_ok) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4)
-        *reinterpret_cast<f32x4*>(po + 32 * nt + 8 * i4 + 4 * hb) =
-            f32x4{acc[nt][4 * i4], acc[nt][4 * i4 + 1], acc[nt][4 * i4 + 2], acc[nt][4 * i4 + 3]};
-    if (hb == 0) {
-      a.parts_ml[rec * 2] = m_run;
-      a.parts_ml[rec * 2 + 1] = l;
+      for (int i = 0; i < NT * 4; ++i) {
+        const f32x4 v = {acc[i / 4][4 * (i % 4)], acc[i / 4][4 * (i % 4) + 1], acc[i / 4][4 * (i % 4) + 2], acc[i / 4][4 * (i % 4) + 3]};
+        if (direct) *reinterpret_cast<f32x4*>(po + 8 * i + 4 * half) = v;
+        else *reinterpret_cast<f32x4*>(RowsOut<4 * HD>::at(ob, r32, 2 * i + half)) = v;
+      }
+      if (half == 0) {
+        a.parts_ml[rec * 2] = m_run;
+        a.parts_ml[rec * 2 + 1] = l;
+      }
     }
+    if (!direct) RowsOut<4 * HD>::store(ob, row_ok ? reinterpret_cast<uint64_t>(po) : 0, ln);
     return;
   }
   const int h = kvh * a.G + h_in_group;
-  store_output<DT>(a, acc, l > 0.0f ? 1.0f / l : 0.0f, row, h, size_t(h) * HD, 0, hb);
+  if (row_ok)
+    finish_output<DT>(a, acc, l > 0.0f ? 1.0f / l : 0.0f, row, h, 0, half, [&](int i, u32x2 v) __attribute__((always_inline)) {
+      *reinterpret_cast<u32x2*>(RowsOut<2 * HD>::at(ob, r32, i) + 8 * half) = v;
+    });
+  RowsOut<2 * HD>::store(ob, row_ok ? reinterpret_cast<uint64_t>(a.O + size_t(row) * a.q_ld + size_t(h) * HD) : 0, ln);
 }
 
 // Workgroups per compute unit and the largest tile each variant takes.

@@ -531,7 +531,8 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
     }
     return;
   }
-  store_output<DT>(a, acc, l > 0.0f ? 1.0f / l : 0.0f, row, h, size_t(h) * kHD, dw, hb);
+  uint16_t* op = a.O + size_t(row) * a.q_ld + size_t(h) * kHD + dw + 4 * hb;
+  finish_output<DT>(a, acc, l > 0.0f ? 1.0f / l : 0.0f, row, h, dw, hb, [&](int i, u32x2 v) { *reinterpret_cast<u32x2*>(op + 8 * i) = v; });
 }
 
 // The dynamic LDS limit of both variants on the current device, ahead of the first launch.

@@ -174,9 +174,9 @@ __device__ __forceinline__ int block_of(const KArgs& a, int table, int j) {
 // as far as the compiler knows, and one load group in front of each store made the end of a workgroup a chain of 16 (head dim
 // 128) or 32 (256) memory round trips. Ten prompts of 512 rows, 32 heads of 128, head-wise gate: each of the 512 slots stood
 // idle 17 us between two workgroups (4 without a gate); six prompts of 77 .. 817 rows, prep to attention, 93 us -> 71.
-template <int DT, int NT>
-__device__ __forceinline__ void store_output(const KArgs& a, const f32x16 (&acc)[NT], float inv, int row, int h, size_t head_off, int d0, int hb) {
-  uint16_t* op = a.O + size_t(row) * a.q_ld + head_off + d0 + 4 * hb;
+// put(i, v) takes dims d0 + 8 i + 4 hb .. + 3 in the storage type.
+template <int DT, int NT, typename Put>
+__device__ __forceinline__ void finish_output(const KArgs& a, const f32x16 (&acc)[NT], float inv, int row, int h, int d0, int hb, Put put) {
   const float* gp = a.gate ? a.gate + size_t(row) * a.gate_ld + size_t(h) * a.gate_hs + a.gate_off : nullptr;
   if (gp && a.gate_ds) {
     using f32x4_any = float __attribute__((ext_vector_type(4), aligned(4)));  // the gate's strides are the caller's
@@ -188,7 +188,7 @@ __device__ __forceinline__ void store_output(const KArgs& a, const f32x16 (&acc)
       f32x4 o;
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[j] = acc[i / 4][4 * (i % 4) + j] * inv / (1.0f + __expf(-g[i][j]));
-      *reinterpret_cast<u32x2*>(op + 8 * i) = u32x2{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])};
+      put(i, u32x2{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])});
     }
     return;
   }
@@ -198,7 +198,7 @@ __device__ __forceinline__ void store_output(const KArgs& a, const f32x16 (&acc)
     f32x4 o;
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[j] = acc[i / 4][4 * (i % 4) + j] * inv;
-    *reinterpret_cast<u32x2*>(op + 8 * i) = u32x2{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])};
+    put(i, u32x2{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])});
   }
 }
 

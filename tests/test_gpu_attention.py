@@ -347,6 +347,14 @@ def test_tiled_kernel_head_dim_512_few_steps(kw, dtype):
     _check(small_case(seed=49, HD=512, H=4, Hkv=2, rows_per_tile=64, dtype=dtype, **kw))
 
 
+@pytest.mark.parametrize("HD", [128, 256])
+@pytest.mark.parametrize("seqs", [((100, 1), (40, 31), (7, 33)), ((200, 127), (0, 128), (65, 97)), ((3000, 40),)])
+@pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
+def test_tiled_kernel_ragged_output_rows(HD, seqs, dtype):
+    """A wavefront's rows leave through LDS together: none, one, all but one and all of its 32."""
+    _check(small_case(seed=53, HD=HD, H=4, Hkv=2, seqs=seqs, rows_per_tile=128, dtype=dtype))
+
+
 @pytest.mark.parametrize("HD,rows", [(128, 128), (512, 64)])
 def test_tiled_kernel_scores_far_below_zero(HD, rows):
     """Every score is near -650 log2 units: nothing of it survives an exponential before the row has a reference. Equal queries of -20 against
