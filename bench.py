@@ -182,8 +182,6 @@ class GateWorkload:
     """esp_head_gate over the rows of one prefill pass: O *= sigmoid(x . Wg[h]) in place (the reference's
     form), or with dots_only the fp32 dots alone, which the attention's own epilogue then applies."""
 
-    kernel = "head_gate_kernel"
-
     def __init__(self, name, H, HD, D, dtype, n_rows, dots_only=False, seed=9):
         import torch
         from espetero_amd import abi, device, synth
@@ -191,7 +189,7 @@ class GateWorkload:
         self.name, self.bound, self.dtype = name, "hbm", dtype
         self.H, self.Hkv, self.HD, self.bt, self.window = H, H, HD, 0, 0
         self.seqs, self.n_rows, self.tiles, self.n_parts, self.pool_pages = [(0, n_rows)], n_rows, [], 0, 0
-        self.dots_only = dots_only
+        self.dots_only, self.kernel = dots_only, "gate_dots_kernel" if dots_only else "head_gate_kernel"
         p, a = synth.make_gate(H, HD, D, dtype, n_rows, seed=seed)
         self.params, self.host = p, a
         tdt = torch.float16 if dtype == abi.ESP_F16 else torch.bfloat16
