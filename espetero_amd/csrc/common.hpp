@@ -169,12 +169,11 @@ __device__ __forceinline__ int block_of(const KArgs& a, int table, int j) {
 }
 
 // The tiled kernels' last step for one lane: dims d0 + 32 nt + 8 i + 4 hb + j of one (row, query head) at acc[nt][4 i + j], times
-// inv, through the optional sigmoid gate, to O. `head_off`: the head's first element in a row of O.
+// inv, through the optional sigmoid gate: put(i, v) takes dims d0 + 8 i + 4 hb .. + 3 in the storage type.
 // Bound by the latency of the gate's loads, so all of them are out before the first store: a store may overlap any later load
 // as far as the compiler knows, and one load group in front of each store made the end of a workgroup a chain of 16 (head dim
 // 128) or 32 (256) memory round trips. Ten prompts of 512 rows, 32 heads of 128, head-wise gate: each of the 512 slots stood
 // idle 17 us between two workgroups (4 without a gate); six prompts of 77 .. 817 rows, prep to attention, 93 us -> 71.
-// put(i, v) takes dims d0 + 8 i + 4 hb .. + 3 in the storage type.
 template <int DT, int NT, typename Put>
 __device__ __forceinline__ void finish_output(const KArgs& a, const f32x16 (&acc)[NT], float inv, int row, int h, int d0, int hb, Put put) {
   const float* gp = a.gate ? a.gate + size_t(row) * a.gate_ld + size_t(h) * a.gate_hs + a.gate_off : nullptr;
