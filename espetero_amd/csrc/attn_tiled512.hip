@@ -257,16 +257,15 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[nt][i] = 0.0f;
-  // Per score row of this lane: the running reference in log2 units of the scaled score (-inf: no key seen yet), what is
-  // subtracted for it, and this lane's share of the row's sum. Without a reference kUnset is subtracted: the first visible score
-  // gives an infinite P and with it a sum that asks for one, and keys the row does not see give 0 as always. ps: the lane's share of the
-  // sum of the step whose P is in LDS, not yet in l_run.
-  constexpr float kUnset = -1e30f;
-  float m_run[2], m_sub[2], l_run[2], ps[2];
+  // Per score row of this lane: the running reference in log2 units of the scaled score and this lane's share of the row's sum. A
+  // row begins at kUnset, the lowest value of the type: the first visible score gives an infinite P and with it a sum that asks for
+  // a reference (a score of kUnset itself has it already), and keys the row does not see give 0 as always. ps: the lane's share of
+  // the sum of the step whose P is in LDS, not yet in l_run.
+  constexpr float kUnset = -__FLT_MAX__;
+  float m_run[2], l_run[2], ps[2];
 #pragma unroll
   for (int rt = 0; rt < 2; ++rt) {
-    m_run[rt] = -INFINITY;
-    m_sub[rt] = kUnset;
+    m_run[rt] = kUnset;
     l_run[rt] = ps[rt] = 0.0f;
   }
   f32x4 s[2];        // scores of the step: s[rt][e] is key 4 q4 + e of sub-block `half`, row 16 rt + c16
@@ -281,7 +280,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
     for (int rt = 0; rt < 2; ++rt) {
       float p[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) p[e] = fast_exp2(__builtin_fmaf(s[rt][e], a.scale_log2, -m_sub[rt]));
+      for (int e = 0; e < 4; ++e) p[e] = fast_exp2(__builtin_fmaf(s[rt][e], a.scale_log2, -m_run[rt]));
       const u32x2 w = {pack2<DT>(p[0], p[1]), pack2<DT>(p[2], p[3])};
       ps[rt] = sum2<DT>(w.y, sum2<DT>(w.x, 0.0f));
       *reinterpret_cast<u32x2*>(p_own + buf * kPBuf + 16 * rt * kPRow) = w;
@@ -307,9 +306,8 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
     for (int rt = 0; rt < 2; ++rt) {
       const float other = mx_sh[(half ^ 1) * 32 + 16 * rt + c16];
       const float m_new = fmaxf(m_run[rt], fmaxf(mx[rt], other) * a.scale_log2);  // scale > 0: the max commutes with it
-      corr[rt] = (m_run[rt] == -INFINITY) ? 1.0f : fast_exp2(m_run[rt] - m_new);  // nothing accumulated without a reference
+      corr[rt] = fast_exp2(m_run[rt] - m_new);
       m_run[rt] = m_new;
-      m_sub[rt] = (m_new == -INFINITY) ? kUnset : m_new;
       l_run[rt] *= corr[rt];
     }
     const float c = (lane & 16) ? corr[1] : corr[0];  // of row l32
@@ -526,7 +524,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
         *reinterpret_cast<f32x4*>(po + 32 * nt + 8 * i4 + 4 * hb) =
             f32x4{acc[nt][4 * i4], acc[nt][4 * i4 + 1], acc[nt][4 * i4 + 2], acc[nt][4 * i4 + 3]};
     if (hb == 0 && dw == 0) {
-      a.parts_ml[rec * 2] = m_mine;
+      a.parts_ml[rec * 2] = m_mine == kUnset && !(l > 0.0f) ? -INFINITY : m_mine;  // no key seen: the merge passes the part over
       a.parts_ml[rec * 2 + 1] = l;
     }
     return;

@@ -371,6 +371,27 @@ def test_tiled_kernel_scores_far_below_zero(HD, rows):
     assert np.abs(f32(run_case(c), c.params.dtype) - brute(c)).max() <= 2e-3
 
 
+@pytest.mark.parametrize("HD,rows", [(128, 128), (512, 64)])
+@pytest.mark.parametrize("log2", [102, 116])
+@pytest.mark.parametrize("low", [1.0, 0.5])
+@pytest.mark.parametrize("split", [False, True])
+def test_tiled_kernel_scores_near_the_lowest_float(HD, rows, log2, low, split):
+    """Scaled scores of -1e32 to -1e36 are scores like any others, in whole tiles and in parts of them: powers of two, so that every
+    score is exact. low 1: all of a row's are equal and it takes the mean of its values; low 0.5: key 37's is half as far from zero and
+    the row takes that key's values."""
+    from gpu_utils import default_options, run_case
+    c = small_case(seed=54, HD=HD, H=4, Hkv=2, seqs=((1000 if split else 100, 70),), rows_per_tile=rows, scale=HD ** -0.5, dtype=abi.ESP_BF16)
+    at = lambda x, shape: synth._bits(np.full(shape, x, np.float32), c.params.dtype)  # noqa: E731
+    c.Q[:] = at(-2.0 ** 50 * 512 / HD, c.Q.shape)
+    c.Kb[:] = at(2.0 ** (log2 - 50), c.Kb.shape)
+    pool = c.pool_ref.reshape(c.n_blocks, 2, c.params.bt, -1)
+    pool[:, 0] = at(2.0 ** (log2 - 50), pool[:, 0].shape)
+    pool[c.blocks[37 // c.params.bt], 0, 37 % c.params.bt] = at(low * 2.0 ** (log2 - 50), pool.shape[3])
+    print(f"case near the lowest float HD={HD} log2={log2} low={low} split={split}", flush=True)
+    got = run_case(c, default_options(c, 256) if split else None)
+    assert max_abs(got, brute(c), c.params.dtype) <= tol_for(c.params.dtype)
+
+
 def test_tiled_kernel_head_dim_512_split_and_gate():
     """Split tiles merged by the combine kernel at head dim 512, with a head-wise gate in the epilogue."""
     import torch
