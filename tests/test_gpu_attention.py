@@ -379,8 +379,8 @@ def test_tiled_kernel_scores_near_the_lowest_float(HD, rows, log2, low, split):
     """Scaled scores of -1e32 to -1e36 are scores like any others, in whole tiles and in parts of them: powers of two, so that every
     score is exact. low 1: all of a row's are equal and it takes the mean of its values; low 0.5: key 37's is half as far from zero and
     the row takes that key's values."""
-    from gpu_utils import default_options, run_case
-    c = small_case(seed=54, HD=HD, H=4, Hkv=2, seqs=((1000 if split else 100, 70),), rows_per_tile=rows, scale=HD ** -0.5, dtype=abi.ESP_BF16)
+    from gpu_utils import run_case
+    c = small_case(seed=54, HD=HD, H=4, Hkv=2, seqs=((3000 if split else 100, 70),), rows_per_tile=rows, scale=HD ** -0.5, dtype=abi.ESP_BF16)
     at = lambda x, shape: synth._bits(np.full(shape, x, np.float32), c.params.dtype)  # noqa: E731
     c.Q[:] = at(-2.0 ** 50 * 512 / HD, c.Q.shape)
     c.Kb[:] = at(2.0 ** (log2 - 50), c.Kb.shape)
@@ -388,7 +388,7 @@ def test_tiled_kernel_scores_near_the_lowest_float(HD, rows, log2, low, split):
     pool[:, 0] = at(2.0 ** (log2 - 50), pool[:, 0].shape)
     pool[c.blocks[37 // c.params.bt], 0, 37 % c.params.bt] = at(low * 2.0 ** (log2 - 50), pool.shape[3])
     print(f"case near the lowest float HD={HD} log2={log2} low={low} split={split}", flush=True)
-    got = run_case(c, default_options(c, 256) if split else None)
+    got = run_case(c, host.options_mi355x(rows, 64 if split else 1))
     assert max_abs(got, brute(c), c.params.dtype) <= tol_for(c.params.dtype)
 
 
