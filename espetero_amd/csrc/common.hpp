@@ -191,12 +191,14 @@ __device__ __forceinline__ void finish_output(const KArgs& a, const f32x16 (&acc
     }
     return;
   }
-  if (gp) inv /= 1.0f + __expf(-gp[0]);  // one gate value for the head
+  // One gate value for the head, a factor of its own: inv times it can lie so far below the normal floats that the product with
+  // acc, itself a number the storage type holds, would keep few of its bits.
+  const float gf = gp ? 1.0f / (1.0f + __expf(-gp[0])) : 1.0f;
 #pragma unroll
   for (int i = 0; i < NT * 4; ++i) {
     f32x4 o;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = acc[i / 4][4 * (i % 4) + j] * inv;
+    for (int j = 0; j < 4; ++j) o[j] = acc[i / 4][4 * (i % 4) + j] * inv * gf;
     put(i, u32x2{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])});
   }
 }

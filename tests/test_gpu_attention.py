@@ -315,6 +315,31 @@ def test_tiled_kernels_gate_of_odd_strides(HD, headwise):
     assert np.abs(got - want).max() <= 2e-3 and (got[::7] == 0).all()
 
 
+@pytest.mark.parametrize("HD,rows", [(128, 128), (256, 128), (512, 64)])
+def test_tiled_kernels_nearly_closed_gate(HD, rows):
+    """A head-wise gate of -84 to -87.3 over the mean of 30000 values between 1 and 2 leaves bf16 outputs of 1.5e-38 and more, normal numbers:
+    each is the nearest (half a unit in the last place, 2^-8 of a power of two with 7 bits behind it) but for fp32 rounding of the sum and of the exponential, whose
+    argument's half unit at 87 is 4e-6: 1e-4 stands for both."""
+    import torch
+    from gpu_utils import run_case
+    c = small_case(seed=55, HD=HD, H=2, Hkv=1, seqs=((30000, 20),), rows_per_tile=rows, dtype=abi.ESP_BF16)
+    p = c.params
+    rng = np.random.default_rng(56)
+    value = lambda shape: synth._bits(rng.uniform(1.0, 2.0, shape).astype(np.float32), p.dtype)  # noqa: E731
+    c.Q[:] = 0
+    c.Vb[:] = value(c.Vb.shape)
+    pool = c.pool_ref.reshape(c.n_blocks, 2, p.bt, -1)
+    pool[:, 1] = value(pool[:, 1].shape)
+    g = np.linspace(-87.3, -84.0, c.n_rows * p.H, dtype=np.float32).reshape(c.n_rows, p.H)
+    gd = torch.from_numpy(g).cuda()
+    p.gate, p.gate_ld, p.gate_hs, p.gate_off, p.gate_headwise = gd.data_ptr(), p.H, 1, 0, 1
+    print(f"case nearly closed gate HD={HD}", flush=True)
+    got = f32(run_case(c, host.options_mi355x(rows, 1)), p.dtype).astype(np.float64)
+    p.gate, p.gate_headwise = None, 0
+    want = brute(c) / (1.0 + np.exp(-np.repeat(g.astype(np.float64), HD, axis=1)))
+    assert np.abs(got / want - 1.0).max() <= 2.0 ** -8 + 1e-4
+
+
 # ---- head dim 512 prefill: 64-row tiles, wavefront pairs split the dims
 @pytest.mark.parametrize("kw", [
     dict(seqs=((0, 200),), H=4, Hkv=2),                                 # first chunk: batch keys only
