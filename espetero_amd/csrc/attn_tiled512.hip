@@ -438,7 +438,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
     } else {
       exp_pack(S);
     }
-    const int mine = __any(!(ps[0] <= 256.0f) || !(ps[1] <= 256.0f));
+    const int mine = __any(ps[0] > 256.0f || ps[1] > 256.0f);
     if (lane == 0) flags[S][wave] = mine;
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // own loads landed, own reads of this iteration's stages done
     if constexpr (!PLAIN) fix(i, S);
