@@ -84,7 +84,18 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
   const int rows_live = min(a.R, end - tile.r0);
   const int rr0 = tile.r0 - tree.base;
 
-  // ---- this lane's two rows of the scores and their Q fragments
+  // ---- Q rows of the tile: a whole row to a load, then through the V^T stages, row r's chunk c at position c ^ (r % 16) as in K.
+  // Loads of the fragments themselves, whose neighbouring lanes are different rows, take the memory path a clock per lane, and every
+  // wavefront needs all dims of its 32 rows: 8192 clocks in front of a tile of 64. One pass of 64 fresh rows (16 / 2 heads) took
+  // 16.7 us so and takes 14.7 through LDS, 32 rows 10.9 and 10.3, 64 rows behind 1000 keys 50.4 and 48.0.
+  u32x4 qrow[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int r = 4 * i + wave;
+    if (r < rows_live) qrow[i] = *reinterpret_cast<const u32x4*>(a.Q + size_t(tile.r0 + r) * a.q_ld + size_t(h) * kHD + 8 * lane);
+  }
+
+  // ---- this lane's two rows of the scores
   int rr[2], qpos[2];
   int4 d[2];
   u32x4 qf[2][KK];
@@ -97,9 +108,6 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
     rr[rt] = rr0 + m;
     d[rt] = a.desc ? a.desc[row] : make_int4(0, 0, 0, 0);
     qpos[rt] = a.window > 0 ? a.pos[row].x : 0;
-    const uint16_t* qp = a.Q + size_t(row) * a.q_ld + size_t(h) * kHD + 8 * q4;
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) qf[rt][kk] = ok ? *reinterpret_cast<const u32x4*>(qp + 32 * kk) : u32x4{0, 0, 0, 0};
     if (ok) kl = max(kl, max(rr[rt], max(d[rt].z - 1, a.bidi ? d[rt].w - 1 : -1)));
   }
 
@@ -109,7 +117,19 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
 #pragma unroll
     for (int o = 8; o >= 1; o >>= 1) kl = max(kl, __shfl_xor(kl, o));  // the lanes of a quarter hold all rows
     if (lane == 0) flags[0][wave] = kl;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = 4 * i + wave;
+      if (r < rows_live) *reinterpret_cast<u32x4*>(lds + kVBase + r * 1024 + ((lane ^ (r & 15)) << 4)) = qrow[i];
+    }
     __syncthreads();
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      const int m = 32 * rg + 16 * rt + c16;
+      const char* qr = lds + kVBase + m * 1024;
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) qf[rt][kk] = m < rows_live ? *reinterpret_cast<const u32x4*>(qr + (((4 * kk + q4) ^ c16) << 4)) : u32x4{0, 0, 0, 0};
+    }
     k_last = max(flags[0][0], flags[0][2]);
     k_last = __builtin_amdgcn_readfirstlane(min(min(k_last, tree.M - 1), tile.last >= 2 ? tile.last - 2 : INT32_MAX));  // last >= 2: the part's batch range ends at row last - 2
   }
@@ -470,8 +490,8 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
 #pragma unroll
     for (int t = 0; t < 2; ++t) fill_k(t, 0, 0);
     wait_loads();
-    fill_v(0, 0);
     __syncthreads();
+    fill_v(0, 0);
 #pragma unroll
     for (int j = 0; j < 4; ++j) ring[0][j] = *lds_ptr(kaddr[j]);
     // Plain iterations lie below p1: steps up to i + 1 are sub-blocks wholly inside the cached range.

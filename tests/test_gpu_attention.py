@@ -365,6 +365,7 @@ def test_tiled_kernel_head_dim_512(kw):
     dict(seqs=((64, 64), (96, 33), (130, 64))),                         # even and odd counts of steps, whole and partial ones
     dict(seqs=((400, 64), (333, 40)), window=40),                       # rows that see nothing of their tile's first steps
     dict(seqs=((0, 150),), window=17),
+    dict(seqs=((0, 16), (7, 17), (20, 31), (3, 32), (40, 63))),         # tiles of a few rows: the Q rows in LDS past the last are none of theirs
 ])
 @pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
 def test_tiled_kernel_head_dim_512_few_steps(kw, dtype):
