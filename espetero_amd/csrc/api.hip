@@ -25,6 +25,7 @@ hipError_t launch_chain_advance(esp_tree* trees, int n_trees, int32_t* pos, int3
 hipError_t launch_vt_stage(const esp_attn_params* p, const void* Vb, void* vt, int n_rows, hipStream_t st);
 hipError_t launch_attn_prep(const PrepArgs& a, int n_rows, hipStream_t st);
 hipError_t launch_head_gate(int dt, const GateArgs& a, hipStream_t st);
+hipError_t gate_init_attributes();
 int tiled_max_rows(int HD);
 hipError_t stream_init_attributes();
 hipError_t tiled_init_attributes();
@@ -139,6 +140,7 @@ int device_state(DeviceState** out, char* err, size_t errlen) {
     if ((e = esp::stream_init_attributes()) != hipSuccess) return hip_fail(err, errlen, "hipFuncSetAttribute (streaming kernels)", e);
     if ((e = esp::tiled_init_attributes()) != hipSuccess) return hip_fail(err, errlen, "hipFuncSetAttribute (tiled kernels)", e);
     if ((e = esp::tiled512_init_attributes()) != hipSuccess) return hip_fail(err, errlen, "hipFuncSetAttribute (tiled kernels, head dim 512)", e);
+    if ((e = esp::gate_init_attributes()) != hipSuccess) return hip_fail(err, errlen, "hipFuncSetAttribute (head gate)", e);
     d.scratch = static_cast<unsigned char*>(ps);
     d.ready = true;
   }
@@ -549,6 +551,10 @@ int esp_head_gate(const esp_gate_params* p, void* O, const void* X, const void* 
     if (p->head_dim == 1 << s) shift = s;
   esp::GateArgs a{static_cast<uint16_t*>(O), static_cast<const uint16_t*>(X), static_cast<const uint16_t*>(Wg), dots,
                   n_rows, p->H, p->head_dim, shift, p->D, p->q_ld, p->x_ld};
+  if (!O) {  // the dots kernel has an LDS limit to raise; in place nothing needs the set-up
+    DeviceState* d = nullptr;
+    if (int rc = device_state(&d, err, errlen)) return rc;
+  }
   const hipError_t e = esp::launch_head_gate(p->dtype, a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(err, errlen, "head_gate launch", e);
   return ESP_OK;

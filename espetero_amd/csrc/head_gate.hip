@@ -251,6 +251,18 @@ hipError_t launch_gate(const GateArgs& a, dim3 grid, hipStream_t st) {
   return hipGetLastError();
 }
 
+// The dots kernels' dynamic LDS limits on the current device, ahead of their first launch.
+template <int DT, int... NBs>
+hipError_t gate_attributes_t() {
+  hipError_t e = hipSuccess;
+  ((e = e == hipSuccess ? allow_dynamic_lds<gate_dots_kernel<DT, NBs>>(GateDots<DT, NBs>::kLds) : e), ...);
+  return e;
+}
+hipError_t gate_init_attributes() {
+  const hipError_t e = gate_attributes_t<ESP_F16, 1, 2, 3, 4>();
+  return e != hipSuccess ? e : gate_attributes_t<ESP_BF16, 1, 2, 3, 4>();
+}
+
 hipError_t launch_head_gate(int dt, const GateArgs& a, hipStream_t st) {
   const dim3 grid((a.n_rows + kGateRows - 1) / kGateRows);
   const int nb = (a.H + 15) / 16;
