@@ -53,16 +53,17 @@ def test_gate_matches_checker(H, HD, D, n_rows, dtype):
 @pytest.mark.parametrize("H,D,n_rows", [(1, 8, 1), (16, 64, 16), (17, 72, 17), (16, 520, 33), (32, 576, 5), (33, 1032, 31), (48, 1600, 16),
                                         (49, 2056, 3), (64, 4104, 18)])
 @pytest.mark.parametrize("skew", [0, 1])
-def test_gate_dots_alone(H, D, n_rows, skew):
+@pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
+def test_gate_dots_alone(H, D, n_rows, skew, dtype):
     """The dots-only call where its split of the model dims can go wrong: fewer pieces of 64 dims than wavefronts, one more than
     they share evenly, a partial last piece, partial row and head blocks; skew 1: rows that start two bytes off a 16-byte
     boundary. Infinities beside the rows are not read. The bound is test_gate_matches_checker's."""
     device.init(0)
-    print(f"gate dots H={H} D={D} rows={n_rows} skew={skew}", flush=True)
-    p, a = synth.make_gate(H, 64, D, abi.ESP_F16, n_rows, seed=H + D)
+    print(f"gate dots H={H} D={D} rows={n_rows} skew={skew} dtype={dtype}", flush=True)
+    p, a = synth.make_gate(H, 64, D, dtype, n_rows, seed=H + D)
     _, want = ob.head_gate(p, a["O"], a["X"], a["Wg"], n_rows, want_dots=True)
     ld = D + 16
-    X = torch.full((n_rows * ld + 8,), 0x7C00, dtype=torch.int16, device="cuda")
+    X = torch.full((n_rows * ld + 8,), 0x7C00 if dtype == abi.ESP_F16 else 0x7F80, dtype=torch.int16, device="cuda")
     X[skew:skew + n_rows * ld].view(n_rows, ld)[:, :D] = _dev(a["X"].view(np.int16))[:, :D]
     dots = torch.full((n_rows + 1, H), 7.0, dtype=torch.float32, device="cuda")
     p.x_ld = ld
@@ -71,6 +72,29 @@ def test_gate_dots_alone(H, D, n_rows, skew):
     got = dots.cpu().numpy()
     assert np.abs(got[:n_rows] - want).max() <= 2e-5 * np.sqrt(D)
     assert (got[n_rows] == 7.0).all()
+
+
+@pytest.mark.parametrize("H,D", [(5, 8), (20, 200), (40, 584), (64, 1160)])
+@pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
+def test_gate_dots_alone_with_infinities(H, D, dtype):
+    """One row and one head whose first value is an infinity: parts past a row's last dim are filled from there, and both operands are
+    cleared of it, since an infinity times the other's zero is not zero. Their dots are infinities of the right sign, every other dot
+    is what it was."""
+    device.init(0)
+    print(f"gate dots with infinities H={H} D={D} dtype={dtype}", flush=True)
+    n_rows, inf = 21, 0x7C00 if dtype == abi.ESP_F16 else 0x7F80
+    p, a = synth.make_gate(H, 64, D, dtype, n_rows, seed=H + D)
+    _, want = ob.head_gate(p, a["O"], a["X"], a["Wg"], n_rows, want_dots=True)
+    r, h = n_rows // 2, H // 2
+    want[:, h] = np.copysign(np.inf, ob.to_f32(a["X"][:, 0], dtype))
+    want[r] = np.copysign(np.inf, ob.to_f32(a["Wg"][:, 0], dtype))
+    want[r, h] = np.inf
+    a["X"][r, 0], a["Wg"][h, 0] = inf, inf
+    dots = torch.full((n_rows, H), 7.0, dtype=torch.float32, device="cuda")
+    device.head_gate(p, None, _dev(a["X"].view(np.int16)), _dev(a["Wg"].view(np.int16)), dots, n_rows)
+    torch.cuda.synchronize()
+    got, fin = dots.cpu().numpy(), np.isfinite(want)
+    assert np.array_equal(got[~fin], want[~fin]) and np.abs(got[fin] - want[fin]).max() <= 2e-5 * np.sqrt(D)
 
 
 def test_gate_strides_padding_and_modes():

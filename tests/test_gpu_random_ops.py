@@ -93,9 +93,12 @@ def test_random_gate_calls():
         O = _dev(a["O"].view(np.int16))
         dots = torch.zeros((n_rows, H), dtype=torch.float32, device="cuda")
         device.head_gate(p, O, _dev(a["X"].view(np.int16)), _dev(a["Wg"].view(np.int16)), dots, n_rows)
+        alone = torch.zeros_like(dots)
+        device.head_gate(p, None, _dev(a["X"].view(np.int16)), _dev(a["Wg"].view(np.int16)), alone, n_rows)
         torch.cuda.synchronize()
         assert _ulps(O.cpu().numpy().view(np.uint16), want).max() <= 1, it
-        assert np.abs(dots.cpu().numpy() - want_dots).max() <= 2e-5 * np.sqrt(D) + 1e-5, it
+        for d in (dots, alone):
+            assert np.abs(d.cpu().numpy() - want_dots).max() <= 2e-5 * np.sqrt(D) + 1e-5, it
 
 
 def test_random_pool_maintenance():
