@@ -837,10 +837,6 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   const int in1 = a_hi > in0 ? in0 + ((a_hi - in0) & ~1) : in0;
   const int in2 = max(in1, min((b_lo + 1) & ~1, even_steps));
   const int in3 = bb_hi > in2 ? in2 + ((bb_hi - in2) & ~1) : in2;
-  // Where the loops' instructions lie in the 32 bytes of a fetch is worth 3 % where workgroups run one to a compute unit (512 rows
-  // behind 2048 keys beside 12 decoding sequences: 65.0 us here and 8 bytes ahead, 66.2 8 bytes on, 67.2 16 bytes on; a 2048-row chunk
-  // at 6144 313 and 315.7): pinned, so that code in front of them does not shift it.
-  asm volatile(".p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
   int i = 0;
 #pragma nounroll
   for (int seg = 0; seg < 3; ++seg) {
