@@ -877,8 +877,10 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
   const int r32 = ln & 31, half = ln >> 5;
   char* ob = lds + wave * KBUF;
-  // A packed tile's part: one wavefront's rows, few of them, and nothing beside it to hide a trip through LDS.
-  const bool direct = packed && tile.part >= 0;
+  // Parts of a tile that leaves a wavefront without rows go straight out: the stores of three do not fill the memory path, and the
+  // trip through LDS is longer than theirs. 64 rows behind 2000 keys, 32 query heads of 128 dims, 18.5 us so and 19.0 through LDS; 33 rows, 16
+  // heads of 256, 25.8 and 27.6; 200 rows, tiles of 128 and 72, 24 heads of 256, 36.1 and 37.1. All four: 128 rows behind 1000 keys 30.7 and 29.7.
+  const bool direct = tile.part >= 0 && (packed || rows_live <= 96);
   if (!direct) __syncthreads();
   if (tile.part >= 0) {
     const size_t rec = (size_t(tile.part) * a.Hkv + kvh) * a.cols + size_t(rr - rr0) * a.G + h_in_group;

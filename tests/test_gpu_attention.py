@@ -381,6 +381,18 @@ def test_tiled_kernel_ragged_output_rows(HD, seqs, dtype):
     _check(small_case(seed=53, HD=HD, H=4, Hkv=2, seqs=seqs, rows_per_tile=128, dtype=dtype))
 
 
+@pytest.mark.parametrize("HD", [128, 256])
+@pytest.mark.parametrize("M", [33, 95, 96, 97, 128])
+@pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
+def test_tiled_kernel_ragged_part_rows(HD, M, dtype):
+    """The parts of split tiles on both sides of the row count from which they leave through LDS. 2500 keys in parts of a few hundred."""
+    from gpu_utils import plan, run_case
+    c = small_case(seed=58, HD=HD, H=4, Hkv=2, seqs=((2500, M), (1700, 40)), rows_per_tile=128, dtype=dtype)
+    assert plan(c, host.options_mi355x(128, 64))[2] >= 4
+    print(f"case ragged part rows HD={HD} M={M} dtype={dtype}", flush=True)
+    assert max_abs(run_case(c, host.options_mi355x(128, 64)), brute(c), dtype) <= tol_for(dtype)
+
+
 @pytest.mark.parametrize("HD,rows", [(128, 128), (512, 64)])
 def test_tiled_kernel_scores_far_below_zero(HD, rows):
     """Every score is near -650 log2 units: nothing of it survives an exponential before the row has a reference. Equal queries of -20 against
