@@ -486,6 +486,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
   };
   constexpr std::false_type general{};
   constexpr std::true_type plain{};
+  float l = 0.0f;  // the row's sum
   if (n_steps > 0) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) fill_k(t, 0, 0);
@@ -504,8 +505,18 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
     // ---- what is left: P V of the last step
     const int S = (n_steps - 1) & 1;
     if (out_of_range) settle(S);
+    // The row's sum: over the lanes that share the row, then over both wavefronts of the group (settle has left the place).
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) l_run[rt] += ps[rt];
+    for (int rt = 0; rt < 2; ++rt) {
+      l_run[rt] += ps[rt];
+      l_run[rt] += __shfl_xor(l_run[rt], 16);
+      l_run[rt] += __shfl_xor(l_run[rt], 32);
+    }
+    float* l_sh = reinterpret_cast<float*>(lds + kMax) + rg * 64;
+    const float l_mine = (lane & 16) ? l_run[1] : l_run[0];
+    if (hb == 0) l_sh[half * 32 + l32] = l_mine;
+    __syncthreads();
+    l = half ? l_sh[l32] + l_mine : l_mine + l_sh[32 + l32];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const u32x4 p = *lds_ptr(paddr + uint32_t(S * kPBuf + 32 * t));
@@ -518,19 +529,8 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
     }
   }
 
-  // ---- output: lane (row l32, half hb) holds dims dw + 32 nt + 8 i + 4 hb + j at acc[nt][4 i + j]. Its row's sum: over the
-  // lanes that share the row, then over both wavefronts of the group.
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    l_run[rt] += __shfl_xor(l_run[rt], 16);
-    l_run[rt] += __shfl_xor(l_run[rt], 32);
-  }
-  float* l_sh = reinterpret_cast<float*>(lds + kMax) + rg * 64;
-  const float l_mine = (lane & 16) ? l_run[1] : l_run[0], m_mine = (lane & 16) ? m_run[1] : m_run[0];
-  __syncthreads();
-  if (hb == 0) l_sh[half * 32 + l32] = l_mine;
-  __syncthreads();
-  const float l = half ? l_sh[l32] + l_mine : l_mine + l_sh[32 + l32];
+  // ---- output: lane (row l32, half hb) holds dims dw + 32 nt + 8 i + 4 hb + j at acc[nt][4 i + j].
+  const float m_mine = (lane & 16) ? m_run[1] : m_run[0];
   const int m_row = 32 * rg + l32;
   const int row = tile.r0 + m_row;
   if (m_row >= rows_live) return;
