@@ -585,17 +585,17 @@ __global__ __launch_bounds__(HD >= 512 ? 128 * NC : 256, OCC) void attn_stream_k
       int kl = -1;
       if (!a.desc) {
         kl = rr0 + rows_live - 1;  // plain rows: the tile's last one sees furthest
-      } else if constexpr (PAIR && NC > 1) {  // over all rows of the tile: every pair scans the same batch units
-        for (int m = lane; m < rows_live; m += 64) {
-          const int4 dm = a.desc ? a.desc[tile.r0 + m] : make_int4(0, 0, 0, 0);
-          kl = max(kl, max(rr0 + m, max(dm.z - 1, a.bidi ? dm.w - 1 : -1)));
-        }
       } else {
+        if constexpr (PAIR && NC > 1) {  // over all rows of the tile: every pair scans the same batch units
+          for (int m = lane; m < rows_live; m += 64) {
+            const int4 dm = a.desc[tile.r0 + m];
+            kl = max(kl, max(rr0 + m, max(dm.z - 1, a.bidi ? dm.w - 1 : -1)));
+          }
+        } else {
 #pragma unroll
-        for (int c = 0; c < NCW; ++c)
-          if (ok[c]) kl = max(kl, max(rr[c], max(dsc[c].z - 1, a.bidi ? dsc[c].w - 1 : -1)));
-      }
-      if (a.desc) {
+          for (int c = 0; c < NCW; ++c)
+            if (ok[c]) kl = max(kl, max(rr[c], max(dsc[c].z - 1, a.bidi ? dsc[c].w - 1 : -1)));
+        }
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) kl = max(kl, __shfl_xor(kl, o));
       }
