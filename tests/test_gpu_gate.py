@@ -151,3 +151,22 @@ def test_attention_headwise_gate_is_attention_then_gate(kw):
                         ag["X"], ag["Wg"], c.n_rows)
     tol = 2e-3 if p.dtype == abi.ESP_F16 else 8e-3
     assert np.abs(f32(fused, p.dtype) - ob.to_f32(want, p.dtype)).max() <= tol
+
+
+@pytest.mark.parametrize("dots_only", [False, True])
+def test_bench_gate_record_checks_the_call_it_times(dots_only):
+    """The error that bench.py prints beside a gate workload's time is that of the same call: with the dots alone no O goes in."""
+    import bench
+    w = bench.GateWorkload("gate", 20, 64, 200, abi.ESP_F16, 40, dots_only=dots_only)
+    calls = []
+
+    class Recorder:
+        @staticmethod
+        def head_gate(p, O, *a):
+            calls.append(O is None)
+            device.head_gate(p, O, *a)
+
+    w.device = Recorder
+    w.step(0)
+    r = bench.gate_cpu_baseline(w)
+    assert calls == [dots_only, dots_only] and r["max_abs_err_vs_gpu"] <= 2e-3 and r["max_abs_dot_err_vs_gpu"] <= 2e-5 * np.sqrt(200)
