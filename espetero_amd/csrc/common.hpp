@@ -191,14 +191,30 @@ __device__ __forceinline__ void finish_output(const KArgs& a, const f32x16 (&acc
     }
     return;
   }
-  // One gate value for the head, a factor of its own: inv times it can lie so far below the normal floats that the product with
-  // acc, itself a number the storage type holds, would keep few of its bits.
-  const float gf = gp ? 1.0f / (1.0f + __expf(-gp[0])) : 1.0f;
+  if (gp) {  // one gate value for the head: in one factor with inv
+    const float gf = 1.0f / (1.0f + __expf(-gp[0])), both = inv * gf;
+    // Unless the product lies so far below the normal floats that its own with acc, a number the storage type holds, would keep few of
+    // its bits. A loop of its own for that, out of the way: two multiplications for every output are 0.15 us of a pass at 128 dims and 0.25 at
+    // 256 (4 fresh rows 8.05 us -> 8.21 and 9.95 -> 10.22, 222 rows at 256 18.1 -> 18.3). The other rows of the wavefront keep their bits.
+    const bool low = both < 1e-30f;
+    if (__builtin_expect(__any(low), 0)) {
+      const float f = low ? inv : both, g = low ? gf : 1.0f;
+#pragma unroll
+      for (int i = 0; i < NT * 4; ++i) {
+        f32x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = acc[i / 4][4 * (i % 4) + j] * f * g;
+        put(i, u32x2{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])});
+      }
+      return;
+    }
+    inv = both;
+  }
 #pragma unroll
   for (int i = 0; i < NT * 4; ++i) {
     f32x4 o;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = acc[i / 4][4 * (i % 4) + j] * inv * gf;
+    for (int j = 0; j < 4; ++j) o[j] = acc[i / 4][4 * (i % 4) + j] * inv;
     put(i, u32x2{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])});
   }
 }

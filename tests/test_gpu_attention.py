@@ -340,7 +340,28 @@ def test_tiled_kernels_nearly_closed_gate(HD, rows):
     assert np.abs(got / want - 1.0).max() <= 2.0 ** -8 + 1e-4
 
 
-# ---- head dim 512 prefill: 64-row tiles, wavefront pairs split the dims
+@pytest.mark.parametrize("HD,rows", [(128, 128), (256, 128), (512, 64)])
+def test_tiled_kernels_closed_gate_is_its_own_affair(HD, rows):
+    """Rows whose head-wise gate is shut take their factors apart, and the rows beside them in the wavefront keep their bits."""
+    import torch
+    from gpu_utils import run_case
+    c = small_case(seed=59, HD=HD, H=4, Hkv=2, seqs=((300, 70),), rows_per_tile=rows)
+    p = c.params
+    g = np.random.default_rng(60).standard_normal((c.n_rows, p.H)).astype(np.float32)
+    outs = []
+    for shut in (False, True):
+        if shut:
+            g[3::9] = -95.0
+        gd = torch.from_numpy(g).cuda()
+        p.gate, p.gate_ld, p.gate_hs, p.gate_off, p.gate_headwise = gd.data_ptr(), p.H, 1, 0, 1
+        print(f"case closed gate HD={HD} shut={shut}", flush=True)
+        outs.append(run_case(c, host.options_mi355x(rows, 1)))
+    keep = np.ones(c.n_rows, bool)
+    keep[3::9] = False
+    assert np.array_equal(outs[0][keep], outs[1][keep]) and (f32(outs[1][~keep], p.dtype) == 0).all()
+
+
+# ---- head dim 512 prefill: 64-row tiles, two wavefronts share a row group: its scores by keys, its output by dims
 @pytest.mark.parametrize("kw", [
     dict(seqs=((0, 200),), H=4, Hkv=2),                                 # first chunk: batch keys only
     dict(seqs=((300, 130), (17, 5)), H=4, Hkv=2, fill_unused=True),     # chunk against a cache, ragged
