@@ -909,7 +909,7 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
 }
 
 // Workgroups per compute unit and the largest tile each variant takes.
-int tiled_max_rows(int HD) { return HD == 512 ? 64 : 128; }  // 512: attn_tiled512_kernel's 2 row groups x 2 dim halves
+int tiled_max_rows(int HD) { return HD == 512 ? 64 : 128; }  // 512: attn_tiled512_kernel's 2 row groups of 32
 size_t tiled_smem_bytes(int HD) { return size_t(4) * 64 * HD * 2 + 64; }  // two stages of K (64 rows) and V^T (64 keys), 16 ints
 
 template <int DT, int HD>
