@@ -33,3 +33,18 @@ def test_every_measured_traffic_figure_has_its_summary_and_multi_launch_steps_ad
     assert bench.measured_traffic("no_such_workload") is None
     for w in bench.WORKLOADS:      # every named workload can at least be described without a device
         assert isinstance(w, str) and w
+
+
+def test_every_measured_traffic_figure_is_that_of_the_kernel_it_stands_under():
+    """The counters of a record are quoted in its summary for the kernel and at the commit that the record names."""
+    with open(os.path.join(ROOT, "profiles", "traffic.json")) as f:
+        t = json.load(f)
+    for w, rec in t.items():
+        if w.startswith("_"):
+            continue
+        text = open(os.path.join(ROOT, "profiles", f"{rec['kernel']}_{w}.txt")).read()
+        counted = [x.split() for x in text.splitlines() if f"::{rec['kernel']}" in x and "FETCH_SIZE" in x]
+        assert len(counted) == 1, w
+        at = counted[0].index("FETCH_SIZE")
+        assert abs(float(counted[0][at + 1]) - rec["fetch_kib"]) <= 0.06 and abs(float(counted[0][at + 3]) - rec["write_kib"]) <= 0.06, w
+        assert f"at commit {rec['measured_at_commit']}" in text and "the traffic counters at" not in text, w
