@@ -355,6 +355,8 @@ int esp_chain_advance(esp_tree* trees, int32_t n_trees, int32_t* pos, int32_t* r
  *     the attention as params.gate with gate_headwise = 1 (gate_ld = H, gate_hs = 1,
  *     gate_off = 0): the attention then multiplies before its one rounding and O makes no
  *     second trip through memory. This call can run before the attention (x is the layer's input).
+ *     The dots alone take 128 to 160 KB of LDS per workgroup (esp_attn_init allows it): no other kernel shares a
+ *     compute unit with them, so they gain nothing from a second stream.
  * At least one of O and dots. X [n_rows][x_ld], Wg [H][D], O [n_rows][q_ld]: storage type
  * (the reference: fp16). D % 8 == 0 (the reference: % 4), head_dim % 8 == 0 and <= 1024
  * as in the reference (:98), H <= 64. */
