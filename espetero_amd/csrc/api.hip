@@ -29,6 +29,7 @@ hipError_t gate_init_attributes();
 int tiled_max_rows(int HD);
 hipError_t stream_init_attributes();
 hipError_t tiled_init_attributes();
+hipError_t tiled256_init_attributes();
 hipError_t tiled512_init_attributes();
 }  // namespace esp
 
@@ -139,6 +140,7 @@ int device_state(DeviceState** out, char* err, size_t errlen) {
     if ((e = hipGetSymbolAddress(&ps, HIP_SYMBOL(scratch))) != hipSuccess) return hip_fail(err, errlen, "hipGetSymbolAddress(scratch)", e);
     if ((e = esp::stream_init_attributes()) != hipSuccess) return hip_fail(err, errlen, "hipFuncSetAttribute (streaming kernels)", e);
     if ((e = esp::tiled_init_attributes()) != hipSuccess) return hip_fail(err, errlen, "hipFuncSetAttribute (tiled kernels)", e);
+    if ((e = esp::tiled256_init_attributes()) != hipSuccess) return hip_fail(err, errlen, "hipFuncSetAttribute (tiled kernels, head dim 256)", e);
     if ((e = esp::tiled512_init_attributes()) != hipSuccess) return hip_fail(err, errlen, "hipFuncSetAttribute (tiled kernels, head dim 512)", e);
     if ((e = esp::gate_init_attributes()) != hipSuccess) return hip_fail(err, errlen, "hipFuncSetAttribute (head gate)", e);
     d.scratch = static_cast<unsigned char*>(ps);

@@ -1,4 +1,4 @@
-// Tiled MFMA attention for passes with many query rows per tree: prefill,
+// Tiled MFMA attention at head dim 128 for passes with many query rows per tree: prefill,
 // chunked prefill against the paged cache, large verify batches. Compute
 // bound: Q K^T and P V run on v_mfma_f32_32x32x16 with K and V^T staged in LDS.
 //
@@ -39,46 +39,13 @@
 
 #include "common.hpp"
 #include "lds_direct.hpp"
+#include "rows_out.hpp"
 
 namespace esp {
-
-// A wavefront's 32 output rows of RB bytes on their way through LDS: written by row (lane % 32), stored 1 KB of consecutive rows at a
-// time. The 16-byte parts of a row are turned by its number, which spreads both sides over the banks.
-template <int RB>
-struct RowsOut {
-  static constexpr int P = RB / 16, RPI = 64 / P;  // parts of a row; rows one store instruction takes
-  static __device__ __forceinline__ char* at(char* ob, int r, int p) { return ob + r * RB + (p ^ (r & (P < 16 ? P - 1 : 15))) * 16; }
-  // dst: where this lane's row (lane % 32) goes, 0 where there is none
-  static __device__ __forceinline__ void store(char* ob, uint64_t dst, int lane) {
-    using out16 = uint32_t __attribute__((ext_vector_type(4), aligned(8)));  // a row of O starts at any multiple of 8 bytes
-    __builtin_amdgcn_wave_barrier();
-    asm volatile("" ::: "memory");  // the rows are written: one wavefront's LDS accesses keep their order
-    const int lo = int(uint32_t(dst)), hi = int(uint32_t(dst >> 32));
-    constexpr int N = 32 / RPI, B = N < 8 ? N : 8;
-#pragma unroll
-    for (int j0 = 0; j0 < N; j0 += B) {
-      u32x4 v[B];
-      uint64_t d[B];
-#pragma unroll
-      for (int j = 0; j < B; ++j) {
-        const int r = (j0 + j) * RPI + lane / P;
-        v[j] = *reinterpret_cast<const u32x4*>(at(ob, r, lane % P));
-        d[j] = uint64_t(uint32_t(__shfl(lo, r))) | uint64_t(uint32_t(__shfl(hi, r))) << 32;
-      }
-#pragma unroll
-      for (int j = 0; j < B; ++j)
-        if (d[j]) *(__attribute__((address_space(1))) out16*)(d[j] + uint64_t(lane % P) * 16) = v[j];
-    }
-  }
-};
 
 template <int DT, int HD, int OCC>
 __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int n_tiles) {
   constexpr int KS = HD / 16, NT = HD / 32;
-  // Head dim 128 runs the softmax without a per-step maximum, in slices laid between the matrix instructions by
-  // hand (measured 3 % faster there); at head dim 256, with one wavefront per SIMD and every register taken,
-  // the same code spilled and ran 3 to 8 % slower than the form with a lazily moved maximum, which it keeps.
-  constexpr bool LEAN = HD == 128;
   constexpr int ROWB = HD * 2;     // bytes of one K row
   constexpr int CH = HD / 8;       // 16-byte chunks per K row
   constexpr int RPI = 64 / CH;     // K rows one load instruction covers
@@ -558,59 +525,6 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
         }
       }
     }
-    // The lane's maximum over the half step (head dim 256's lazy rescale; see softmax_move).
-    float x = -INFINITY;
-    if constexpr (!LEAN) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) x = fmaxf(x, sv[i]);
-      x *= a.scale_log2;  // scale > 0: the max commutes with it
-    }
-    return x;
-  };
-  // Lazy rescale: the running reference m_run only moves when some lane's maximum exceeds
-  // it by more than 8 (log2 units), so P stays below 2^8 and the accumulators are rescaled
-  // a handful of times per row instead of once per step. The two lanes of a row agree on
-  // m_run because both take the maximum over the pair whenever either wants to move.
-  auto softmax_move = [&](auto kt_c, float x, bool move) __attribute__((always_inline)) {
-    constexpr int kt = decltype(kt_c)::value;
-    if (move) {
-      asm volatile("s_nop 0");  // a real branch: this block must not be speculated into the loop body
-      const float m_new = fmaxf(m_run, fmaxf(x, __shfl_xor(x, 32)));
-      const float corr = (m_new == -INFINITY) ? 1.0f : fast_exp2(m_run - m_new);
-      m_run = m_new;
-      l_run *= corr;
-      if constexpr (kt == 0) {
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[nt] *= corr;
-      } else {
-        // P V of the first half step is still to be accumulated and its P is relative to the old
-        // reference: the accumulators take this factor once those products are in.
-        corr_late = corr;
-        late = true;
-      }
-    }
-  };
-  // Head dim 256: the straight-line part with the scale and the reference in one fused multiply-add per score.
-  // T0 .. T1: which of the half step's two sub-blocks of 16 keys (8 scores of this lane each) to do now: with
-  // two groups of matrix instructions per half step the second sub-block waits for the second group.
-  auto softmax_exp_fma = [&]<int T0, int T1>(auto kt_c) __attribute__((always_inline)) {
-    constexpr int kt = decltype(kt_c)::value;
-    const float m_safe = (m_run == -INFINITY) ? 0.0f : m_run;
-    float ps = 0.0f;
-#pragma unroll
-    for (int t = T0; t < T1; ++t) {
-      float p[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) p[e] = fast_exp2(__builtin_fmaf(s[kt][8 * t + e], a.scale_log2, -m_safe));
-      pb[kt][t] = u32x4{pack2<DT>(p[0], p[1]), pack2<DT>(p[2], p[3]), pack2<DT>(p[4], p[5]), pack2<DT>(p[6], p[7])};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ps = sum2<DT>(pb[kt][t][e], ps);  // the sum of the P the products use (see slice_pack)
-      // Pin the results here: without a use in this block the arithmetic above is sunk to the
-      // block of its first real use, away from the matrix instructions it should overlap with.
-      asm volatile("" : "+v"(pb[kt][t]));
-    }
-    l_run += ps;
-    asm volatile("" : "+v"(l_run));
   };
   // The straight-line part in eight slices, one pair of scores each: slice q subtracts the reference and
   // takes the exponentials of pair q, and packs and sums pair q - 1, whose exponentials have had a slice's
@@ -683,70 +597,33 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
     // issued instruction, a wait included, is time the matrix pipe idles.
     __builtin_amdgcn_s_waitcnt(G + 1 < NG ? kWaitLgkm8 : kWaitLgkm0);
     if constexpr (G == GK || G == 2 * GK) {
-      if constexpr (LEAN) {
-        // On the mask-free path there is no branchy part and the whole group carries the arithmetic.
-        constexpr int HEAD = decltype(interior)::value ? 0 : 3;  // (2, 4, 5: equal or slower - measured)
-        mma_group.template operator()<G, 0, HEAD>(ring[G & 1]);
-        __builtin_amdgcn_sched_barrier(0);
-        softmax_pre(step, std::integral_constant<int, G == GK ? 0 : 1>{}, interior);
-        __builtin_amdgcn_sched_barrier(0);
-        // One matrix instruction, then its share of the eight slices, fenced so that the order stands.
-        // The group's last matrix instructions wait until the half step's sum has been compared with its limit:
-        // they do not depend on P, and the branch on that comparison - a vector compare that the scalar unit has
-        // to wait for - then stands behind matrix instructions in flight instead of behind an idle pipe.
-        constexpr int TAILM = 2;  // (1: the same, 3: no gain - measured)
-        constexpr int NM = GP - HEAD - TAILM, KT = G == GK ? 0 : 1;
-        [&]<int... M>(std::integer_sequence<int, M...>) __attribute__((always_inline)) {
-          ([&]<int MI>() __attribute__((always_inline)) {
-            mma_group.template operator()<G, HEAD + MI, HEAD + MI + 1>(ring[G & 1]);
-            [&]<int... Q>(std::integer_sequence<int, Q...>) __attribute__((always_inline)) {
-              (slice.template operator()<KT, (8 * MI) / NM + Q>(), ...);
-            }(std::make_integer_sequence<int, (8 * (MI + 1)) / NM - (8 * MI) / NM>{});
-            __builtin_amdgcn_sched_barrier(0);
-          }.template operator()<M>(), ...);
-        }(std::make_integer_sequence<int, NM>{});
-        const float ps = softmax_finish.template operator()<KT>();
-        const bool out_of_range = __any(!(ps <= p_limit));
-        __builtin_amdgcn_sched_barrier(0);
-        mma_group.template operator()<G, GP - TAILM, GP>(ring[G & 1]);
-        __builtin_amdgcn_sched_barrier(0);
-        softmax_settle(std::integral_constant<int, G == GK ? 0 : 1>{}, ps, out_of_range);
-      } else {
-        // The first matrix instructions of the group go out before the branchy part of the softmax,
-        // whose wait for the previous group's results they cover; the rest carry the arithmetic,
-        // one matrix instruction then its share.
-        // (On steps with masks to work out five go first: 3 -> 5 is 1.3 % on sliding layers, 1 costs as much; 6 as 5.)
-        constexpr int HEAD = decltype(interior)::value ? 3 : 5, TAILH = 1;  // (TAILH 0: 1 % slower on full layers, 2: as 1 - measured)
-        constexpr std::integral_constant<int, G == GK ? 0 : 1> kt_c{};
-        mma_group.template operator()<G, 0, HEAD>(ring[G & 1]);
-        __builtin_amdgcn_sched_barrier(0);
-        const float x = softmax_pre(step, kt_c, interior);
-        const bool move = __any(x > m_run + 8.0f);
-        __builtin_amdgcn_sched_barrier(0);
-        // (matrix instructions between the comparison and the branch on it, as at head dim 128)
-        mma_group.template operator()<G, HEAD, HEAD + TAILH>(ring[G & 1]);
-        __builtin_amdgcn_sched_barrier(0);
-        softmax_move(kt_c, x, move);
-        __builtin_amdgcn_sched_barrier(0);
-        mma_group.template operator()<G, HEAD + TAILH, GP>(ring[G & 1]);
-        constexpr bool TWO = GK >= 2;  // the half step's Q K^T (or P V) is two groups: the second carries the other half
-        softmax_exp_fma.template operator()<0, TWO ? 1 : 2>(kt_c);
-#pragma unroll
-        for (int j = HEAD + TAILH; j < GP; ++j) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, (TWO ? 35 : 65) / (GP - HEAD - TAILH), 0);
-        }
-      }
-    } else if constexpr (!LEAN && GK >= 2 && (G == GK + 1 || G == 2 * GK + 1)) {
-      // the second sub-block's share of the softmax beside the half step's second group of matrix instructions
+      // On the mask-free path there is no branchy part and the whole group carries the arithmetic.
+      constexpr int HEAD = decltype(interior)::value ? 0 : 3;  // (2, 4, 5: equal or slower - measured)
+      mma_group.template operator()<G, 0, HEAD>(ring[G & 1]);
       __builtin_amdgcn_sched_barrier(0);
-      mma_group.template operator()<G, 0, GP>(ring[G & 1]);
-      softmax_exp_fma.template operator()<1, 2>(std::integral_constant<int, G == GK + 1 ? 0 : 1>{});
-#pragma unroll
-      for (int j = 0; j < GP; ++j) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
-      }
+      softmax_pre(step, std::integral_constant<int, G == GK ? 0 : 1>{}, interior);
+      __builtin_amdgcn_sched_barrier(0);
+      // One matrix instruction, then its share of the eight slices, fenced so that the order stands.
+      // The group's last matrix instructions wait until the half step's sum has been compared with its limit:
+      // they do not depend on P, and the branch on that comparison - a vector compare that the scalar unit has
+      // to wait for - then stands behind matrix instructions in flight instead of behind an idle pipe.
+      constexpr int TAILM = 2;  // (1: the same, 3: no gain - measured)
+      constexpr int NM = GP - HEAD - TAILM, KT = G == GK ? 0 : 1;
+      [&]<int... M>(std::integer_sequence<int, M...>) __attribute__((always_inline)) {
+        ([&]<int MI>() __attribute__((always_inline)) {
+          mma_group.template operator()<G, HEAD + MI, HEAD + MI + 1>(ring[G & 1]);
+          [&]<int... Q>(std::integer_sequence<int, Q...>) __attribute__((always_inline)) {
+            (slice.template operator()<KT, (8 * MI) / NM + Q>(), ...);
+          }(std::make_integer_sequence<int, (8 * (MI + 1)) / NM - (8 * MI) / NM>{});
+          __builtin_amdgcn_sched_barrier(0);
+        }.template operator()<M>(), ...);
+      }(std::make_integer_sequence<int, NM>{});
+      const float ps = softmax_finish.template operator()<KT>();
+      const bool out_of_range = __any(!(ps <= p_limit));
+      __builtin_amdgcn_sched_barrier(0);
+      mma_group.template operator()<G, GP - TAILM, GP>(ring[G & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+      softmax_settle(std::integral_constant<int, G == GK ? 0 : 1>{}, ps, out_of_range);
     } else {
       __builtin_amdgcn_sched_barrier(0);
       mma_group.template operator()<G, 0, GP>(ring[G & 1]);
@@ -922,23 +799,21 @@ static hipError_t launch_tiled_t(const KArgs& a, int n_tiles, hipStream_t st) {
   return hipGetLastError();
 }
 
+hipError_t launch_tiled256(int dt, const KArgs& a, int n_tiles, hipStream_t st);
 hipError_t launch_tiled512(int dt, const KArgs& a, int n_tiles, hipStream_t st);
 
 // The dynamic LDS limit of every variant on the current device, ahead of the first launch.
 hipError_t tiled_init_attributes() {
   hipError_t e = allow_dynamic_lds<attn_tiled_kernel<ESP_F16, 128, tiled_occ(128)>>(tiled_smem_bytes(128));
-  if (e == hipSuccess) e = allow_dynamic_lds<attn_tiled_kernel<ESP_F16, 256, tiled_occ(256)>>(tiled_smem_bytes(256));
   if (e == hipSuccess) e = allow_dynamic_lds<attn_tiled_kernel<ESP_BF16, 128, tiled_occ(128)>>(tiled_smem_bytes(128));
-  if (e == hipSuccess) e = allow_dynamic_lds<attn_tiled_kernel<ESP_BF16, 256, tiled_occ(256)>>(tiled_smem_bytes(256));
   return e;
 }
 
 hipError_t launch_tiled(int dt, int HD, const KArgs& a, int n_tiles, hipStream_t st) {
   if (HD == 512 && (dt == ESP_F16 || dt == ESP_BF16)) return launch_tiled512(dt, a, n_tiles, st);
+  if (HD == 256 && (dt == ESP_F16 || dt == ESP_BF16)) return launch_tiled256(dt, a, n_tiles, st);
   if (dt == ESP_F16 && HD == 128) return launch_tiled_t<ESP_F16, 128>(a, n_tiles, st);
-  if (dt == ESP_F16 && HD == 256) return launch_tiled_t<ESP_F16, 256>(a, n_tiles, st);
   if (dt == ESP_BF16 && HD == 128) return launch_tiled_t<ESP_BF16, 128>(a, n_tiles, st);
-  if (dt == ESP_BF16 && HD == 256) return launch_tiled_t<ESP_BF16, 256>(a, n_tiles, st);
   return hipErrorInvalidValue;
 }
 

@@ -394,6 +394,22 @@ def test_tiled_kernel_head_dim_512_few_steps(kw, dtype):
     _check(small_case(seed=49, HD=512, H=4, Hkv=2, rows_per_tile=64, dtype=dtype, **kw))
 
 
+@pytest.mark.parametrize("kw", [
+    dict(seqs=((0, 63), (0, 64), (0, 65), (0, 1))),                     # either side of a row group; a group without rows beside one with
+    dict(seqs=((64, 64), (63, 127), (65, 128), (128, 3))),              # whole steps of cached keys, one key over and under; the first mask-free step
+    dict(seqs=((16, 5), (48, 33), (1100, 97)), fill_unused=True),       # the pass's last group of rows is cut; what was never written is NaN
+    dict(seqs=((4200, 70), (4160, 2)), H=2, Hkv=1),                     # more than 64 steps: addresses worked out twice
+    dict(seqs=((400, 64), (333, 40)), window=40),                       # rows that see nothing of their tile's first steps
+    dict(seqs=((0, 150), (200, 130)), window=17),                       # a window within the batch rows
+    dict(seqs=((0, 16), (7, 17), (20, 31), (3, 32), (40, 63)), bt=64),
+])
+@pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
+@pytest.mark.parametrize("with_desc", [True, False])
+def test_tiled_kernel_head_dim_256_edges(kw, dtype, with_desc):
+    """Two wavefronts share a step's scores by keys and its output by dims, P V a step behind: what begins and ends rows, ranges and steps."""
+    _check(small_case(seed=61, HD=256, rows_per_tile=128, dtype=dtype, **{"H": 4, "Hkv": 2, **kw}), with_desc=with_desc)
+
+
 @pytest.mark.parametrize("HD", [128, 256])
 @pytest.mark.parametrize("seqs", [((100, 1), (40, 31), (7, 33)), ((200, 127), (0, 128), (65, 97)), ((3000, 40),)])
 @pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])

@@ -15,7 +15,7 @@ import isa_hazards
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "espetero_amd", "csrc")
 HIPCC = "/opt/rocm/bin/hipcc"
-SOURCES = ["attn_stream.hip", "attn_tiled.hip", "attn_tiled512.hip", "head_gate.hip"]
+SOURCES = ["attn_stream.hip", "attn_tiled.hip", "attn_tiled256.hip", "attn_tiled512.hip", "head_gate.hip"]
 
 
 def test_scanner_flags_a_reader_behind_a_branch_and_not_a_padded_one():
