@@ -151,15 +151,15 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
   // sub-block; the lane that fills chunk position `lane` of row r brings chunk lane ^ r.
   // V^T: this wavefront brings pieces 256 wave .. + 255 of each sub-block's
   // 1024 (piece c: keys 8 (c % 2) .. + 7 of dim c / 2); position p holds piece p ^ ((p >> 4) & 1).
-  const uint32_t lds_base = uint32_t(uintptr_t(lds));
+  constexpr uint32_t lds_base = 0;  // the dynamic array is the only LDS object
   // Pool addresses of the sub-blocks, 64 at a time: lane l holds the byte address of the K rows of sub-block adr0 + l
   // (block list entry, the head's place in the block, the sub-block's place in the head, worked out by 64 lanes at
   // once), so that in front of a sub-block's staging loads stand two lane reads instead of a dependent memory access
   // and the scalar arithmetic behind it. V^T of a sub-block lies bt rows' worth of bytes behind its K rows.
   uint32_t kadr_lo = 0, kadr_hi = 0;
-  int adr0 = -(1 << 30);
+  int adr0 = -64;
   auto pool_k = [&](int sidx) __attribute__((always_inline)) {
-    if (sidx < adr0 || sidx >= adr0 + 64) {
+    if (sidx - adr0 >= 64) {  // (sub-blocks are asked for in order)
       adr0 = sidx;
       const int sl = sidx + lane;
       const int js = sl < n_c ? (c0 + sl) << 4 : (in_pool && sl < n_sb) ? ((a0 + sl - n_c) << 4) + pool_shift : -1;
@@ -170,6 +170,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
       }
       kadr_lo = uint32_t(adr);
       kadr_hi = uint32_t(adr >> 32);
+      asm volatile("" : "+v"(kadr_lo), "+v"(kadr_hi));  // arrived here: a wait at the lane reads below would drain the staging loads
     }
     const int idx = sidx - adr0;
     const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(kadr_lo), idx)), hi = uint32_t(__builtin_amdgcn_readlane(int(kadr_hi), idx));
@@ -186,19 +187,19 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
     k_src = pool_k(2 * step + t) + wave * 4096;
     v_src[t] = k_src + size_t(a.bt) * 1024;  // the 16-token sub-block: 16 KB contiguous
   };
-  auto load_k = [&]<int H>(int t, int stage) __attribute__((always_inline)) {
+  auto load_k = [&](int t, int stage) __attribute__((always_inline)) {
     const uint32_t kl = uint32_t(lane);
-    load_to_lds16_x2<H>(k_src, (kl ^ (kx + 2 * H)) << 4, (kl ^ (kx + 2 * H + 1)) << 4, lds_base + stage * kKStage + (16 * t + 4 * wave) * 1024);
+    load_to_lds16_x4(k_src, (kl ^ kx) << 4, (kl ^ (kx + 1)) << 4, (kl ^ (kx + 2)) << 4, (kl ^ (kx + 3)) << 4,
+                     lds_base + stage * kKStage + (16 * t + 4 * wave) * 1024);
   };
-  auto load_v = [&]<int H>(int t, int stage) __attribute__((always_inline)) {
-    load_to_lds16_x2<H>(v_src[t], voff, voff, lds_base + kVBase + stage * kVStage + t * kVSub + wave * 4096);
+  auto load_v = [&](int t, int stage) __attribute__((always_inline)) {
+    load_to_lds16_x4(v_src[t], voff, voff, voff, voff, lds_base + kVBase + stage * kVStage + t * kVSub + wave * 4096);
   };
   auto fill_k = [&](int t, int step, int stage) __attribute__((always_inline)) {
     const int sidx = 2 * step + t;
     if (sidx < n_c || (in_pool && sidx < n_sb)) {
       locate_k(t, step);
-      load_k.template operator()<0>(t, stage);
-      load_k.template operator()<1>(t, stage);
+      load_k(t, stage);
     } else if (sidx < n_sb) {
       const int g = a0 + (sidx - n_c);
       const int lim = a.n_rows - 1 - 16 * g;  // batch rows past the pass's last row do not exist: repeat the last (masked)
@@ -214,8 +215,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
   };
   auto fill_v = [&](int t, int stage) __attribute__((always_inline)) {
     if (v_src[t]) {
-      load_v.template operator()<0>(t, stage);
-      load_v.template operator()<1>(t, stage);
+      load_v(t, stage);
     } else {  // V^T must be finite
 #pragma unroll
       for (int q = 0; q < 4; ++q)
@@ -385,7 +385,6 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
 #pragma unroll
       for (int j = 0; j < 4; ++j) buf[j] = *lds_ptr(kaddr[j] + off);
     };
-    const uint32_t koff = uint32_t(S * kKStage);
     const uint32_t va = vaddr + uint32_t((S ^ 1) * kVStage), pa = paddr + uint32_t((S ^ 1) * kPBuf);
     auto read_v = [&](u32x4 (&buf)[4], int t, int nt0) __attribute__((always_inline)) {
 #pragma unroll
@@ -408,7 +407,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       if (g < 3) {
-        read_k(ring[(g + 1) & 1], koff + uint32_t(256 * (g + 1)));
+        read_k(ring[(g + 1) & 1], uint32_t(256 * (g + 1)));
       } else {
         read_v(ring[0], 0, 0);
 #pragma unroll
@@ -422,12 +421,9 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
         if (PLAIN && (j & 1)) {
           const int slot = 2 * g + (j >> 1);
           __builtin_amdgcn_sched_barrier(0);
-          if (slot == 0) load_v.template operator()<0>(1, S);
-          if (slot == 1) load_v.template operator()<1>(1, S);
-          if (slot == 2) locate_k(0, i + 1), load_k.template operator()<0>(0, S ^ 1);
-          if (slot == 3) load_k.template operator()<1>(0, S ^ 1);
-          if (slot == 4) locate_k(1, i + 1), load_k.template operator()<0>(1, S ^ 1);
-          if (slot == 5) load_k.template operator()<1>(1, S ^ 1);
+          if (slot == 0) load_v(1, S);
+          if (slot == 2) locate_k(0, i + 1), load_k(0, S ^ 1);
+          if (slot == 4) locate_k(1, i + 1), load_k(1, S ^ 1);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -459,12 +455,14 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
       exp_pack(S);
     }
     const int mine = __any(ps[0] > 256.0f || ps[1] > 256.0f);
-    if (lane == 0) flags[S][wave] = mine;
+    *reinterpret_cast<__attribute__((address_space(3))) int*>(uint32_t(kFlags + S * 16 + wave * 4)) = mine;  // (every lane the same: cheaper than one alone)
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // own loads landed, own reads of this iteration's stages done
     if constexpr (!PLAIN) fix(i, S);
     __syncthreads();
-    const u32x4 fl = *lds_ptr(lds_base + uint32_t(kFlags + S * 16));
-    read_k(ring[0], koff ^ uint32_t(kKStage));
+    const int fl = *reinterpret_cast<const __attribute__((address_space(3))) int*>(uint32_t(kFlags + S * 16 + (lane & 3) * 4));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) kaddr[j] ^= uint32_t(kKStage);  // the other stage
+    read_k(ring[0], 0);
     __builtin_amdgcn_sched_barrier(0);
     auto left = [&](int j) __attribute__((always_inline)) {
       if (PLAIN || i > 0) acc[4 + j] = mfma32x16<DT>(carry[j], pf[1], acc[4 + j]);
@@ -473,16 +471,14 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
     left(0);
     left(1);
     if constexpr (PLAIN) {
-      load_v.template operator()<0>(0, S ^ 1);
+      load_v(0, S ^ 1);
     } else {
       if (i + 1 < n_steps) fill_v(0, S ^ 1);
     }
     __builtin_amdgcn_sched_barrier(0);
     left(2);
     left(3);
-    if constexpr (PLAIN) load_v.template operator()<1>(0, S ^ 1);
-    __builtin_amdgcn_sched_barrier(0);
-    out_of_range = __builtin_amdgcn_readfirstlane(int(fl.x | fl.y | fl.z | fl.w));
+    out_of_range = __any(fl != 0);
   };
   constexpr std::false_type general{};
   constexpr std::true_type plain{};
