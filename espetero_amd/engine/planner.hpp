@@ -474,6 +474,45 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
       mixed = true;
       choose(std::max(room, parts_in(ns_of)));
     }
+    // A pass of few workgroups, at most one for two compute units, that nothing has cut so far - behind a window, or behind few keys - ends
+    // with its longest tile while the rest of the chip stands idle: its tiles are cut until the parts fill the chip once, as long as
+    // that is shorter with the merge's dispatch and the records there and back. In us: what a lone workgroup takes for 64 keys, 7 for
+    // the merge and 0.35 for each MB of records. 100 rows behind a window of 1024, 16 / 8 heads of 256: 41.5 whole, 29.8 in four parts; 356 rows,
+    // 8 / 2 heads: 46.2 and 32.6; six of 41 .. 82 rows 40.1 and 29.2; three of 128 rows 43.0 and 34.9; 128 rows over 900 keys, 32 / 4 heads
+    // of 128: 28.0 and 20.6. Not two chunks of 300 rows over 500 keys, 16 heads of 256: 35.0 whole, 40.8 in two parts each; and not beyond
+    // what the rule above has cut (100 rows over 6871 keys 40.3 in its eight parts, 42.8 in fourteen). Passes with decoding rows are left
+    // to the rules above, and whatever is planned fits esp_attn_forward_static.
+    if (shape.family < 0 && !o.cut_batch && parts_in(ns_of) == 0 && grid * 2 <= esp::kComputeUnits && slots >= esp::kComputeUnits && o.part_steps > 0 &&
+        std::none_of(rts.begin(), rts.end(), [&](const RowTile& rt) { return rt.r == 0 && live_rows(rt) <= 16; })) {
+      const double step_us = shape.head_dim == 128 ? 1.3 : shape.head_dim == 256 ? 1.75 : 2.0;
+      const long long room = most_static_parts();
+      auto lone_us = [&](const std::vector<int>& ns_v) {
+        long long keys = 0;
+        double records = 0;
+        for (int i = 0; i < n_tiles; ++i) {
+          const RowTile& rt = rts[size_t(i)];
+          const long long ns = ns_v[size_t(i)], per = (rt.span + rt.batch + ns - 1) / ns, step = (per + o.granule - 1) / o.granule * o.granule;
+          keys = std::max(keys, ns > 1 ? std::max(step, rt.span + rt.batch - (ns - 1) * step) : (long long)(rt.span) + rt.batch);
+          if (ns > 1) records += double(ns) * live_rows(rt);
+        }
+        const double bytes = records * groups * shape.head_dim * 4;
+        return double((keys + o.granule - 1) / o.granule) * step_us + (records > 0 ? 7 + bytes * 0.35e-6 : 0);
+      };
+      double best = lone_us(ns_of);
+      for (long long c = c_hi - 1; c >= 2; --c) {
+        long long records = 0;
+        for (int i = 0; i < n_tiles; ++i) {
+          const RowTile& rt = rts[size_t(i)];
+          // parts of c steps, none of them without cached keys
+          const long long chunk = c * o.granule;
+          cand[size_t(i)] = int(std::clamp<long long>(std::min((rt.span + rt.batch + chunk - 1) / chunk, rt.span / chunk + 1), 1, o.max_splits));
+          records += cand[size_t(i)];
+        }
+        if (records * groups > esp::kComputeUnits || parts_in(cand) > room) break;
+        const double t = lone_us(cand);
+        if (t < best) best = t, ns_of = cand;
+      }
+    }
     order_records(ns_of);
   } else if (o.balanced && n_tiles > 0) {
     ns_of = stream_split(rts, o, shape, std::max(1, o.groups_target / std::max(1, groups)), most_static_parts(), parts_of);

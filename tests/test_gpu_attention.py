@@ -592,6 +592,19 @@ def test_tiled_kernel_cuts_the_batch_keys_of_a_tile(kw):
     assert np.abs(f32(got, c.params.dtype) - f32(whole, c.params.dtype)).max() <= 2e-3
 
 
+@pytest.mark.parametrize("HD", [128, 256, 512])
+@pytest.mark.parametrize("kw", [
+    dict(seqs=((1500, 100),), window=1024),                 # a window's keys in parts, the last with the batch rows
+    dict(seqs=((3000, 60), (1020, 33)), window=1024),
+    dict(seqs=((900, 70),), dtype=abi.ESP_BF16),            # fewer keys than the other rules cut
+])
+def test_tiled_kernels_few_workgroups_are_cut(HD, kw):
+    from gpu_utils import default_options, plan
+    c = small_case(seed=63, HD=HD, H=4, Hkv=2, rows_per_tile=64 if HD == 512 else 128, **kw)
+    assert plan(c, default_options(c))[2] >= 2
+    _check(c)
+
+
 def test_tiled_kernel_split_tiles_and_combine():
     """A single long-context tile group is split over key ranges and merged."""
     c = small_case(seed=42, seqs=((3000, 100),), H=4, Hkv=2, rows_per_tile=128)

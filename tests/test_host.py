@@ -807,6 +807,25 @@ def test_a_layer_that_no_kernel_serves_is_planned_for_any_layer():
             assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("layer,slots,seqs", [
+    ((32, 4, 128), 512, ((896, 128),)), ((16, 8, 256), 256, ((960, 100),)), ((8, 2, 256), 256, ((704, 300), (960, 17))), ((16, 2, 512), 512, ((960, 64),)),
+])
+def test_passes_of_few_workgroups_are_cut(layer, slots, seqs):
+    """Valid parts that fill the chip at most once and fit the library's own array; whole as before with decoding rows among them,
+    with more workgroups, or where the layer is not known."""
+    H, Hkv, HD = layer
+    rows = 64 if HD == 512 else 128
+    o = host.options_mi355x(rows, slots)
+    plan = lambda s, g: host.plan_tiles(_pass_of(s), g, 0, None, o)  # noqa: E731
+    tiles, jobs, parts = plan(seqs, _layer_groups(H, Hkv, HD, rows))
+    assert parts >= 2 and len(tiles) * H <= 256
+    _check_tiled_partition(_pass_of(seqs), tiles, jobs, parts, o)
+    assert _static_scratch(layer, rows, _pass_of(seqs), parts) <= abi.ESP_STATIC_SCRATCH_BYTES
+    assert plan(seqs, H)[2] == 0
+    assert plan(seqs + ((800, 1),), _layer_groups(H, Hkv, HD, rows))[2] == 0
+    assert plan(seqs * 40, _layer_groups(H, Hkv, HD, rows))[2] == 0
+
+
 def _ones(*cached):
     return tuple((P, 1) for P in cached)
 
