@@ -212,34 +212,38 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   int k_last = -1, seg_max = 0, qpos_max = 0;
   bool anc_any = false;  // does any row of the tile see ancestors (keys below its segment)?
   {
-    int kl = -1, sm = 0, am = 0, qm = INT32_MIN;
-    if (row_ok) {
-      kl = max(rr, max(d.z - 1, a.bidi ? d.w - 1 : -1));
-      sm = d.x;
-      am = d.z;
-      qm = qpos;
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      kl = max(kl, __shfl_xor(kl, o));
-      sm = max(sm, __shfl_xor(sm, o));
-      am = max(am, __shfl_xor(am, o));
-      qm = max(qm, __shfl_xor(qm, o));
-    }
-    if (lane == 0) {
-      red[wave][0] = kl;
-      red[wave][1] = sm;
-      red[wave][2] = am;
-      red[wave][3] = qm;
-    }
-    __syncthreads();
     int anc_max = 0;
+    if (!a.desc && a.window == 0) {  // rows see what lies below them, and that is all
+      k_last = rr0 + rows_live - 1;
+    } else {
+      int kl = -1, sm = 0, am = 0, qm = INT32_MIN;
+      if (row_ok) {
+        kl = max(rr, max(d.z - 1, a.bidi ? d.w - 1 : -1));
+        sm = d.x;
+        am = d.z;
+        qm = qpos;
+      }
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      k_last = max(k_last, red[w][0]);
-      seg_max = max(seg_max, red[w][1]);
-      anc_max = max(anc_max, red[w][2]);
-      qpos_max = max(qpos_max, red[w][3]);
+      for (int o = 32; o >= 1; o >>= 1) {
+        kl = max(kl, __shfl_xor(kl, o));
+        sm = max(sm, __shfl_xor(sm, o));
+        am = max(am, __shfl_xor(am, o));
+        qm = max(qm, __shfl_xor(qm, o));
+      }
+      if (lane == 0) {
+        red[wave][0] = kl;
+        red[wave][1] = sm;
+        red[wave][2] = am;
+        red[wave][3] = qm;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        k_last = max(k_last, red[w][0]);
+        seg_max = max(seg_max, red[w][1]);
+        anc_max = max(anc_max, red[w][2]);
+        qpos_max = max(qpos_max, red[w][3]);
+      }
     }
     // The same in every lane; saying so keeps everything derived from them in scalar registers.
     // a part whose batch range is cut ends at row last - 2 of the tree (last = 1: open, up to what its rows see)
@@ -778,7 +782,11 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
     finish_output<DT>(a, acc, l > 0.0f ? 1.0f / l : 0.0f, row, h, 0, half, [&](int i, u32x2 v) __attribute__((always_inline)) {
       *reinterpret_cast<u32x2*>(RowsOut<2 * HD>::at(ob, r32, i) + 8 * half) = v;
     });
-  RowsOut<2 * HD>::store(ob, row_ok ? reinterpret_cast<uint64_t>(a.O + size_t(row) * a.q_ld + size_t(h) * HD) : 0, ln);
+  if (packed && a.G > 1) {
+    RowsOut<2 * HD>::store(ob, row_ok ? reinterpret_cast<uint64_t>(a.O + size_t(row) * a.q_ld + size_t(h) * HD) : 0, ln);
+  } else {
+    RowsOut<2 * HD>::store_even(ob, a.O + size_t(tile.r0 + 32 * wave) * a.q_ld + size_t(h) * HD, uint32_t(a.q_ld) * 2, rows_live - 32 * wave, ln);
+  }
 }
 
 // Workgroups per compute unit and the largest tile each variant takes.
