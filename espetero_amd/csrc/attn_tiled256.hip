@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
   u32x4 qrow[16];
   {
     const char* q0 = reinterpret_cast<const char*>(a.Q + size_t(tile.r0) * a.q_ld + size_t(kvh * a.G + hg) * kHD);
-    const uint32_t ld = uint32_t(a.q_ld) * 2, last = uint32_t(a.n_rows - 1 - tile.r0) * ld + uint32_t(l32) * 16;
+    const uint32_t ld = uint32_t(a.q_ld) * 2, last = uint32_t(min(a.n_rows - 1 - tile.r0, 127)) * ld + uint32_t(l32) * 16;
     uint32_t at = uint32_t(2 * wave + hb) * ld + uint32_t(l32) * 16;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
