@@ -901,7 +901,7 @@ def timed_run(w, torch, steps, warmup, kernel_samples=None):
 
 def kernel_name(w):
     return getattr(w, "kernel", None) or ("attn_stream_kernel" if w.params.rows_per_tile * (w.H // w.Hkv) <= 32
-                                          else "attn_tiled512_kernel" if w.HD == 512 else "attn_tiled_kernel")
+                                          else {512: "attn_tiled512_kernel", 256: "attn_tiled256_kernel"}.get(w.HD, "attn_tiled_kernel"))
 
 
 def roofline(w, per_step_ms):
