@@ -13,9 +13,9 @@
 //   P^T = exp2(S^T - m)                                                        left in LDS in 16 bits
 //   O^T[128 dims][64 rows] += V^T . P^T                                        its 128 dims, all 64 keys; A = V^T and B = P^T from LDS
 // so that every operand read from LDS feeds two matrix instructions. P V runs one step behind Q K^T: one barrier per step publishes
-// the staged data and the P at once, and the softmax of step i stands
-// beside P V instructions that do not depend on it. K runs one step ahead of V in the staging. The row's reference m moves only where a
-// lane's share of a step's sum says so, and in the whole workgroup at once: the two wavefronts of a row group multiply each other's P.
+// the staged data and the P at once, and the softmax of step i stands beside P V instructions that do not depend on it. K runs one step
+// ahead of V in the staging. The row's reference m moves only where a lane's share of a step's sum says so, and in the whole workgroup at
+// once: the two wavefronts of a row group multiply each other's P.
 //
 // What bounds it: the issue of a lone wavefront per SIMD (accumulators 128 registers, Q 128, the rest 146). Such a wavefront issues an
 // instruction every 8 clocks (measured: 2, 4, 6, 8 multiply-adds behind every v_mfma_f32_32x32x16 make it 33, 38, 51, 66 clocks; two
