@@ -381,33 +381,31 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
     }
   }
 
-  // After this wavefront's loads of V^T of `step` have landed: cached keys outside [k0, k1) may be memory never written and keys
-  // past the range are not its own; their V must not reach the products.
+  // After this wavefront's loads of V^T of `step` have landed: cached keys outside [k0, k1) may be memory never written, other trees' rows
+  // and keys past the range are not its own; their V must not reach the products (0 x infinity).
   auto fix = [&](int step, int stage) __attribute__((always_inline)) {
     const int s = 4 * step + wave;
-    // keys [v0, v1) of the sub-block's own numbering count: the tile's cached range, or, for batch rows read from the
-    // pool, everything up to the tree's last row (what lies below its first row is the end of its cached keys)
+    // keys [v0, v1) of the sub-block's own numbering count: the tile's cached range, or the tree's rows. (In Kb / Vb the
+    // rows beside them are other trees'; in the pool what lies below its first row is the end of its cached keys.)
     int j0 = 0, v0 = 0, v1 = 0;
     if (s < n_c) {
       j0 = (c0 + s) << 4;
       v0 = tile.k0;
       v1 = tile.k1;
     } else if (s < n_sb) {
-      if (!in_pool) return;
       j0 = ((a0 + s - n_c) << 4) - tree.base;
-      v0 = INT32_MIN;
-      v1 = tree.M;
+      v0 = in_pool ? -16 : 0;  // (a sub-block begins less than 16 rows in front of the tree)
+      v1 = !in_pool && end == a.n_rows ? 1 << 30 : tree.M;  // (past the pass's last row the staged V^T is zero)
     }
     if (j0 >= v0 && j0 + 16 <= v1) return;
     const int jv = j0 + 8 * hb;
+    const int e0 = min(max(v0 - jv, 0), 8), e1 = min(max(v1 - jv, e0), 8);
+    const uint32_t in = (1u << e1) - (1u << e0);  // this lane's 8 keys, a bit each
     u32x4 msk;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bool lo = jv + 2 * e >= v0 && jv + 2 * e < v1;
-      const bool hi = jv + 2 * e + 1 >= v0 && jv + 2 * e + 1 < v1;
-      msk[e] = (lo ? 0xffffu : 0u) | (hi ? 0xffff0000u : 0u);
-    }
-#pragma unroll 2
+    for (int e = 0; e < 4; ++e)
+      msk[e] = (uint32_t(__builtin_amdgcn_sbfe(int(in), 2 * e, 1)) & 0xffffu) | uint32_t(__builtin_amdgcn_sbfe(int(in), 2 * e + 1, 1)) << 16;
+#pragma unroll 4
     for (int q = 0; q < 8; ++q) {
       u32x4* p = reinterpret_cast<u32x4*>(lds + kVBase + stage * kVStage + wave * kVSub + q * 1024 + lane * 16);
       *p = *p & msk;
@@ -512,7 +510,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
   };
   // Some lane of the workgroup found a reference too low for the step whose P is in buffer `buf` (or not set): every row takes the
   // maximum of that step over both wavefronts of its group, moves its reference, rescales what is accumulated, and the step's P is
-  // written again. Every wavefront of the workgroup comes through here together (one without rows only to its barriers).
+  // written again. Every wavefront of the workgroup comes through here together (one whose group has ended only to its barriers).
   auto settle = [&](int buf) __attribute__((always_inline)) {
     asm volatile("s_nop 0");  // a real branch: this block must not be speculated into the loop body
     char* mx_sh = lds + kPBase + buf * kPBuf;
@@ -539,6 +537,19 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
   };
 
   const int wave_first[2] = {__builtin_amdgcn_readfirstlane(rr[0]), __builtin_amdgcn_readfirstlane(rr[1])};  // of either row tile
+  // Steps this row group computes: batch steps past its last row hold nothing it can see, and their V, infinities among them, must not
+  // reach its products. A group without a row (or with nothing to see) has only its share of the staging to do. `both`: the first
+  // row tile sees something of the group's last step too.
+  int my_steps = wave_first[0] < rr0 + rows_live ? n_steps : 0;
+  bool both = true;
+  if (seg_max != INT32_MAX) {
+    auto step_end = [&](int rt) __attribute__((always_inline)) {  // one past the last step with a key at or below the row tile's last row
+      const int last = min(__builtin_amdgcn_readlane(rr[rt], 31), rr0 + rows_live - 1);
+      return last < tile.b0 ? (n_c + 3) >> 2 : (n_c + ((tree.base + last) >> 4) - a0 + 4) >> 2;
+    };
+    my_steps = min(my_steps, step_end(1));
+    both = step_end(0) >= my_steps;
+  }
   // Keys this lane's rows see: cached ones [lo_c, k1), batch ones [lo_b, end_b), or b0 <= j < anc. b0 is the first batch key any
   // row of the tile sees (the window's lower edge; 0 without one): the first sub-block starts at a multiple of 16 rows at or below it,
   // and what lies below b0 is invisible.
@@ -733,8 +744,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
   // of them: cached steps [int_lo, c_hi) - inside [k0, k1) and inside every row's window - and batch steps
   // [b_lo, b_hi), whose rows all lie below the tile's first row (and at or above b0, inside every segment,
   // with no ancestors and no per-key window test pending). Where the cached range ends on a step boundary
-  // the two runs are one. Steps that
-  // hold nothing a row group can see it computes all the same, fully masked: the workgroup's other group has them to do.
+  // the two runs are one.
   int int_lo, c_hi, b_lo = 0, b_hi = 0;
   {
     const int first = c0 << 4;  // key of sub-block 0
@@ -756,66 +766,77 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
     }
   }
 
-  auto l_sh = [&]() __attribute__((always_inline)) { return reinterpret_cast<float*>(lds + kPBase + (n_steps & 1) * kPBuf); };
+  // Where a row group's sums cross: each wavefront's in its own P, in the buffer that the last step's does not take.
+  auto l_sh = [&](int w) __attribute__((always_inline)) { return reinterpret_cast<float*>(lds + kPBase + (my_steps & 1) * kPBuf + w * kPWave); };
   if (n_steps > 0) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // K of step 0 landed, Q fragments read
     __syncthreads();
-    if (wave_first[0] < rr0 + rows_live) {
+    if (my_steps > 0) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) ring[0][j] = k_operand.template operator()<0>(j);
       iter.template operator()<true>(0, false);
       clear();
 #pragma nounroll
-      for (int i = 1; i < n_steps; ++i) {
+      for (int i = 1; i < my_steps; ++i) {
         if (out_of_range) settle((i - 1) & 1);
         iter.template operator()<false>(i, (i >= int_lo && i < c_hi) || (i >= b_lo && i < b_hi));
       }
-      // ---- what is left: P V of the last step
-      const int S = (n_steps - 1) & 1;
-      if (out_of_range) settle(S);
-      const uint32_t va = vaddr + uint32_t(S * kVStage), pa = paddr + uint32_t(S * kPBuf);
-#pragma unroll
-      for (int rt = 0; rt < 2; ++rt) {  // the rows' sums, for the group's other wavefront: in the buffer of the P before
-        l_run[rt] += ps[rt];
-        l_run[rt] += __shfl_xor(l_run[rt], 32);
-        if (hb == 0) l_sh()[(wave * 2 + rt) * 32 + l32] = l_run[rt];
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) ring[0][nt] = v_operand(va, t, nt);
-#pragma unroll
-        for (int rt = 0; rt < 2; ++rt) pf[0][rt] = p_operand(pa, t, rt);
-#pragma unroll
-        for (int n = 0; n < 8; ++n) mul_v1(ring[0], pf[0], n);
-      }
-    } else {  // a group without a row has only its share of the staging to do
+      if (out_of_range) settle((my_steps - 1) & 1);
+      out_of_range = false;
+    } else {
       clear();
       if (lane < 2) *reinterpret_cast<int*>(lds + kPBase + lane * kPBuf + wave * kPWave + kFlagAt) = 0;  // its P never asks for a reference
-#pragma nounroll
-      for (int i = 0; i < n_steps; ++i) {
-        if (out_of_range) settle_beside();
-        const int S = i & 1;
-        if (i == 0) {
-          __syncthreads();  // (the maxima of the first step)
-        } else {
+    }
+    // ---- what is left: P V of the group's last step, and its share of the staging of those that the other group goes on with. (Its own
+    // flags stay clear from here on: a settled step's are, and the other buffer's it clears itself.)
+    bool left = my_steps > 0;
+    for (int i = my_steps;; ++i) {
+      const int S = i & 1;
+      if (out_of_range) settle_beside();
+      if (i < n_steps) {
+        if (i > 0) {
           load_v.template operator()<2>(S);
           load_v.template operator()<3>(S);
         }
         locate(i + 1);
         load_k_all(S ^ 1);
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        if (cut_src) {
-          load_cut(S ^ 1);
-          wait_loads();
-        }
-        fix(i, S);
-        __syncthreads();
-        out_of_range = __any(flags_of(S) < 0) != 0;
-        load_v.template operator()<0>(S ^ 1);
-        load_v.template operator()<1>(S ^ 1);
       }
-      if (out_of_range) settle_beside();
+      if (left) {
+        left = false;
+        const uint32_t va = vaddr + uint32_t((S ^ 1) * kVStage), pa = paddr + uint32_t((S ^ 1) * kPBuf);
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+          l_run[rt] += ps[rt];
+          l_run[rt] += __shfl_xor(l_run[rt], 32);
+          if (hb == 0) l_sh(wave)[32 * rt + l32] = l_run[rt];
+        }
+        if (lane == 0) l_sh(wave)[kFlagAt / 4] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+#pragma unroll
+          for (int nt = 0; nt < 4; ++nt) ring[0][nt] = v_operand(va, t, nt);
+#pragma unroll
+          for (int rt = 0; rt < 2; ++rt) pf[0][rt] = p_operand(pa, t, rt);
+          if (both) {
+#pragma unroll
+            for (int n = 0; n < 8; n += 2) mul_v1(ring[0], pf[0], n);
+          }
+#pragma unroll
+          for (int n = 1; n < 8; n += 2) mul_v1(ring[0], pf[0], n);
+        }
+      }
+      if (i >= n_steps) break;
+      if (i == 0) __syncthreads();  // (the maxima of the first step)
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      if (cut_src) {
+        load_cut(S ^ 1);
+        wait_loads();
+      }
+      fix(i, S);
+      __syncthreads();
+      out_of_range = __any(flags_of(S) < 0) != 0;
+      load_v.template operator()<0>(S ^ 1);
+      load_v.template operator()<1>(S ^ 1);
     }
     wait_loads();
   } else {
@@ -824,10 +845,10 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
 
   __syncthreads();  // every wavefront is through with the stages and with P
   float l[2] = {0.0f, 0.0f};
-  if (n_steps > 0) {
+  if (my_steps > 0) {
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
-      const float other = l_sh()[((wave ^ 1) * 2 + rt) * 32 + l32];
+      const float other = l_sh(wave ^ 1)[32 * rt + l32];
       l[rt] = half ? other + l_run[rt] : l_run[rt] + other;
     }
   }

@@ -410,6 +410,49 @@ def test_tiled_kernel_head_dim_256_edges(kw, dtype, with_desc):
     _check(small_case(seed=61, HD=256, rows_per_tile=128, dtype=dtype, **{"H": 4, "Hkv": 2, **kw}), with_desc=with_desc)
 
 
+def _bits_with_infinite_values(c, rows, **kw):
+    """The pass's output as it is, and with infinite V in `rows` of it."""
+    from gpu_utils import run_case
+    print(f"case infinite values HD={c.params.head_dim} rows={rows} {kw}", flush=True)
+    clean, kept = run_case(c, **kw), c.Vb.copy()
+    c.Vb[list(rows)] = 0x7c00 if c.params.dtype == abi.ESP_F16 else 0x7f80
+    got = run_case(c, **kw)
+    c.Vb[:] = kept
+    return clean, got
+
+
+@pytest.mark.parametrize("P,M,at", [(0, 128, 100), (0, 128, 64), (16, 128, 100), (16, 128, 50), (48, 115, 80), (5, 128, 120), (0, 300, 270), (2500, 128, 127)])
+@pytest.mark.parametrize("rows_in_pool", [False, True])
+@pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
+def test_tiled_kernel_head_dim_256_infinite_values_stay_with_their_step(P, M, at, rows_in_pool, dtype):
+    """A row that overflowed in the projection has an infinite V. The 32 rows of a row tile compute the steps of 64 keys up to their last row's;
+    behind that their P is 0, and 0 x infinity is not: none of those products may be theirs. The rows that see the key are infinite or NaN."""
+    if rows_in_pool and P % 16:
+        P += 16 - P % 16
+    c = small_case(seed=66, HD=256, H=4, Hkv=2, seqs=((P + M, M),), rows_per_tile=128, dtype=dtype)
+    c.trees["P"] = P  # (the block list reaches as far as the rows)
+    options = host.options_mi355x(128, 64) if P > 2000 else host.options_mi355x(128, 1)
+    clean, got = _bits_with_infinite_values(c, [at], rows_in_pool=rows_in_pool, options=options)
+    step = lambda row: ((P + 15) // 16 + row // 16) // 4  # noqa: E731
+    same = [r for r in range(M) if step(min(r // 32 * 32 + 31, M - 1)) < step(at)]
+    assert len(same) >= 32 and max(same) < at
+    assert np.array_equal(got[same], clean[same])
+    assert not np.isfinite(f32(got[at:], dtype)).any()
+
+
+@pytest.mark.parametrize("HD,rows", [(256, 128)])
+@pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
+def test_tiled_kernel_other_trees_infinite_values(HD, rows, dtype):
+    """Rows of two trees share a group of 16: what one of them cannot see of the other's V does not reach it."""
+    c = small_case(seed=67, HD=HD, H=4, Hkv=2, seqs=((16, 40), (33, 30), (0, 43)), rows_per_tile=rows, dtype=dtype)
+    begin = [0, 40, 70, 113]
+    for bad in range(3):
+        at = range(begin[bad], begin[bad + 1])
+        clean, got = _bits_with_infinite_values(c, at)
+        others = [r for r in range(113) if r not in at]
+        assert np.array_equal(got[others], clean[others])
+
+
 @pytest.mark.parametrize("HD", [128, 256])
 @pytest.mark.parametrize("seqs", [((100, 1), (40, 31), (7, 33)), ((200, 127), (0, 128), (65, 97)), ((3000, 40),)])
 @pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
