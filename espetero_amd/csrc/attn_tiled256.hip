@@ -339,6 +339,11 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
   const int n_b = (tile.last && k_last >= tile.b0) ? ((tree.base + k_last) >> 4) - a0 + 1 : 0;
   n_sb = n_c + n_b;
   const int n_steps = (n_sb + 3) >> 2;
+  // A tile none of whose rows reaches b0: step 0 may have left with batch rows all the same; the sub-blocks that follow are the pool's.
+  if (n_b == 0) {
+    k_ld = kRowB;
+    k_row = uint32_t(hb) * kRowB;
+  }
 
   // Windowed layers: do this tile's batch keys need a window test at all? Not when the oldest position among
   // them is inside the window of the row with the largest position. Where they do and their positions rise by
@@ -838,10 +843,10 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
       load_v.template operator()<0>(S ^ 1);
       load_v.template operator()<1>(S ^ 1);
     }
-    wait_loads();
   } else {
     clear();
   }
+  wait_loads();  // nothing is on its way to LDS any more (step 0 left before it was known whether there is one)
 
   __syncthreads();  // every wavefront is through with the stages and with P
   float l[2] = {0.0f, 0.0f};

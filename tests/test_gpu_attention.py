@@ -410,6 +410,44 @@ def test_tiled_kernel_head_dim_256_edges(kw, dtype, with_desc):
     _check(small_case(seed=61, HD=256, rows_per_tile=128, dtype=dtype, **{"H": 4, "Hkv": 2, **kw}), with_desc=with_desc)
 
 
+@pytest.mark.parametrize("HD", [128, 256, 512])
+@pytest.mark.parametrize("P", [0, 16, 32, 48, 64, 80, 160])
+@pytest.mark.parametrize("rows_in_pool", [False, True])
+def test_tiled_kernels_tile_whose_rows_end_below_its_first_batch_key(HD, P, rows_in_pool):
+    """Records that esp_attn_validate takes and the planner does not make: `last` with b0 behind the tile's last row. Its rows see their cached
+    keys alone, or nothing at all; what the kernel asked for before it knew must neither be counted nor land in what it writes."""
+    import torch
+    from gpu_utils import append_rows, dev_u16, native_pool, to_host_u16
+    from espetero_amd import device
+    device.init(0)
+    R, M = (64, 90) if HD == 512 else (128, 170)
+    c = small_case(seed=68, HD=HD, H=4, Hkv=2, seqs=((P + M, M),), rows_per_tile=R)
+    c.trees["P"] = P
+    tiles = np.zeros(2, abi.TILE_DT)
+    tiles["k1"], tiles["part"], tiles["last"], tiles["r0"] = P, -1, 1, (0, R)
+    tiles["b0"][0] = R + 2
+    pool = native_pool(c)
+    dp = device.DevicePass(c.params, c.trees, tiles, np.zeros(0, abi.COMBINE_DT), 0, c.n_rows, c.blocks, c.desc, c.pos, pool_blocks=c.n_blocks,
+                           rows_in_pool=rows_in_pool)
+    Q, Kb, Vb = dev_u16(c.Q), dev_u16(c.Kb), dev_u16(c.Vb)
+    O = torch.full_like(Q, 0x1234)
+    if rows_in_pool:
+        append_rows(c, pool)
+        Kb = Vb = None
+    print(f"case b0 behind the rows HD={HD} P={P} rows_in_pool={rows_in_pool}", flush=True)
+    dp.run(Q, Kb, Vb, pool, O)
+    torch.cuda.synchronize()
+    got = f32(to_host_u16(O), c.params.dtype).reshape(M, 4, HD)
+    want = brute(c).reshape(M, 4, HD)
+    kv = f32(c.pool_ref, c.params.dtype).astype(np.float64).reshape(c.n_blocks, 2, c.params.bt, 2, HD)[c.blocks].swapaxes(0, 1).reshape(2, -1, 2, HD)[:, :P]
+    q = f32(c.Q, c.params.dtype).astype(np.float64).reshape(M, 4, HD)
+    for h in range(4):
+        s = q[:R, h] @ kv[0, :, h // 2].T * c.params.scale
+        w = np.exp(s - s.max(axis=1, keepdims=True)) if P else s
+        want[:R, h] = w / w.sum(axis=1, keepdims=True) @ kv[1, :, h // 2] if P else 0.0
+    assert np.abs(got - want).max() <= 2e-3
+
+
 def _bits_with_infinite_values(c, rows, **kw):
     """The pass's output as it is, and with infinite V in `rows` of it."""
     from gpu_utils import run_case
