@@ -317,6 +317,29 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
     }
     return lo;
   };
+  // Balanced rule: the batch keys count as work of the last part, so the cached range is
+  // cut into parts of (cached + batch) / ns keys and the last part keeps what is left.
+  auto step_of = [&](const RowTile& rt, int ns) {
+    const int per = (rt.span + rt.batch + ns - 1) / ns;
+    return (per + o.granule - 1) / o.granule * o.granule;
+  };
+  // A tile's ns parts, batch keys uncut: all but the last are `step` cached keys on page multiples; the last keeps the
+  // rest of the cached range (possibly nothing) and the batch keys.
+  auto for_cached_parts = [&](const RowTile& rt, int ns, auto&& part) {
+    const int P = A.trees[size_t(rt.tree)].P, step = step_of(rt, ns);
+    int k = rt.k0;
+    for (int p = 0; p < ns; ++p) {
+      const bool is_last = p + 1 == ns;
+      int k1 = P;
+      if (!is_last) {
+        k1 = std::min(P, k + step);
+        if (k1 < P) k1 = std::min(P, std::max(k + o.granule, k1 / o.granule * o.granule));
+        if (k1 == k) continue;  // the cached range ran out: the batch keys alone fill the last part
+      }
+      part(k, k1, is_last);
+      k = k1;
+    }
+  };
   std::vector<int> ns_of;  // balanced rule: parts of every row tile, once chosen
   std::vector<int> emit(size_t(n_tiles), 0);  // row tiles in the order their records are written
   for (int i = 0; i < n_tiles; ++i) emit[size_t(i)] = i;
@@ -476,40 +499,44 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
     }
     // A pass of few workgroups, at most one for two compute units, that nothing has cut so far - behind a window, or behind few keys - ends
     // with its longest tile while the rest of the chip stands idle: its tiles are cut until the parts fill the chip once, as long as
-    // that is shorter with the merge's dispatch and the records there and back. In us: what a lone workgroup takes for 64 keys, 7 for
-    // the merge and 0.35 for each MB of records. 100 rows behind a window of 1024, 16 / 8 heads of 256: 41.5 whole, 29.8 in four parts; 356 rows,
-    // 8 / 2 heads: 46.2 and 32.6; six of 41 .. 82 rows 40.1 and 29.2; three of 128 rows 43.0 and 34.9; 128 rows over 900 keys, 32 / 4 heads
-    // of 128: 28.0 and 20.6. Not two chunks of 300 rows over 500 keys, 16 heads of 256: 35.0 whole, 40.8 in two parts each; and not beyond
-    // what the rule above has cut (100 rows over 6871 keys 40.3 in its eight parts, 42.8 in fourteen). Passes with decoding rows are left
-    // to the rules above, and whatever is planned fits esp_attn_forward_static.
+    // that is shorter with the merge's dispatch and the records there and back. In us: what a lone workgroup takes for 64 keys, 4 for
+    // the merge and 0.5 for each MB of records, of the parts as they are emitted (fitted to 65 passes whole and in every even cut, 412 plans:
+    // what it picks takes 1.5 % longer than the best of them in geometric mean, 11 % at worst, whole passes 30 %). The
+    // last part of a tile may hold its batch keys alone: 960 keys + 100 rows, 16 / 8 heads of 256, 37.1 us whole, 26.0 in five parts and those, 27.6 in
+    // the most parts that all have cached keys. No tile in more than eight: nine cost the merge another 12 us there. Not two chunks of 300
+    // rows over 500 keys, 16 heads of 256: 35.2 whole, 40.8 in two parts each; and not beyond what the rule above has cut (100 rows over
+    // 6871 keys 40.3 in its eight parts, 42.8 in fourteen). Passes with decoding rows are left to the rules above, and whatever is planned
+    // fits esp_attn_forward_static.
     if (shape.family < 0 && !o.cut_batch && parts_in(ns_of) == 0 && grid * 2 <= esp::kComputeUnits && slots >= esp::kComputeUnits && o.part_steps > 0 &&
         std::none_of(rts.begin(), rts.end(), [&](const RowTile& rt) { return rt.r == 0 && live_rows(rt) <= 16; })) {
-      const double step_us = shape.head_dim == 128 ? 1.3 : shape.head_dim == 256 ? 1.75 : 2.0;
+      const double step_us = shape.head_dim == 128 ? 1.3 : shape.head_dim == 256 ? 1.75 : 3.4;
       const long long room = most_static_parts();
-      auto lone_us = [&](const std::vector<int>& ns_v) {
-        long long keys = 0;
-        double records = 0;
+      long long parts = 0, tiles = 0;  // of the plan priced last
+      auto price = [&](const std::vector<int>& ns_v) {
+        long long steps = 0, rows = 0;
+        parts = 0, tiles = n_tiles;
         for (int i = 0; i < n_tiles; ++i) {
           const RowTile& rt = rts[size_t(i)];
-          const long long ns = ns_v[size_t(i)], per = (rt.span + rt.batch + ns - 1) / ns, step = (per + o.granule - 1) / o.granule * o.granule;
-          keys = std::max(keys, ns > 1 ? std::max(step, rt.span + rt.batch - (ns - 1) * step) : (long long)(rt.span) + rt.batch);
-          if (ns > 1) records += double(ns) * live_rows(rt);
+          int used = 0;
+          for_cached_parts(rt, ns_v[size_t(i)], [&](int k, int k1, bool last) {
+            steps = std::max(steps, (long long)(k1 - k + (last ? rt.batch : 0) + o.granule - 1) / o.granule);
+            ++used;
+          });
+          if (ns_v[size_t(i)] <= 1) continue;
+          parts += used, tiles += used - 1, rows += used * live_rows(rt);
         }
-        const double bytes = records * groups * shape.head_dim * 4;
-        return double((keys + o.granule - 1) / o.granule) * step_us + (records > 0 ? 7 + bytes * 0.35e-6 : 0);
+        return double(steps) * step_us + (parts ? 4 + double(rows) * groups * shape.head_dim * 4 * 0.5e-6 : 0);
       };
-      double best = lone_us(ns_of);
-      for (long long c = c_hi - 1; c >= 2; --c) {
-        long long records = 0;
+      double best = price(ns_of);
+      for (long long c = c_hi - 1; c >= 2; c -= std::max<long long>(1, c_hi / 32)) {
+        const long long chunk = c * o.granule;
         for (int i = 0; i < n_tiles; ++i) {
           const RowTile& rt = rts[size_t(i)];
-          // parts of c steps, none of them without cached keys
-          const long long chunk = c * o.granule;
-          cand[size_t(i)] = int(std::clamp<long long>(std::min((rt.span + rt.batch + chunk - 1) / chunk, rt.span / chunk + 1), 1, o.max_splits));
-          records += cand[size_t(i)];
+          const long long most = rt.span > chunk ? std::min(o.max_splits, 8) : 1;
+          cand[size_t(i)] = int(std::clamp<long long>((rt.span + rt.batch + chunk - 1) / chunk, 1, most));
         }
-        if (records * groups > esp::kComputeUnits || parts_in(cand) > room) break;
-        const double t = lone_us(cand);
+        const double t = price(cand);
+        if (tiles * groups > esp::kComputeUnits || parts > room) break;
         if (t < best) best = t, ns_of = cand;
       }
     }
@@ -539,10 +566,7 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
       A.tiles.push_back({rt.tree, t.base + rt.r, rt.k0, t.P, -1, 1, rt.b0, pad});
       continue;
     }
-    // Balanced rule: the batch keys count as work of the last part, so the cached range is
-    // cut into parts of (cached + batch) / ns keys and the last part keeps what is left.
-    const int per = (span + rt.batch + ns - 1) / ns;
-    const int step = (per + o.granule - 1) / o.granule * o.granule;
+    const int step = step_of(rt, ns);
     const int part0 = A.parts;
     int used = 0;
     if (o.balanced && o.cut_batch && span < (ns - 1) * step) {
@@ -585,21 +609,10 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
         continue;
       }
     } else if (o.balanced) {
-      // ns parts: all but the last are `step` cached keys on page multiples; the last keeps the
-      // rest of the cached range (possibly nothing) and the batch keys.
-      int k = rt.k0;
-      for (int p = 0; p < ns; ++p) {
-        const bool is_last = p + 1 == ns;
-        int k1 = t.P;
-        if (!is_last) {
-          k1 = std::min(t.P, k + step);
-          if (k1 < t.P) k1 = std::min(t.P, std::max(k + o.granule, k1 / o.granule * o.granule));
-          if (k1 == k) continue;  // the cached range ran out: the batch keys alone fill the last part
-        }
-        A.tiles.push_back({rt.tree, t.base + rt.r, k, k1, A.parts++, is_last ? 1 : 0, rt.b0, pad});
-        k = k1;
+      for_cached_parts(rt, ns, [&](int k, int k1, bool last) {
+        A.tiles.push_back({rt.tree, t.base + rt.r, k, k1, A.parts++, last ? 1 : 0, rt.b0, pad});
         ++used;
-      }
+      });
     } else {
       for (int k = rt.k0; k < t.P; k += step, ++used) {
         const int k1 = std::min(t.P, k + step);

@@ -826,6 +826,45 @@ def test_passes_of_few_workgroups_are_cut(layer, slots, seqs):
     assert plan(seqs * 40, _layer_groups(H, Hkv, HD, rows))[2] == 0
 
 
+def _price_of_few_workgroups(layer, trees, tiles, rows):
+    """What the planner's rule for such passes says of records: the longest in steps of 64 keys, a merge, the records there and back."""
+    H, _, HD = layer
+    steps = live = 0
+    for x in tiles:
+        base, _, _, M = trees[x["tree"]]
+        r = int(x["r0"] - base)
+        batch = min(int(M), r + rows) - int(x["b0"]) if x["last"] else 0
+        steps = max(steps, -(-(int(x["k1"] - x["k0"]) + batch) // 64))
+        live += min(rows, int(M) - r) if x["part"] >= 0 else 0
+    return steps * {128: 1.3, 256: 1.75, 512: 3.4}[HD] + (4 + live * H * HD * 4 * 0.5e-6 if live else 0)
+
+
+@pytest.mark.parametrize("layer,slots", [((32, 4, 128), 512), ((8, 2, 128), 512), ((16, 8, 256), 256), ((8, 2, 256), 256), ((16, 2, 512), 256)])
+@pytest.mark.parametrize("window", [0, 1024])
+def test_cuts_of_passes_of_few_workgroups_cost_less_than_none(layer, slots, window):
+    """By the rule's own price of the records as they are: none is cut for nothing, none into more than eight parts."""
+    rng = np.random.default_rng(layer[2] + window)
+    rows = 64 if layer[2] == 512 else 128
+    o = host.options_mi355x(rows, slots)
+    n_cut = 0
+    passes = [((282, 474), (502, 89), (205, 210))] + [[(int(rng.integers(0, 3000 if window else 1021)), int(rng.integers(17, 500))) for _ in range(rng.integers(1, 4))]
+                                                      for _ in range(300)]
+    for seqs in passes:
+        trees = _pass_of(seqs)
+        pos = np.concatenate([np.repeat(P + np.arange(M)[:, None], 4, 1) for P, M in seqs]).astype(np.int32) if window else None
+        plan = lambda g: host.plan_tiles(trees, g, window, pos, o)  # noqa: E731
+        if plan(layer[0])[2]:
+            continue                                                 # another rule's
+        tiles, jobs, parts = plan(_layer_groups(*layer, rows))
+        whole = plan(layer[0])[0]
+        if parts:
+            n_cut += 1
+            assert _price_of_few_workgroups(layer, trees, tiles, rows) < _price_of_few_workgroups(layer, trees, whole, rows), seqs
+            assert len(tiles) * layer[0] <= 256 and max(int(j["nparts"]) for j in jobs) <= 8
+            assert ((tiles["k1"] > tiles["k0"]) | (tiles["last"] == 1)).all()
+    assert n_cut >= 25
+
+
 def _ones(*cached):
     return tuple((P, 1) for P in cached)
 
