@@ -528,11 +528,12 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
         return double(steps) * step_us + (parts ? 4 + double(rows) * groups * shape.head_dim * 4 * 0.5e-6 : 0);
       };
       double best = price(ns_of);
-      for (long long c = c_hi - 1; c >= 2; c -= std::max<long long>(1, c_hi / 32)) {
+      // The limits a caller sets bind here at a quarter: parts of 128 keys and ranges of 256 with the tuned ones.
+      for (long long c = c_hi - 1; c >= std::max(2, o.min_chunk / 4 / o.granule); c -= std::max<long long>(1, c_hi / 32)) {
         const long long chunk = c * o.granule;
         for (int i = 0; i < n_tiles; ++i) {
           const RowTile& rt = rts[size_t(i)];
-          const long long most = rt.span > chunk ? std::min(o.max_splits, 8) : 1;
+          const long long most = rt.span > chunk && rt.span >= o.min_span / 4 ? std::min(o.max_splits, 8) : 1;
           cand[size_t(i)] = int(std::clamp<long long>((rt.span + rt.batch + chunk - 1) / chunk, 1, most));
         }
         const double t = price(cand);

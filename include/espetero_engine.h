@@ -31,10 +31,12 @@ typedef struct esp_plan_options {
   int32_t rows_per_tile; /* query rows per tile (reference: 8) */
   int32_t groups_target; /* workgroups a few-tile pass is split up to (reference: 256) */
   int32_t split;         /* reference rule: largest chunk a split is sized to (attn_split, 512) */
-  int32_t min_chunk;     /* fewest cached keys of a split tile (attn_min_chunk, 32) */
+  int32_t min_chunk;     /* fewest cached keys of a split tile (attn_min_chunk, 32); a quarter of it where the balanced rule cuts a tiled
+                            kernel's pass of few workgroups (at most one for two compute units) for a known layer */
   int32_t granule;       /* split boundaries are multiples of this (32) */
   int32_t max_splits;    /* parts per tile group (64) */
-  int32_t min_span;      /* shorter cached ranges are not split (64) */
+  int32_t min_span;      /* shorter cached ranges are not split (64); a quarter of it in such a pass. Raised (1 << 30), either keeps
+                            passes whole */
   int32_t balanced;      /* 0: the reference's per-tree budget rule; 1: equal keys per workgroup */
   int32_t item_steps;    /* balanced rule, tiled kernel (> 0): groups_target is the workgroups resident at once and the
                             split chunk is the one whose workgroups finish earliest when handed to those slots in

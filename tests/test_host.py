@@ -824,6 +824,12 @@ def test_passes_of_few_workgroups_are_cut(layer, slots, seqs):
     assert plan(seqs, H)[2] == 0
     assert plan(seqs + ((800, 1),), _layer_groups(H, Hkv, HD, rows))[2] == 0
     assert plan(seqs * 40, _layer_groups(H, Hkv, HD, rows))[2] == 0
+    longest = max(P for P, _ in seqs)
+    for limit, below, above in (("min_span", 4 * min(P for P, _ in seqs), 4 * (longest + 1)), ("min_chunk", 4 * 128, 4 * longest)):
+        for value, cut in ((below, True), (above, False), (1 << 30, False)):
+            o = host.options_mi355x(rows, slots)
+            setattr(o, limit, value)
+            assert (plan(seqs, _layer_groups(H, Hkv, HD, rows))[2] > 0) == cut, (limit, value)
 
 
 def _price_of_few_workgroups(layer, trees, tiles, rows):
