@@ -27,8 +27,8 @@
 // what a workgroup waits for instructions it has not run before), masks worked out as bits. The form before, wavefronts of 32 rows with all
 // keys and all dims, read 256 KB of operands per step where this one reads 160 and had 420 others beside its 64: 4400 clocks. 8 x 1024 rows
 // over 15360 keys, 16 / 8 heads: 2180 us before, 1930 so; with a window of 1024 224 and 212; 100 rows over 6871 keys 44.5 and 40.4, with the
-// window 47.2 and 41.1; prompts of 300 rows 24.8 and 23.0, of 32 10.8 and 10.9; of 2 .. 7 rows from Kb / Vb 12.1 and 13.5 (two more barriers
-// and the longer way of a first step, in instructions the compute unit has not run before).
+// window 47.2 and 41.1; prompts of 300 rows 24.8 and 22.9, of 32 10.7 and 9.9, one of 48 10.4 and 10.2, one of 128 14.2 and 12.8; of 2 .. 7
+// rows side by side from Kb / Vb 12.1 and 12.9 (their groups of 16 hold each other's rows, whose V is zeroed in LDS).
 //
 // LDS layout (all 160 KB). K of a stage: 64 rows of 512 bytes, unpadded; the 16-byte chunk c of row r lies at chunk position
 // c ^ (pi(r) & 15), where pi swaps bits 2 and 3 of a row index. The lane with S^T row l reads key row pi(l): its chunk position is
@@ -81,16 +81,28 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
   // Loads of the fragments themselves, whose neighbouring lanes are different rows, take the memory path a clock per lane, and
   // both wavefronts of a row group need all dims of its 64 rows. The loads need the tile's record only: a row past the
   // pass's last one reads that row instead, one past the tree's is zeroed once the tree's record says so.
+  // Tiles of up to 32 rows take four of the 16, of up to 64 eight, and a row group without rows reads no fragments: what a short prompt waits for.
   u32x4 qrow[16];
+  auto q_loads = [](int rows, auto&& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f(i);
+    if (rows > 32) {
+#pragma unroll
+      for (int i = 4; i < 8; ++i) f(i);
+    }
+    if (rows > 64) {
+#pragma unroll
+      for (int i = 8; i < 16; ++i) f(i);
+    }
+  };
   {
     const char* q0 = reinterpret_cast<const char*>(a.Q + size_t(tile.r0) * a.q_ld + size_t(kvh * a.G + hg) * kHD);
     const uint32_t ld = uint32_t(a.q_ld) * 2, last = uint32_t(min(a.n_rows - 1 - tile.r0, 127)) * ld + uint32_t(l32) * 16;
     uint32_t at = uint32_t(2 * wave + hb) * ld + uint32_t(l32) * 16;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    q_loads(a.n_rows - tile.r0, [&](int i) __attribute__((always_inline)) {
       qrow[i] = *reinterpret_cast<const u32x4*>(q0 + min(at, last));
       at += 8 * ld;
-    }
+    });
   }
   // ---- this lane's two rows of the scores: places 64 rg + 32 rt + l32
   int m[2], row_of[2], qpos[2];
@@ -125,14 +137,13 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
     }
     int pr = (2 * wave + hb) / a.G, ph = 2 * wave + hb - pr * a.G;
     const int step_r = 8 / a.G, step_h = 8 - step_r * a.G;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    q_loads(places, [&](int i) __attribute__((always_inline)) {
       const int row = min(tile.r0 + pr, a.n_rows - 1);
       qrow[i] = *reinterpret_cast<const u32x4*>(a.Q + size_t(row) * a.q_ld + size_t(kvh * a.G + ph) * kHD + 8 * l32);
       pr += step_r;
       ph += step_h;
       if (ph >= a.G) ph -= a.G, ++pr;
-    }
+    });
   }
   const int rr[2] = {rr0 + m[0], rr0 + m[1]};
 
@@ -290,16 +301,14 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
         red[wave][3] = qm;
       }
     }
-    if (places < 128) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (8 * i + 2 * wave + hb >= places) qrow[i] = u32x4{0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    auto q_place = [&](int i) __attribute__((always_inline)) {
       const int r = 8 * i + 2 * wave + hb;
-      *reinterpret_cast<u32x4*>(lds + (i < 8 ? kKStage : kPBase - 64 * kRowB) + r * kRowB + ((l32 ^ (r & 15)) << 4)) = qrow[i];
-    }
+      return reinterpret_cast<u32x4*>(lds + (i < 8 ? kKStage : kPBase - 64 * kRowB) + r * kRowB + ((l32 ^ (r & 15)) << 4));
+    };
+    q_loads(places, [&](int i) __attribute__((always_inline)) { *q_place(i) = qrow[i]; });
+#pragma nounroll
+    for (int i = places >> 3; i < (places > 64 ? 16 : 8); ++i)
+      if (8 * i + 2 * wave + hb >= places) *q_place(i) = u32x4{0, 0, 0, 0};
     __syncthreads();
     int anc_max = 0;
     if (plain) {
@@ -326,15 +335,18 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
   // row's reference.
   u32x4 qf[2][KS];
   const int q_at = rg == 0 ? kKStage : kPBase - 64 * kRowB;
+  if (64 * rg < places) {
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    const int r = 64 * rg + 32 * rt + l32;
+    for (int rt = 0; rt < 2; ++rt) {
+      const int r = 64 * rg + 32 * rt + l32;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      qf[rt][ks] = *reinterpret_cast<const u32x4*>(lds + q_at + r * kRowB + (((2 * ks + hb) ^ (r & 15)) << 4));
-      asm volatile("" : "+a"(qf[rt][ks]));
+      for (int ks = 0; ks < KS; ++ks) qf[rt][ks] = *reinterpret_cast<const u32x4*>(lds + q_at + r * kRowB + (((2 * ks + hb) ^ (r & 15)) << 4));
     }
   }
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+a"(qf[rt][ks]));
 
   const int n_b = (tile.last && k_last >= tile.b0) ? ((tree.base + k_last) >> 4) - a0 + 1 : 0;
   n_sb = n_c + n_b;
@@ -710,6 +722,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
       __syncthreads();
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt) m_run[rt] = new_reference(mx_sh, mx, rt);
+      clear();  // (beside the softmax)
       all_slices(0);
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // own loads landed, own reads of this iteration's stages done
@@ -780,7 +793,6 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
 #pragma unroll
       for (int j = 0; j < 4; ++j) ring[0][j] = k_operand.template operator()<0>(j);
       iter.template operator()<true>(0, false);
-      clear();
 #pragma nounroll
       for (int i = 1; i < my_steps; ++i) {
         if (out_of_range) settle((i - 1) & 1);
