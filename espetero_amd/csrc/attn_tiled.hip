@@ -335,33 +335,32 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
     }
   };
   // After this wavefront's loads of `step` have landed: cached keys outside [k0, k1) may be
-  // memory never written; their V must not reach the products.
+  // memory never written, and rows beside the tree's are another's; their V must not reach the products (0 x infinity).
   auto fix = [&](int step, int stage) __attribute__((always_inline)) {
     const int s = 4 * step + wave;
-    // keys [v0, v1) of the sub-block's own numbering are memory that has been written: the tile's cached range, or,
-    // for batch rows read from the pool, everything up to the tree's last row (what lies below its first row is the
-    // end of its cached keys)
+    // keys [v0, v1) of the sub-block's own numbering count: the tile's cached range, or the tree's rows. (In the pool what lies below its
+    // first row is the end of its cached keys; a sub-block begins less than 16 rows in front of the tree. In Kb / Vb the staged V^T past the
+    // pass's last row is zero.)
     int j0, v0, v1;
     if (s < n_c) {
       j0 = (c0 + s) << 4;
       v0 = tile.k0;
       v1 = tile.k1;
-    } else if (in_pool && s < n_sb) {
+    } else if (s < n_sb) {
       j0 = ((a0 + s - n_c) << 4) - tree.base;
-      v0 = INT32_MIN;
-      v1 = tree.M;
+      v0 = in_pool ? -16 : 0;
+      v1 = !in_pool && end == a.n_rows ? 1 << 30 : tree.M;
     } else {
       return;
     }
     if (j0 >= v0 && j0 + 16 <= v1) return;
     const int jv = j0 + 8 * hb;
+    const int e0 = min(max(v0 - jv, 0), 8), e1 = min(max(v1 - jv, e0), 8);
+    const uint32_t in = (1u << e1) - (1u << e0);  // this lane's 8 keys, a bit each
     u32x4 msk;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bool lo = jv + 2 * e >= v0 && jv + 2 * e < v1;
-      const bool hi = jv + 2 * e + 1 >= v0 && jv + 2 * e + 1 < v1;
-      msk[e] = (lo ? 0xffffu : 0u) | (hi ? 0xffff0000u : 0u);
-    }
+    for (int e = 0; e < 4; ++e)
+      msk[e] = (uint32_t(__builtin_amdgcn_sbfe(int(in), 2 * e, 1)) & 0xffffu) | uint32_t(__builtin_amdgcn_sbfe(int(in), 2 * e + 1, 1)) << 16;
 #pragma unroll
     for (int q = 0; q < VP; ++q) {
       u32x4* p = reinterpret_cast<u32x4*>(lds + VOFF + stage * VBUF + wave * SUBV + q * 1024 + lane * 16);

@@ -223,22 +223,22 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
     }
   };
   // After this wavefront's loads of V^T of `step` have landed: cached keys outside [k0, k1) may be memory
-  // never written; their V must not reach the products.
+  // never written, and rows beside the tree's are another's; their V must not reach the products (0 x infinity).
   auto fix = [&](int step, int stage) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int sidx = 2 * step + t;
-      // keys [v0, v1) of the sub-block's own numbering are memory that has been written: the tile's cached range,
-      // or, for batch rows read from the pool, everything up to the tree's last row
+      // keys [v0, v1) of the sub-block's own numbering count: the tile's cached range, or the tree's rows. (In the pool what
+      // lies below its first row is the end of its cached keys; in Kb / Vb the staged V^T past the pass's last row is zero.)
       int j0, v0, v1;
       if (sidx < n_c) {
         j0 = (c0 + sidx) << 4;
         v0 = tile.k0;
         v1 = tile.k1;
-      } else if (in_pool && sidx < n_sb) {
+      } else if (sidx < n_sb) {
         j0 = ((a0 + sidx - n_c) << 4) - tree.base;
-        v0 = INT32_MIN;
-        v1 = tree.M;
+        v0 = in_pool ? INT32_MIN : 0;
+        v1 = !in_pool && tree.base + tree.M == a.n_rows ? 1 << 30 : tree.M;
       } else {
         continue;
       }

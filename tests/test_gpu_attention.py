@@ -478,7 +478,7 @@ def test_tiled_kernel_head_dim_256_infinite_values_stay_with_their_step(P, M, at
     assert not np.isfinite(f32(got[at:], dtype)).any()
 
 
-@pytest.mark.parametrize("HD,rows", [(256, 128)])
+@pytest.mark.parametrize("HD,rows", [(128, 128), (256, 128), (512, 64)])
 @pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
 def test_tiled_kernel_other_trees_infinite_values(HD, rows, dtype):
     """Rows of two trees share a group of 16: what one of them cannot see of the other's V does not reach it."""
