@@ -43,7 +43,12 @@
 
 namespace esp {
 
-template <int DT, int HD, int OCC>
+namespace {
+constexpr int HD = 128, OCC = tiled_occ(HD);       // dims of a head; workgroups per compute unit
+constexpr int kLds = 4 * 64 * HD * 2 + 64;         // two stages of K (64 rows) and V^T (64 keys), 16 ints
+}  // namespace
+
+template <int DT>
 __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int n_tiles) {
   constexpr int KS = HD / 16, NT = HD / 32;
   constexpr int ROWB = HD * 2;     // bytes of one K row
@@ -401,47 +406,43 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
     return ((a0 + s0 - n_c) << 4) - tree.base > wave_last;
   };
 
-  // A step's matrix work is 4 KS operand reads from LDS, each feeding one matrix instruction:
-  // Q K^T of keys 0..31 (KS reads of K), Q K^T of keys 32..63, P V of keys 0..31 (KS reads of
-  // V^T), P V of keys 32..63. They run in groups of GP operands through two register buffers:
+  // A step's matrix work is 32 operand reads from LDS, each feeding one matrix instruction, in four groups:
+  // Q K^T of keys 0..31 (8 reads of K), Q K^T of keys 32..63, P V of keys 0..31 (8 reads of
+  // V^T), P V of keys 32..63. They go through two register buffers:
   // while the matrix cores consume one group, the reads of the next are in flight, and the
   // softmax of a half step sits beside the matrix work of the following group.
-  constexpr int GP = 8;           // operands per group
-  constexpr int GK = KS / GP;     // groups per half step of Q K^T (and of P V)
-  constexpr int NG = 4 * GK;      // groups per step
+  constexpr int GP = KS;          // operands per group
+  constexpr int NG = 4;           // groups per step
   f32x16 s[2];                    // S^T of the two half steps: s[kt][4 i + j] is S^T row 8 i + 4 hb + j, which is key
                                   // 32 kt + pi(8 i + 4 hb + j) = 32 kt + 16 (i / 2) + 8 hb + 4 (i % 2) + j of the step
   u32x4 pb[2][2];                 // P^T of the two half steps as matrix operands
   u32x4 ring[2][GP];
 
   auto read_group = [&]<int S, int G>(u32x4 (&buf)[GP]) __attribute__((always_inline)) {
-    if constexpr (G < 2 * GK) {
-      constexpr int kt = G / GK, ks0 = (G % GK) * GP;
+    constexpr int kt = G & 1;
+    if constexpr (G < 2) {
 #pragma unroll
-      for (int j = 0; j < GP; ++j) buf[j] = *lds_ptr(kaddr[ks0 + j] + uint32_t(S * KBUF + kt * 32 * ROWB));
+      for (int j = 0; j < GP; ++j) buf[j] = *lds_ptr(kaddr[j] + uint32_t(S * KBUF + kt * 32 * ROWB));
     } else {
-      // Operand o = 2 nt + t of half step kt: keys 8 hb .. 8 hb + 7 of sub-block 2 kt + t, dims 32 nt .. : the
+      // Operand j = 2 nt + t of half step kt: keys 8 hb .. 8 hb + 7 of sub-block 2 kt + t, dims 32 nt .. : the
       // lane's 16 bytes of that sub-block's dim group.
-      constexpr int kt = (G - 2 * GK) / GK, o0 = ((G - 2 * GK) % GK) * GP;
 #pragma unroll
-      for (int j = 0; j < GP; ++j)
-        buf[j] = *lds_ptr(vaddr + uint32_t(S * VBUF + 2 * kt * SUBV + ((o0 + j) & 1) * SUBV + ((o0 + j) >> 1) * 1024));
+      for (int j = 0; j < GP; ++j) buf[j] = *lds_ptr(vaddr + uint32_t(S * VBUF + 2 * kt * SUBV + (j & 1) * SUBV + (j >> 1) * 1024));
     }
   };
   // Operands [J0, J1) of group G.
   auto mma_group = [&]<int G, int J0, int J1>(const u32x4 (&buf)[GP]) __attribute__((always_inline)) {
-    if constexpr (G < 2 * GK) {
-      constexpr int kt = G / GK, ks0 = (G % GK) * GP;
-      if constexpr (ks0 == 0 && J0 == 0) {
+    constexpr int kt = G & 1;
+    if constexpr (G < 2) {
+      if constexpr (J0 == 0) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) s[kt][i] = 0.0f;
       }
 #pragma unroll
-      for (int j = J0; j < J1; ++j) s[kt] = mfma32x16<DT>(buf[j], qf[ks0 + j], s[kt]);
+      for (int j = J0; j < J1; ++j) s[kt] = mfma32x16<DT>(buf[j], qf[j], s[kt]);
     } else {
-      constexpr int kt = (G - 2 * GK) / GK, o0 = ((G - 2 * GK) % GK) * GP;
 #pragma unroll
-      for (int j = J0; j < J1; ++j) acc[(o0 + j) >> 1] = mfma32x16<DT>(buf[j], pb[kt][(o0 + j) & 1], acc[(o0 + j) >> 1]);
+      for (int j = J0; j < J1; ++j) acc[j >> 1] = mfma32x16<DT>(buf[j], pb[kt][j & 1], acc[j >> 1]);
     }
   };
 
@@ -592,22 +593,21 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   auto phase = [&]<int S, int G>(int step, auto interior) __attribute__((always_inline)) {
     if constexpr (G + 1 < NG) read_group.template operator()<S, G + 1>(ring[(G + 1) & 1]);
     // One wait for the whole group (its GP reads went out a group ago; the GP just issued stay in
-    // flight) instead of one in front of every matrix instruction: at one wavefront per SIMD every
-    // issued instruction, a wait included, is time the matrix pipe idles.
+    // flight) instead of one in front of every matrix instruction, which would be an instruction more each.
     __builtin_amdgcn_s_waitcnt(G + 1 < NG ? kWaitLgkm8 : kWaitLgkm0);
-    if constexpr (G == GK || G == 2 * GK) {
+    if constexpr (G == 1 || G == 2) {
       // On the mask-free path there is no branchy part and the whole group carries the arithmetic.
       constexpr int HEAD = decltype(interior)::value ? 0 : 3;  // (2, 4, 5: equal or slower - measured)
       mma_group.template operator()<G, 0, HEAD>(ring[G & 1]);
       __builtin_amdgcn_sched_barrier(0);
-      softmax_pre(step, std::integral_constant<int, G == GK ? 0 : 1>{}, interior);
+      softmax_pre(step, std::integral_constant<int, G - 1>{}, interior);
       __builtin_amdgcn_sched_barrier(0);
       // One matrix instruction, then its share of the eight slices, fenced so that the order stands.
       // The group's last matrix instructions wait until the half step's sum has been compared with its limit:
       // they do not depend on P, and the branch on that comparison - a vector compare that the scalar unit has
       // to wait for - then stands behind matrix instructions in flight instead of behind an idle pipe.
       constexpr int TAILM = 2;  // (1: the same, 3: no gain - measured)
-      constexpr int NM = GP - HEAD - TAILM, KT = G == GK ? 0 : 1;
+      constexpr int NM = GP - HEAD - TAILM, KT = G - 1;
       [&]<int... M>(std::integer_sequence<int, M...>) __attribute__((always_inline)) {
         ([&]<int MI>() __attribute__((always_inline)) {
           mma_group.template operator()<G, HEAD + MI, HEAD + MI + 1>(ring[G & 1]);
@@ -622,13 +622,13 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
       __builtin_amdgcn_sched_barrier(0);
       mma_group.template operator()<G, GP - TAILM, GP>(ring[G & 1]);
       __builtin_amdgcn_sched_barrier(0);
-      softmax_settle(std::integral_constant<int, G == GK ? 0 : 1>{}, ps, out_of_range);
+      softmax_settle(std::integral_constant<int, KT>{}, ps, out_of_range);
     } else {
       __builtin_amdgcn_sched_barrier(0);
       mma_group.template operator()<G, 0, GP>(ring[G & 1]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (G == 3 * GK - 1) {  // P V of the first half step is in: the deferred rescale
+    if constexpr (G == 2) {  // P V of the first half step is in: the deferred rescale
       if (late) {
         asm volatile("s_nop 0");
 #pragma unroll
@@ -744,8 +744,8 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
 
   // ---- output: lane (row l32, half hb) holds dims 32 nt + 8 i + 4 hb + j at acc[nt][4 i + j]. The wavefront's 32 rows go
   // through its quarter of the stages, which all four have read, so that neighbouring lanes store one row's bytes: a store whose
-  // neighbouring lanes are different rows takes the memory path a clock per lane, 1.7 us of a workgroup at D = 128. Six prompts of 40 to
-  // 900 rows, prep to attention, 65.1 us -> 62.7; 8 x 1024 rows at 15360, 256 dims, 3913 -> 3885.
+  // neighbouring lanes are different rows takes the memory path a clock per lane, 1.7 us of a workgroup. Six prompts of 40 to
+  // 900 rows, prep to attention, 65.1 us -> 62.7.
   const float l = l_run + __shfl_xor(l_run, 32);
   const int h_in_group = packed ? m_row % a.G : hg;
   // The lane's number anew: addresses made from it before the loop would be carried through it, in registers it has not got.
@@ -754,8 +754,8 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   const int r32 = ln & 31, half = ln >> 5;
   char* ob = lds + wave * KBUF;
   // Parts of a tile that leaves a wavefront without rows go straight out: the stores of three do not fill the memory path, and the
-  // trip through LDS is longer than theirs. 64 rows behind 2000 keys, 32 query heads of 128 dims, 18.5 us so and 19.0 through LDS; 33 rows, 16
-  // heads of 256, 25.8 and 27.6; 200 rows, tiles of 128 and 72, 24 heads of 256, 36.1 and 37.1. All four: 128 rows behind 1000 keys 30.7 and 29.7.
+  // trip through LDS is longer than theirs. 64 rows behind 2000 keys, 32 query heads, 18.5 us so and 19.0 through LDS; all four: 128 rows
+  // behind 1000 keys 30.7 and 29.7.
   const bool direct = tile.part >= 0 && (packed || rows_live <= 96);
   if (!direct) __syncthreads();
   if (tile.part >= 0) {
@@ -788,36 +788,33 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
   }
 }
 
-// Workgroups per compute unit and the largest tile each variant takes.
-int tiled_max_rows(int HD) { return HD == 512 ? 64 : 128; }  // 512: attn_tiled512_kernel's 2 row groups of 32
-size_t tiled_smem_bytes(int HD) { return size_t(4) * 64 * HD * 2 + 64; }  // two stages of K (64 rows) and V^T (64 keys), 16 ints
+// The largest tile of either kernel.
+int tiled_max_rows(int head_dim) { return head_dim == 512 ? 64 : 128; }  // 512: attn_tiled512_kernel's 2 row groups of 32
 
-template <int DT, int HD>
+template <int DT>
 static hipError_t launch_tiled_t(const KArgs& a, int n_tiles, hipStream_t st) {
-  const size_t smem = tiled_smem_bytes(HD);
-  constexpr auto k = attn_tiled_kernel<DT, HD, tiled_occ(HD)>;
-  const hipError_t e = allow_dynamic_lds<k>(smem);
+  constexpr auto k = attn_tiled_kernel<DT>;
+  const hipError_t e = allow_dynamic_lds<k>(kLds);
   if (e != hipSuccess) return e;
-  launch_timed(k, dim3(unsigned(n_tiles) * a.H), dim3(256), smem, st, a, n_tiles);
+  launch_timed(k, dim3(unsigned(n_tiles) * a.H), dim3(256), size_t(kLds), st, a, n_tiles);
   return hipGetLastError();
 }
 
 hipError_t launch_tiled256(int dt, const KArgs& a, int n_tiles, hipStream_t st);
 hipError_t launch_tiled512(int dt, const KArgs& a, int n_tiles, hipStream_t st);
 
-// The dynamic LDS limit of every variant on the current device, ahead of the first launch.
+// The dynamic LDS limit of both variants on the current device, ahead of the first launch.
 hipError_t tiled_init_attributes() {
-  hipError_t e = allow_dynamic_lds<attn_tiled_kernel<ESP_F16, 128, tiled_occ(128)>>(tiled_smem_bytes(128));
-  if (e == hipSuccess) e = allow_dynamic_lds<attn_tiled_kernel<ESP_BF16, 128, tiled_occ(128)>>(tiled_smem_bytes(128));
-  return e;
+  const hipError_t e = allow_dynamic_lds<attn_tiled_kernel<ESP_F16>>(kLds);
+  return e != hipSuccess ? e : allow_dynamic_lds<attn_tiled_kernel<ESP_BF16>>(kLds);
 }
 
-hipError_t launch_tiled(int dt, int HD, const KArgs& a, int n_tiles, hipStream_t st) {
-  if (HD == 512 && (dt == ESP_F16 || dt == ESP_BF16)) return launch_tiled512(dt, a, n_tiles, st);
-  if (HD == 256 && (dt == ESP_F16 || dt == ESP_BF16)) return launch_tiled256(dt, a, n_tiles, st);
-  if (dt == ESP_F16 && HD == 128) return launch_tiled_t<ESP_F16, 128>(a, n_tiles, st);
-  if (dt == ESP_BF16 && HD == 128) return launch_tiled_t<ESP_BF16, 128>(a, n_tiles, st);
-  return hipErrorInvalidValue;
+hipError_t launch_tiled(int dt, int head_dim, const KArgs& a, int n_tiles, hipStream_t st) {
+  if (dt != ESP_F16 && dt != ESP_BF16) return hipErrorInvalidValue;
+  if (head_dim == 512) return launch_tiled512(dt, a, n_tiles, st);
+  if (head_dim == 256) return launch_tiled256(dt, a, n_tiles, st);
+  if (head_dim != HD) return hipErrorInvalidValue;
+  return dt == ESP_F16 ? launch_tiled_t<ESP_F16>(a, n_tiles, st) : launch_tiled_t<ESP_BF16>(a, n_tiles, st);
 }
 
 }  // namespace esp
