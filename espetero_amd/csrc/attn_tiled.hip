@@ -701,6 +701,10 @@ __global__ __launch_bounds__(256, OCC) void attn_tiled_kernel(const KArgs a, int
     wait_loads();
     fix(0, 0);
   }
+  // Q has arrived with step 0; said here, or the compiler waits for it in the loop, on the counter of the staging loads: a step's
+  // matrix work then waits for the next step's keys (a lone workgroup per compute unit 1005 ns a step, 940 so).
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
   __syncthreads();
   if (n_steps > 1) fill(1, 1, general);
   read_group.template operator()<0, 0>(ring[0]);

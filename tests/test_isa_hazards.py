@@ -56,15 +56,42 @@ def _assembly(src, out_dir):
     return open(out).read()
 
 
-@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
-def test_no_matrix_result_is_read_across_a_block_boundary_too_early(tmp_path):
+@pytest.fixture(scope="module")
+def listings(tmp_path_factory):
+    """{source: [(kernel, lines)]} of every source with matrix instructions."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not installed")
+    out = str(tmp_path_factory.mktemp("isa"))
     with ThreadPoolExecutor(len(SOURCES)) as pool:
-        texts = list(pool.map(lambda s: _assembly(s, str(tmp_path)), SOURCES))
+        texts = list(pool.map(lambda s: _assembly(s, out), SOURCES))
+    return {src: list(isa_hazards.kernels(text)) for src, text in zip(SOURCES, texts)}
+
+
+def test_no_matrix_result_is_read_across_a_block_boundary_too_early(listings):
     n_kernels, n_mfma, bad = 0, 0, []
-    for src, text in zip(SOURCES, texts):
-        for name, lines in isa_hazards.kernels(text):
+    for src, kernels in listings.items():
+        for name, lines in kernels:
             n_kernels += 1
             n_mfma += sum(1 for l in lines if l[0] == "ins" and l[1].startswith("v_mfma"))
             bad += [(src, name[:80]) + v for v in isa_hazards.violations(lines)]
     assert n_kernels >= 30 and n_mfma > 2000          # the listing really was parsed
     assert not bad, bad[:5]
+
+
+@pytest.mark.parametrize("src", ["attn_tiled.hip", "attn_tiled256.hip", "attn_tiled512.hip"])
+def test_matrix_instructions_of_a_step_do_not_wait_for_the_next_steps_keys(listings, src):
+    """The staging loads of the tiled kernels are on their way through a step and waited for at its barrier. A value loaded in front of the
+    loop and first used in it makes the compiler wait on the same counter among the matrix instructions, in every step."""
+    assert len(listings[src]) == 2
+    for name, lines in listings[src]:
+        seen = waits = found = 0
+        for kind, op, args in lines:
+            if kind == "label" or op.startswith(("s_cbranch", "s_branch")):
+                seen = waits = 0
+            elif op.startswith("v_mfma"):
+                seen += 1
+                found = max(found, seen)
+                assert seen < 8 or not waits, (name[:60], seen)
+            elif op == "s_waitcnt" and any(a.startswith("vmcnt") for a in args):
+                waits += 1
+        assert found >= 20
