@@ -94,4 +94,6 @@ def test_matrix_instructions_of_a_step_do_not_wait_for_the_next_steps_keys(listi
                 assert seen < 8 or not waits, (name[:60], seen)
             elif op == "s_waitcnt" and any(a.startswith("vmcnt") for a in args):
                 waits += 1
+            elif op == "s_barrier":
+                waits = 0
         assert found >= 20
