@@ -17,18 +17,21 @@
 // ahead of V in the staging. The row's reference m moves only where a lane's share of a step's sum says so, and in the whole workgroup at
 // once: the two wavefronts of a row group multiply each other's P.
 //
-// What bounds it: the issue of a lone wavefront per SIMD (accumulators 128 registers, Q 128, the rest 146). Such a wavefront issues an
+// What bounds it: the issue of a lone wavefront per SIMD (accumulators 128 registers, Q 128, the rest 143). Such a wavefront issues an
 // instruction every 8 clocks (measured: 2, 4, 6, 8 multiply-adds behind every v_mfma_f32_32x32x16 make it 33, 38, 51, 66 clocks; two
 // wavefronts on the SIMD 32, 33, 37, 45), so three instructions hide behind a matrix instruction's 32 clocks and every further one is
-// matrix time lost; a v_dot2 waits for the matrix pipe to drain, 14 clocks wherever one stands alone. A step of mask-free keys is 64 matrix
-// instructions (2048 clocks) and 270 others: 3300 clocks, of which 1300 in Q K^T with 12 of the 16 loads, 1450 in three quarters of P V
-// with the softmax, 180 in wait and barrier, 370 in the rest of P V with the other loads. So an instruction taken out of the step counts more than
-// one moved: loads in pairs on one LDS base, one form of the loop for masked and mask-free steps (a second copy cost spills and
-// what a workgroup waits for instructions it has not run before), masks worked out as bits. The form before, wavefronts of 32 rows with all
-// keys and all dims, read 256 KB of operands per step where this one reads 160 and had 420 others beside its 64: 4400 clocks. 8 x 1024 rows
-// over 15360 keys, 16 / 8 heads: 2180 us before, 1930 so; with a window of 1024 224 and 212; 100 rows over 6871 keys 44.5 and 40.4, with the
-// window 47.2 and 41.1; prompts of 300 rows 24.8 and 22.9, of 32 10.7 and 9.9, one of 48 10.4 and 10.2, one of 128 14.2 and 12.8; of 2 .. 7
-// rows side by side from Kb / Vb 12.1 and 12.9 (their groups of 16 hold each other's rows, whose V is zeroed in LDS).
+// matrix time lost; a v_dot2 waits for the matrix pipe to drain, 14 clocks wherever one stands alone. A step of mask-free keys in the pool
+// is 64 matrix instructions (2048 clocks) and 331 others as compiled, 39 of them waits and s_nops: 139 beyond three each, 1100 clocks, and
+// 3300 were measured, of which 1300 in Q K^T with 12 of the 16 loads, 1450 in three quarters of P V with the softmax, 180 in wait and
+// barrier, 370 in the rest of P V with the other loads. So an instruction taken out of the step counts more than one moved: loads in pairs on
+// one LDS base, one form of the loop for masked and mask-free steps (a second copy cost spills and what a workgroup waits for instructions it
+// has not run before), masks worked out as bits. The form before, wavefronts of 32 rows with all keys and all dims, had 310 others but read
+// 256 KB of operands per step through an LDS path of 128 bytes a clock, where this one reads 160: 4400 clocks.
+// Behind a window, rows whose first key lies past their tile's first step have no reference until then: their first P is infinite, and the
+// workgroup settles (four barriers, 128 multiplications, the step's softmax again) in one or two of a tile's 18 steps.
+// 8 x 1024 rows over 15360 keys, 16 / 8 heads: 2180 us before, 1930 so; with a window of 1024 232 and 217; 100 rows over 6871 keys 44.5 and
+// 40.4, with the window 47.2 and 41.1; prompts of 300 rows 24.8 and 22.9, of 32 10.7 and 9.6, one of 48 10.4 and 10.1, one of 128 14.2 and
+// 12.8; of 2 .. 7 rows side by side from Kb / Vb 12.1 and 12.5 (their groups of 16 hold each other's rows, whose V is zeroed in LDS).
 //
 // LDS layout (all 160 KB). K of a stage: 64 rows of 512 bytes, unpadded; the 16-byte chunk c of row r lies at chunk position
 // c ^ (pi(r) & 15), where pi swaps bits 2 and 3 of a row index. The lane with S^T row l reads key row pi(l): its chunk position is

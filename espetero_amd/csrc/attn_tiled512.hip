@@ -25,9 +25,10 @@
 // The row's reference m moves only where a lane's share of a step's sum says so, and in the whole workgroup at once: the two
 // wavefronts of a row group multiply each other's P.
 // What bounds it: one wavefront per SIMD (accumulators 128 registers, Q 128, the rest 130), which issues in order, and the 64 KB a
-// step brings through the compute unit's vector memory path at 64 B per clock. A step of whole cached sub-blocks takes 2150 clocks:
+// step brings through the compute unit's vector memory path at 64 B per clock. A step of whole cached sub-blocks is 242
+// instructions, 48 of them matrix ones, and takes 880 ns of a lone workgroup (910 with the 293 it had, 2150 clocks by the counter then:
 // 1010 in the 32 instructions of Q K^T (512 clocks) with 12 of a wavefront's 16 loads between them, 690 in 12 of P V (384) with
-// the softmax, 170 in the wait and the barrier, 280 in the last 4 of P V with the other 4 loads; with all 16 loads in a row behind
+// the softmax, 170 in the wait and the barrier, 280 in the last 4 of P V with the other 4 loads); with all 16 loads in a row behind
 // the barrier that stretch alone was 990, with four of them beside P V they landed too late (a wait of 440). Two prompt
 // chunks of 700 .. 1024 rows over 3000 .. 7000 keys, 16 / 2 heads: kernel 412 us before, 325 so (the step's scores by dims halves 3340
 // clocks; a lone branch that moved the reference inside the step's matrix instructions cost 70 register moves in every step).
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
   const uint32_t kx = uint32_t(4 * wave);
   const uint32_t voff = uint32_t((lane ^ ((lane >> 4) & 1)) << 4);
   // Staging of a step whose sub-blocks the pool holds: where this wavefront's share of the K of sub-block t lies (and, bt rows' worth
-  // of bytes behind it, of its V^T: kept for an iteration later), and two of its four loads of either. fill_k and fill_v: all four, whatever
+  // of bytes behind it, of its V^T: kept for an iteration later), and its four loads of either, on one LDS base. fill_k and fill_v: the same, whatever
   // the sub-block (v_src null: past the range).
   const char* k_src = nullptr;
   const char* v_src[2] = {nullptr, nullptr};
@@ -377,7 +378,7 @@ __global__ __launch_bounds__(256, 1) void attn_tiled512_kernel(const KArgs a, in
   // Q K^T of step i, then P V of step i - 1 but for four instructions, with the softmax of step i between them, and leaves P of step i.
   // Those four instructions stand behind the barrier that publishes it and cover the first reads and requests of the next.
   // plain: every key of steps i and i + 1 is a cached key inside [k0, k1) of a layer without a window, i >= 1, and no reference has to
-  // move. The loads stand between the matrix instructions there, two at a time.
+  // move. The loads stand between the matrix instructions there, a sub-block's four at a time.
   auto iter = [&](int i, auto plain) __attribute__((always_inline)) {
     constexpr bool PLAIN = decltype(plain)::value;
     const int S = i & 1;
