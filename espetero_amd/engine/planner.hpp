@@ -499,17 +499,18 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
     }
     // A pass of few workgroups, at most one for two compute units, that nothing has cut so far - behind a window, or behind few keys - ends
     // with its longest tile while the rest of the chip stands idle: its tiles are cut until the parts fill the chip once, as long as
-    // that is shorter with the merge's dispatch and the records there and back. In us: what a lone workgroup takes for 64 keys, 4 for
-    // the merge and 0.5 for each MB of records, of the parts as they are emitted (fitted to 65 passes whole and in every even cut, 412 plans:
-    // what it picks takes 1.5 % longer than the best of them in geometric mean, 11 % at worst, whole passes 30 %). The
-    // last part of a tile may hold its batch keys alone: 960 keys + 100 rows, 16 / 8 heads of 256, 37.1 us whole, 26.0 in five parts and those, 27.6 in
-    // the most parts that all have cached keys. No tile in more than eight: nine cost the merge another 12 us there. Not two chunks of 300
-    // rows over 500 keys, 16 heads of 256: 35.2 whole, 40.8 in two parts each; and not beyond what the rule above has cut (100 rows over
-    // 6871 keys 40.3 in its eight parts, 42.8 in fourteen). Passes with decoding rows are left to the rules above, and whatever is planned
-    // fits esp_attn_forward_static.
+    // that is shorter with the merge's dispatch and the records there and back. In steps of 64 keys of the longest part, of the parts as they
+    // are emitted: 2.5 for the merge and 0.6 for each MB of records at 128 dims (where a step behind a window counts 1.4), 4.5 and 0.15 at
+    // 256, 2 and 0.15 at 512. Fitted to 217 passes of 40 .. 1900 rows timed whole and in every even cut, 1295 plans: what it picks takes
+    // 1.6 % longer than the best of them in geometric mean, 18 % at worst, never more than 2.5 % longer than the whole pass, which takes
+    // 24 % more than the best. The last part of a tile may hold its batch keys alone: 960 keys + 100 rows, 16 / 8 heads of 256, 37.1 us
+    // whole, 26.0 in five parts and those, 27.6 in the most parts that all have cached keys. No tile in more than eight: nine cost the merge
+    // another 12 us there. Not beyond what the rule above has cut (100 rows over 6871 keys 40.3 in its eight parts, 42.8 in fourteen).
+    // Passes with decoding rows are left to the rules above, and whatever is planned fits esp_attn_forward_static.
     if (shape.family < 0 && !o.cut_batch && parts_in(ns_of) == 0 && grid * 2 <= esp::kComputeUnits && slots >= esp::kComputeUnits && o.part_steps > 0 &&
         std::none_of(rts.begin(), rts.end(), [&](const RowTile& rt) { return rt.r == 0 && live_rows(rt) <= 16; })) {
-      const double step_us = shape.head_dim == 128 ? 1.3 : shape.head_dim == 256 ? 1.75 : 3.4;
+      const double merge = shape.head_dim == 128 ? 2.5 : shape.head_dim == 256 ? 4.5 : 2.0;
+      const double per_mb = shape.head_dim == 128 ? 0.6 : 0.15;
       const long long room = most_static_parts();
       long long parts = 0, tiles = 0;  // of the plan priced last
       auto price = [&](const std::vector<int>& ns_v) {
@@ -525,16 +526,18 @@ inline void plan_tiles(AttnPlan& A, int groups, int window, const int32_t* pos, 
           if (ns_v[size_t(i)] <= 1) continue;
           parts += used, tiles += used - 1, rows += used * live_rows(rt);
         }
-        return double(steps) * step_us + (parts ? 4 + double(rows) * groups * shape.head_dim * 4 * 0.5e-6 : 0);
+        return double(steps) * (shape.head_dim == 128 && window > 0 ? 1.4 : 1.0) + (parts ? merge + per_mb * 4e-6 * double(rows) * groups * shape.head_dim : 0);
       };
       double best = price(ns_of);
       // The limits a caller sets bind here at a quarter: parts of 128 keys and ranges of 256 with the tuned ones.
-      for (long long c = c_hi - 1; c >= std::max(2, o.min_chunk / 4 / o.granule); c -= std::max<long long>(1, c_hi / 32)) {
+      const int min_step = std::max(2 * o.granule, o.min_chunk / 4), min_span = std::max(1, o.min_span / 4);
+      for (long long c = c_hi - 1; c >= 2; c -= std::max<long long>(1, c_hi / 32)) {
         const long long chunk = c * o.granule;
         for (int i = 0; i < n_tiles; ++i) {
           const RowTile& rt = rts[size_t(i)];
-          const long long most = rt.span > chunk && rt.span >= o.min_span / 4 ? std::min(o.max_splits, 8) : 1;
-          cand[size_t(i)] = int(std::clamp<long long>((rt.span + rt.batch + chunk - 1) / chunk, 1, most));
+          int ns = int(std::clamp<long long>((rt.span + rt.batch + chunk - 1) / chunk, 1, rt.span >= min_span ? std::min(o.max_splits, 8) : 1));
+          while (ns > 1 && step_of(rt, ns) < min_step) --ns;
+          cand[size_t(i)] = ns;
         }
         const double t = price(cand);
         if (tiles * groups > esp::kComputeUnits || parts > room) break;

@@ -832,7 +832,7 @@ def test_passes_of_few_workgroups_are_cut(layer, slots, seqs):
             assert (plan(seqs, _layer_groups(H, Hkv, HD, rows))[2] > 0) == cut, (limit, value)
 
 
-def _price_of_few_workgroups(layer, trees, tiles, rows):
+def _price_of_few_workgroups(layer, trees, tiles, rows, window):
     """What the planner's rule for such passes says of records: the longest in steps of 64 keys, a merge, the records there and back."""
     H, _, HD = layer
     steps = live = 0
@@ -842,7 +842,8 @@ def _price_of_few_workgroups(layer, trees, tiles, rows):
         batch = min(int(M), r + rows) - int(x["b0"]) if x["last"] else 0
         steps = max(steps, -(-(int(x["k1"] - x["k0"]) + batch) // 64))
         live += min(rows, int(M) - r) if x["part"] >= 0 else 0
-    return steps * {128: 1.3, 256: 1.75, 512: 3.4}[HD] + (4 + live * H * HD * 4 * 0.5e-6 if live else 0)
+    merge, per_mb = {128: (2.5, 0.6), 256: (4.5, 0.15), 512: (2.0, 0.15)}[HD]
+    return steps * (1.4 if HD == 128 and window else 1.0) + (merge + per_mb * 4e-6 * live * H * HD if live else 0)
 
 
 @pytest.mark.parametrize("layer,slots", [((32, 4, 128), 512), ((8, 2, 128), 512), ((16, 8, 256), 256), ((8, 2, 256), 256), ((16, 2, 512), 256)])
@@ -865,7 +866,7 @@ def test_cuts_of_passes_of_few_workgroups_cost_less_than_none(layer, slots, wind
         whole = plan(layer[0])[0]
         if parts:
             n_cut += 1
-            assert _price_of_few_workgroups(layer, trees, tiles, rows) < _price_of_few_workgroups(layer, trees, whole, rows), seqs
+            assert _price_of_few_workgroups(layer, trees, tiles, rows, window) < _price_of_few_workgroups(layer, trees, whole, rows, window), seqs
             assert len(tiles) * layer[0] <= 256 and max(int(j["nparts"]) for j in jobs) <= 8
             assert ((tiles["k1"] > tiles["k0"]) | (tiles["last"] == 1)).all()
     assert n_cut >= 25
