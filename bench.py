@@ -1112,7 +1112,7 @@ class Ceilings:
         return out
 
 
-    SHAPES256 = ("4 wavefronts x 32 rows, one per SIMD (as built)", "8 wavefronts as 4 pairs, P through LDS",
+    SHAPES256 = ("4 wavefronts x 32 rows, one per SIMD (the kernel's first form)", "8 wavefronts as 4 pairs, P through LDS",
                  "8 wavefronts x 16 rows, v_mfma_f32_16x16x32")
     LOADS256 = ("no staging loads", "64 KB per step staged behind the barrier", "one load behind each of the first 16 matrix instructions",
                 "a second barrier in mid-step, each wavefront's loads beside two groups of matrix instructions of its own",

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256, 2) void issue_kernel(float* out, int iters, ui
 //        per matrix instruction), laid by hand behind each matrix instruction
 //   4  + each wavefront staging 8 KB per step from global memory straight into LDS (global_load_lds_dwordx4),
 //        from a 4 MB window of `src` that stays in the caches
-// ROWS: 1 = 32 query rows per wavefront (the kernels as built), 2 = 64 rows: every operand read feeds two
+// ROWS: 1 = 32 query rows per wavefront (the 128-dim kernel), 2 = 64 rows: every operand read feeds two
 // matrix instructions, at one wavefront per SIMD. clk[2 w], clk[2 w + 1]: cycles and 100 MHz ticks workgroup w
 // was alive, which give the clock the part ran at under this load.
 __device__ __forceinline__ void stage_to_lds(const char* base, uint32_t lane_off, uint32_t lds_addr) {
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256, ROWS == 2 ? 1 : 2) void step_kernel(float* out
 // The head-dim-256 prefill step as bare instruction streams: per step a compute unit multiplies 64 keys with 128 query
 // rows of one 256-dim head (256 v_mfma_f32_32x32x16 or as many flops in 16x16x32), every A operand read from LDS,
 // 32 scores per row-lane of softmax work, one barrier, 64 KB staged from `src` into LDS. Three shapes of the workgroup:
-//   0  4 wavefronts x 32 rows, one per SIMD: the kernel as built (64 matrix instructions per wavefront and step)
+//   0  4 wavefronts x 32 rows, one per SIMD: the kernel's first form (64 matrix instructions per wavefront and step)
 //   1  8 wavefronts as 4 pairs: a wavefront takes half of the step's keys through Q K^T and the softmax, hands its
 //      packed P to its partner through LDS and multiplies all 64 keys' P with its half of the dims
 //   2  8 wavefronts x 16 rows on v_mfma_f32_16x16x32: every wavefront a whole head, reading all of K and V^T

@@ -43,7 +43,7 @@ int esp_ceiling_mfma_issue(int32_t valu_per_mfma, int32_t exp_per_mfma, int32_t 
  * LDS a group ahead; 2 = + a workgroup barrier per step; 3 = + the softmax's share of vector work behind the
  * matrix instructions of two of the four groups; 4 = + every wavefront staging 8 KB per step from `src` (a
  * device buffer of at least 4 MB + 64 KB, cache resident) straight into LDS. rows: 1 = 32 query rows per wavefront,
- * two workgroups per compute unit (the kernels as built); 2 = 64 rows, every operand read feeding two matrix
+ * two workgroups per compute unit (the 128-dim kernel); 2 = 64 rows, every operand read feeding two matrix
  * instructions, one workgroup per compute unit (stages 1, 3, 4 only). What stage 4 reaches is the ceiling of
  * that kernel design; the difference between stages is what each ingredient costs. clk (NULL or 2 * workgroups
  * 64-bit words): cycles and 100 MHz ticks each workgroup was alive; cycles / ticks * 100 MHz is the clock the
@@ -54,7 +54,7 @@ int esp_ceiling_prefill_step(int32_t stage, int32_t rows, int32_t random_data, i
 /* The key step of the 256-dim prefill kernel as bare instruction streams, in three shapes of the workgroup. Per step a
  * compute unit multiplies 64 keys with 128 query rows of one head (the flops of 256 v_mfma_f32_32x32x16), every A operand
  * read from LDS, with 32 scores per row of softmax arithmetic and one barrier. shape: 0 = 4 wavefronts x 32 rows, one per
- * SIMD (the kernel as built); 1 = 8 wavefronts as 4 pairs, each wavefront taking half of the step's keys through Q K^T and
+ * SIMD (the kernel's first form; the present one, two row groups of 64 rows x 2, is none of them); 1 = 8 wavefronts as 4 pairs, each wavefront taking half of the step's keys through Q K^T and
  * the softmax, handing its packed P to its partner through LDS and multiplying all 64 keys' P with its half of the dims;
  * 2 = 8 wavefronts x 16 rows on v_mfma_f32_16x16x32, each a whole head. loads: 0 = none, 1 = the step's 64 KB staged from
  * `src` (a device buffer of at least 8 MB + 64 KB, cache resident) straight into LDS behind the barrier, 2 (shape 0 only) =
