@@ -1088,7 +1088,7 @@ class Ceilings:
 
     def prefill_step(self, cases=((0, 1, 1), (1, 1, 1), (2, 1, 1), (3, 1, 1), (4, 1, 1), (4, 1, 0), (1, 2, 1), (3, 2, 1), (4, 2, 1)), iters=3000):
         """TFLOP/s of the prefill kernel's step as a bare instruction stream, one ingredient more per stage, at 32
-        rows per wavefront and two workgroups per compute unit (the kernels as built) or 64 rows and one, on random
+        rows per wavefront and two workgroups per compute unit (the 128-dim kernel) or 64 rows and one, on random
         or constant operands; with the clock each launch ran at, read inside the kernel."""
         t = self.torch
         src = t.full(((4 << 20) + 65536,), 0x5b, dtype=t.uint8, device="cuda")
