@@ -252,8 +252,8 @@ __global__ __launch_bounds__(256, 1) void attn_tiled256_kernel(const KArgs a, in
     load_k.template operator()<3>(stage);
   };
 
-  // Step 0 leaves now and lands while the rows' facts are worked out. They may show that the range ends sooner than the tree:
-  // what is brought beyond it is there all the same, and masked.
+  // Step 0 leaves now, behind the Q rows, and has landed at the first barrier with them (the store of the last Q row waits on the same
+  // counter). The rows' facts may show that the range ends sooner than the tree: what is brought beyond it is there all the same, and masked.
   n_sb = n_c + ((tile.last && tree.M > tile.b0) ? ((end - 1) >> 4) - a0 + 1 : 0);
   if (n_sb > 0) {
     locate(0);
