@@ -198,6 +198,8 @@ def test_tiled_kernel_short_tiles(kw, split):
     dict(seqs=((0, 400),)),                            # the batch run only
     dict(seqs=((40, 300), (333, 70))),                 # a cached range that ends inside a half step, then batch rows
     dict(seqs=((1000, 140),), HD=256, H=4),            # head dim 256: the lazily moved maximum
+    dict(seqs=((0, 400),), HD=256, H=4),
+    dict(seqs=((40, 300), (333, 70)), HD=256, H=4),
     dict(seqs=((600, 70),), HD=512, H=4, rows_per_tile=64),
     dict(seqs=((900, 1), (77, 1)), H=16, rows_per_tile=1),                                          # streaming kernel, decode
     dict(seqs=((500, 4),), H=16, rows_per_tile=4, desc_fn=lambda M: synth.verify_desc(M, 1)),     # and verify
@@ -446,6 +448,21 @@ def test_tiled_kernels_tile_whose_rows_end_below_its_first_batch_key(HD, P, rows
         w = np.exp(s - s.max(axis=1, keepdims=True)) if P else s
         want[:R, h] = w / w.sum(axis=1, keepdims=True) @ kv[1, :, h // 2] if P else 0.0
     assert np.abs(got - want).max() <= 2e-3
+
+
+@pytest.mark.parametrize("P,M", [(0, 128), (0, 300), (16, 100), (70, 128), (2500, 128)])
+@pytest.mark.parametrize("at", [64, 80])
+@pytest.mark.parametrize("dtype", [abi.ESP_F16, abi.ESP_BF16])
+def test_tiled_kernel_head_dim_256_references_move_when_a_row_group_has_ended(P, M, at, dtype):
+    """Keys from row `at` on score far above the others: the rows that see them move their references in steps behind the first row
+    group's last one, which that group's wavefronts only stage and meet at the barriers."""
+    c = small_case(seed=69, HD=256, H=4, Hkv=2, seqs=((P, M),), rows_per_tile=128, dtype=dtype)
+    c.Kb[at:] = synth._bits(f32(c.Kb[at:], dtype) * 12.0, dtype)
+    from gpu_utils import run_case
+    print(f"case references behind an ended group P={P} M={M} at={at} dtype={dtype}", flush=True)
+    want = brute(c)
+    err, err_checker = (max_abs(x, want, dtype) for x in (run_case(c), oracle_direct(c, threads=8)))
+    assert err <= tol_for(dtype) and err_checker <= tol_for(dtype), (err, err_checker)
 
 
 def _bits_with_infinite_values(c, rows, **kw):
