@@ -55,7 +55,8 @@ int esp_ceiling_prefill_step(int32_t stage, int32_t rows, int32_t random_data, i
  * compute unit multiplies 64 keys with 128 query rows of one head (the flops of 256 v_mfma_f32_32x32x16), every A operand
  * read from LDS, with 32 scores per row of softmax arithmetic and one barrier. shape: 0 = 4 wavefronts x 32 rows, one per
  * SIMD (the kernel's first form; the present one, two row groups of 64 rows x 2, is none of them); 1 = 8 wavefronts as 4
- * pairs, each wavefront taking half of the step's keys through Q K^T and the softmax, handing its packed P to its partner through LDS and multiplying all 64 keys' P with its half of the dims;
+ * pairs, each wavefront taking half of the step's keys through Q K^T and the softmax, handing its packed P to its partner
+ * through LDS and multiplying all 64 keys' P with its half of the dims;
  * 2 = 8 wavefronts x 16 rows on v_mfma_f32_16x16x32, each a whole head. loads: 0 = none, 1 = the step's 64 KB staged from
  * `src` (a device buffer of at least 8 MB + 64 KB, cache resident) straight into LDS behind the barrier, 2 (shape 0 only) =
  * one load behind each of the step's first 16 matrix instructions, 3 (shape 0 only) = a second barrier in mid-step and
